@@ -47,15 +47,16 @@ TRACE_LIB = os.path.join(LIB_DIR, "trace", "libkvexp_hip_trace.so")
 ASM_DIR = os.path.join(HERE, "_build", "asm")
 
 ARCH = "gfx950"
-# the split kernel's instantiation units first (the longest compiles), so
+# the split kernels' instantiation units first (the longest compiles), so
 # that a parallel build starts them at once
 SOURCES = [
-    "csrc/hip/attention_wave_d256_o1.hip",
-    "csrc/hip/attention_wave_d256_o0.hip",
-    "csrc/hip/attention_wave_d128_o1.hip",
-    "csrc/hip/attention_wave_d128_o0.hip",
     "csrc/hip/attention_wave_d64_o1.hip",
     "csrc/hip/attention_wave_d64_o0.hip",
+    *(f"csrc/hip/attention_team_d{d}_o{o}.hip" for d in (256, 224, 192, 160, 128, 96) for o in (1, 0)),
+    "csrc/hip/attention_team_d112_o0.hip",
+    "csrc/hip/attention_team_d80_o0.hip",
+    "csrc/hip/attention_wave_d32_o1.hip",
+    "csrc/hip/attention_wave_d32_o0.hip",
     "csrc/hip/attention_wave.hip",
     "csrc/hip/codec_kernels.hip",
     "csrc/hip/attention_kernels.hip",
@@ -63,6 +64,7 @@ SOURCES = [
 ]
 CXX_SOURCES = ["csrc/host/kvexp_cpp_api.cpp"]
 HEADERS = [
+    "csrc/hip/attention_team.h",
     "csrc/hip/attention_wave.h",
     "csrc/hip/kvexp_device.h",
     "csrc/hip/kvexp_expf.h",

@@ -1,25 +1,22 @@
-// The one-wave split kernel and its merge (templates), shared by the
-// translation units that instantiate them: attention_wave.hip (head_dim 64
-// and 128, the merges, the entry points) and attention_wave256.hip (head_dim
-// 256), compiled in parallel.
+// The one-wave split kernel (templates; head_dim 32 and 64, instantiated in
+// attention_wave_d<D>_o<O>.hip), the helpers it shares with the team kernel
+// (attention_team.h, the larger head_dims), and the merge.
 #pragma once
-// gfx950 fused decode attention, head_dim 64, 128 or 256, scalar/AVX2 and
-// AVX-512 BF16 score orders: one wave64 per split, no workgroup barriers on
-// the hot path.
+// gfx950 fused decode attention, head_dim 32 or 64, scalar/AVX2 and AVX-512
+// BF16 score orders: one wave64 per split, no workgroup barriers on the hot
+// path.
 //
 // A split [tok_begin, tok_end) of one KV head is processed in chunks of up to
 // 64 tokens that never cross a K or V block; the order below is the loop's,
 // except that the softmax (4) runs before the V decode (3), so that the
 // scores are no longer live while V is decoded. Per chunk the wave:
-//   1. decodes the chunk's K rows from registers loaded one chunk ahead (16-
-//      channel pieces, consecutive lanes on consecutive bytes, so every load
-//      instruction reads a few whole cache lines) into a BF16 tile in its own
-//      LDS slice (row t: token t): a coded element is
+//   1. decodes the chunk's K rows from registers loaded one chunk ahead into a
+//      BF16 tile in its own LDS slice (row t: token t): a coded element is
 //      (sm & 0x80) << 8 | (base + code) << 7 | (sm & 0x7F), built two at a
 //      time with v_perm_b32 / v_lshl_add_u32 / v_bfi_b32 on packed pairs;
 //      escape words are then written over their elements from the plan's
 //      escape records (position and word in one dword; a cursor per tensor:
-//      the window of 256 (2,048 at head_dim 256) loaded with the rows starts at the chunk's first
+//      the window of 256 loaded with the rows starts at the chunk's first
 //      escape, and a chunk is cut short where its escapes would not fit);
 //      raw blocks are copied in chunks of at most 48 rows (the registers of
 //      64 coded rows). Every lane issues the same loads on every path, so
@@ -41,10 +38,7 @@
 //      token moves the running maximum, alpha = exp(m_prev - m), with an
 //      exact DPP prefix maximum seeded by the maxima held in scalar registers
 //      and the glibc-identical expf; e and alpha go to LDS by query row;
-//   5. folds the chunk's tokens in order (lane = channel; at head_dim 128
-//      each lane holds channels lane and lane + 64), unrolled (at head_dim
-//      256 a group of 16 tokens that moves a maximum runs as a loop, to keep
-//      the code within the instruction cache):
+//   5. folds the chunk's tokens in order (lane = channel), unrolled:
 //      acc = fma(e, v, acc) as one rank-1 product per token and row group
 //      (e of four rows in A, picked per token by the block broadcast; the
 //      token's V row in B), with acc scaled by alpha first only on the tokens
@@ -77,24 +71,15 @@ static __device__ unsigned long long g_phase_trace[kTraceWaves * kTraceWords];
 #endif
 
 constexpr int kChunk = 64;      // tokens per chunk (one per lane)
-// Escape records a chunk can patch, loaded with its rows: four per lane per
-// 16-byte load, one load at head_dim 64 and 128, eight at 256 (where escape-
-// dense blocks would otherwise cut chunks short: c5's 4-bit K blocks hold
-// about 1,300 escapes per 64 rows).
-template <int D>
-constexpr int kEscLoads = D == 256 ? 8 : 1;
-template <int D>
-constexpr int kEscWindow = 256 * kEscLoads<D>;
+constexpr int kEscWindow = 256; // escape records a chunk can patch, loaded with its rows: four per lane
 constexpr int kRawRows = 48;    // rows of a raw block per chunk: 64 lanes x 3D/2 bytes = 48 rows of 2D bytes
 constexpr uint16_t kNegZeroBf16 = 0x8000u; // V of a token past the chunk's end: fma(0, -0, acc) == acc exactly
 constexpr int kSlotQ = 8;       // partial-state slot: m[8], l[8], acc[8][head_dim]
 
 // How a chunk's coded rows are loaded (see Rows): whole rows (lane = row) at
 // head_dim 64, where a row's 64 sign/mantissa and 32 code bytes take six
-// 16-byte loads per lane; 16-channel pieces at 128 and 256, where whole rows
-// would put every load instruction on 64 different cache lines. Measured on
-// c2 (head_dim 64), whole rows: 93.7 us per step against 97.7 for pieces; on
-// c4 (head_dim 128), pieces: 2,726 against 3,323 for whole rows.
+// 16-byte loads per lane; 16-channel pieces at 32. Measured on c2 (head_dim
+// 64), whole rows: 93.7 us per step against 97.7 for pieces.
 template <int D>
 constexpr bool kWholeRows = D == 64;
 // Whether K rows of a chunk without escapes may skip the tile (whole rows:
@@ -103,19 +88,18 @@ constexpr bool kWholeRows = D == 64;
 template <int D, int ORDER>
 constexpr bool kDirectK = kWholeRows<D>;
 
-// The kernel's sizes for head_dim D (64, 128 or 256).
+// The kernel's sizes for head_dim D, and the slot size of every head_dim.
 template <int D>
 struct Shape {
     static constexpr int kTileStride = 2 * D + 16;  // bytes per tile row: D BF16 + 16 (conflict-free 16-byte rows)
     static constexpr int kSlotFloats = kSlotQ * (D + 2);
-    static constexpr int kPieces = D / 16;          // 16-channel pieces per row, and pieces per lane per chunk
-    static constexpr int kPieceRows = kChunk / kPieces; // chunk rows between a lane's consecutive pieces
+    static constexpr int kPieces = D / 16;          // 16-channel pieces per row
+    static constexpr int kPieceRows = kChunk / kPieces; // whole chunk rows one register's lanes cover
+    static constexpr int kPieceLanes = kPieceRows * kPieces; // their lanes
+    static constexpr int kPieceRegs = (kChunk + kPieceRows - 1) / kPieceRows; // pieces per lane per chunk
     static constexpr int kSmRegs = D / 16;          // whole rows: 16-byte registers of a row's sign/mantissa bytes
     static constexpr int kRowRegs = kSmRegs + D / 32; // + its 4-bit codes: what a coded row needs
-    static constexpr int kHalves = D / 64;          // channels per lane in the fold (lane, lane + 64, ...)
-    static constexpr int kWaves = D == 64 ? 4 : (D == 128 ? 2 : 1); // waves per workgroup (LDS: see WaveLds)
-    // splits per merge batch (one per lane; their rows in flight together)
-    static constexpr int kMergeBatch = D == 256 ? 32 : 64;
+    static constexpr int kWaves = 4;                // waves per workgroup (LDS: see WaveLds)
 };
 
 // Per-wave LDS. The tile holds the chunk's K rows (row t: the D BF16 of
@@ -124,8 +108,7 @@ struct Shape {
 // lane reads four tokens of its row in one access. At D = 64 and G <= 7 a
 // wave takes 13,152 bytes and a workgroup of four waves with the shared table
 // 52,864 bytes, which leaves room for three workgroups per CU (the limit lies
-// between 53,760 and 54,016 bytes per workgroup). At D = 128 and G = 4 a wave
-// takes 19,840 bytes; workgroups of two waves, four per CU.
+// between 53,760 and 54,016 bytes per workgroup).
 constexpr int kRowPad = kChunk + 4; // floats per eT / aT row: 16 spare bytes keep the rows' reads conflict-free
 
 template <int G, int D>
@@ -195,12 +178,12 @@ __device__ __forceinline__ int lane_here() {
 }
 
 // Position of one tensor inside its XKV container. The scalar fields are
-// wave-uniform; erec holds the block's next escape records (component j of
-// erec[i] at lane l: escape ecur + 256 i + 4 l + j, meaningful below
-// n_escape; kEscLoads of them are loaded); basew holds base exponents of
+// wave-uniform; erec holds the block's next escape records (component j at
+// lane l: escape ecur + 4 l + j, meaningful below n_escape; the team kernel
+// holds one per lane, escape ecur + l, in x); basew holds base exponents of
 // the block: whole rows, lane p < D / 2: base[2p], base[2p + 1]; pieces,
 // bytes 4j .. 4j + 3 of channel column c (channels 16 c .. 16 c + 15, see
-// Rows) at lane c + (D / 16) j, j < 4 (lanes past 4 D / 16 repeat them).
+// Rows) at lane c + (D / 16) j, j < 4 (later lanes repeat them).
 struct Cursor {
     const BlockDesc *d;  // descriptor of the current block (the next one follows it)
     const uint8_t *blk;  // current block's header
@@ -209,7 +192,8 @@ struct Cursor {
     uint32_t meta;       // mode | n_tokens << 8 | n_escape << 16
     int ecur;            // first escape of the block not yet written into a tile
     int lrows;           // rows requested by the last load_rows (the raw piece layout depends on it)
-    uint4 erec[8];
+    int shift;           // the rows were loaded from 2 bytes below their start (see load_team_rows)
+    uint4 erec;
     uint32_t basew;
     __device__ int mode() const { return int(meta & 0xFFu); }
     __device__ int ntok() const { return int((meta >> 8) & 0xFFu); }
@@ -248,24 +232,20 @@ __device__ __forceinline__ void block_vectors(Cursor &c) {
     if constexpr (kWholeRows<D>) c.basew = *(g_u16 *)(c.blk + 8 + 2 * (lane & (D / 2 - 1)));
     else c.basew = *(g_u32 *)(c.blk + 8 + 16 * (lane % NP) + 4 * ((lane / NP) & 3));
     const int left = c.nesc() - c.ecur; // records of the block not yet written
-#pragma unroll
-    for (int i = 0; i < kEscLoads<D>; ++i) {
-        const int first = 256 * i + 4 * lane;
-        u32x4 r = {0u, 0u, 0u, 0u};
-        if (first < left || lane == 0) r = *(g_u32x4 *)(c.esc + c.ecur + first);
-        c.erec[i] = make_uint4(r.x, r.y, r.z, r.w);
-    }
+    u32x4 r = {0u, 0u, 0u, 0u};
+    if (4 * lane < left || lane == 0) r = *(g_u32x4 *)(c.esc + c.ecur + 4 * lane);
+    c.erec = make_uint4(r.x, r.y, r.z, r.w);
 }
 
 // Rows of the cursor's block from row r0 on that the next chunk may take so
 // that its escapes all lie in the loaded window: when more than kEscWindow
 // escapes remain, the rows before the one holding the window's last record (its
-// position, read from lane 63). A row holds at most D <= 256 escapes, so the
-// answer is at least 1 (a row of 256 escapes fills the window alone).
+// position, read from lane 63). A row holds at most D escapes, so the answer is
+// at least 1.
 template <int D>
 __device__ __forceinline__ int escape_rows(const Cursor &c, int r0) {
-    if (c.nesc() - c.ecur <= kEscWindow<D>) return kChunk;
-    const uint32_t last = __builtin_amdgcn_readlane(c.erec[kEscLoads<D> - 1].w, kWave - 1) & 0xFFFFu;
+    if (c.nesc() - c.ecur <= kEscWindow) return kChunk;
+    const uint32_t last = __builtin_amdgcn_readlane(c.erec.w, kWave - 1) & 0xFFFFu;
     return max(1, int(last / D) - r0);
 }
 
@@ -275,10 +255,11 @@ __device__ __forceinline__ int escape_rows(const Cursor &c, int r0) {
 // repeated) code bytes; a raw block (at most kRawRows rows) as 16-byte pieces
 // (piece p: column p % (D / 8) of row p / (D / 8)), kRowRegs consecutive ones
 // per lane from raw_start.
-// Pieces (head_dim 128, 256): one piece per lane per register pair. Coded
+// Pieces: one piece per lane per register pair. Coded
 // block: piece p of the chunk is channels 16 (p % (D / 16)) .. + 16 of its
-// row p / (D / 16), and lane l holds pieces l + 64 k (k < D / 16): one
-// channel column c = l % (D / 16) in rows kPieceRows k + l / (D / 16). s[k]
+// row p / (D / 16), and lane l holds pieces l + kPieceLanes k (k <
+// kPieceRegs): one channel column c = l % (D / 16) in rows kPieceRows k +
+// l / (D / 16). s[k]
 // holds the piece's 16 sign/mantissa bytes, c[k] the 8 bytes that end with
 // its last code byte (4-bit: its 8 code bytes; 3-bit: 2 bytes before its 6;
 // 2-bit: 4 bytes before its 4; so no load reaches past the block, and one
@@ -286,12 +267,12 @@ __device__ __forceinline__ int escape_rows(const Cursor &c, int r0) {
 // sign/mantissa bytes). Consecutive lanes read consecutive bytes: each load
 // covers a few whole cache lines instead of one line per lane. Raw block (at
 // most kRawRows rows): s[k] holds bytes 1024 k + 16 l of the chunk's rows,
-// c[k] bytes 64 D + 512 k + 8 l (rows 32 .. 47), clamped to the last piece of
-// the rows loaded.
+// c[k] bytes 1024 kPieceRegs + 512 k + 8 l, clamped to the last piece of the
+// rows loaded.
 template <int D, bool W = kWholeRows<D>>
 struct Rows {
-    uint4 s[Shape<D>::kPieces];
-    uint2 c[Shape<D>::kPieces];
+    uint4 s[Shape<D>::kPieceRegs];
+    uint2 c[Shape<D>::kPieceRegs];
 };
 template <int D>
 struct Rows<D, true> {
@@ -343,37 +324,40 @@ __device__ __forceinline__ void load_whole_rows(Cursor &c, int r0, int rows, Row
 // merge before their use.
 template <int D>
 __device__ __forceinline__ void load_pieces(Cursor &c, int r0, int rows, Rows<D, false> &R) {
-    constexpr int NP = Shape<D>::kPieces;
+    constexpr int NP = Shape<D>::kPieces, NR = Shape<D>::kPieceRegs, NL = Shape<D>::kPieceLanes;
     const int mode = c.mode();
     const bool raw = mode == 0;
     c.lrows = rows;
     rows = max(rows, 1); // (rows <= 0 only past a plan's zero-token sentinel block: row r0 then)
     const int lane = lane_here();
     const uint8_t *b = c.blk + 8;
-    // sign/mantissa stream: 16 bytes per lane, 1,024 per register
-    int s0, se;
+    // sign/mantissa stream: 16 bytes per lane, ss per register
+    int s0, se, ss;
     // code stream: w bytes per lane (8 bytes loaded, ending with the piece's codes), cs per register
-    int c0, ce, cw;
+    int c0, ce, cw, cs;
     if (!raw) {
         const int cbytes = mode * (D / 8); // code bytes per coded row
         s0 = D + r0 * D;
         se = s0 + rows * D - 16;
+        ss = 16 * NL;
         cw = 2 * mode;
+        cs = cw * NL;
         c0 = D + c.ntok() * D + r0 * cbytes + cw - 8;
         ce = c0 + (rows * NP - 1) * cw;
     } else {
-        const int rn = 2 * D * min(rows, kRawRows); // raw bytes loaded: rows [0, 32) in s, [32, 48) in c
+        const int rn = 2 * D * min(rows, kRawRows); // raw bytes loaded: the first 1024 NR in s, the rest in c
         s0 = r0 * (2 * D);
         se = s0 + rn - 16;
+        ss = 1024;
         cw = 8;
-        c0 = s0 + 64 * D;
+        cs = 512;
         ce = s0 + rn - 8;
+        c0 = min(s0 + 1024 * NR, ce);
     }
-    const int cs = 64 * cw;
     const uint32_t ls = uint32_t(16 * lane), lc = uint32_t(cw * lane);
 #pragma unroll
-    for (int k = 0; k < NP; ++k) {
-        const int bs = min(s0 + 1024 * k, se), bc = min(c0 + cs * k, ce);
+    for (int k = 0; k < NR; ++k) {
+        const int bs = min(s0 + ss * k, se), bc = min(c0 + cs * k, ce);
         R.s[k] = ld16(b + bs + min(ls, uint32_t(se - bs)));
         R.c[k] = ld8(b + bc + min(lc, uint32_t(ce - bc)));
     }
@@ -389,7 +373,7 @@ __device__ __forceinline__ void load_rows(Cursor &c, int r0, int rows, Rows<D> &
 template <int D>
 __device__ __forceinline__ uint32_t last_loaded(const Rows<D> &R) {
     if constexpr (kWholeRows<D>) return R.r[Shape<D>::kRowRegs - 1].w;
-    else return R.c[Shape<D>::kPieces - 1].y;
+    else return R.c[Shape<D>::kPieceRegs - 1].y;
 }
 
 __device__ __forceinline__ uint32_t comp(const uint4 &v, int i) {
@@ -565,13 +549,7 @@ template <int D>
 __device__ __forceinline__ void decode_pieces(const Cursor &c, Rows<D, false> &R, uint8_t *tile, int rows,
                                               uint32_t smm) {
     constexpr int NP = Shape<D>::kPieces, RS = Shape<D>::kPieceRows, TS = Shape<D>::kTileStride;
-    // At head_dim 256 the coded pieces go in two passes of eight, the last
-    // eight registers moved into the first eight in between: one copy of each
-    // mode's body instead of two keeps the chunk loop within the instruction
-    // cache (64 KiB; the kernel's code, 149 KiB fully unrolled, is now 63 KiB
-    // at eight query rows). Four passes of four cost more in register moves
-    // than they save (c5: 1,992 against 1,936 us per step).
-    constexpr int NPASS = D == 256 ? 2 : 1, PP = NP / NPASS;
+    constexpr int NR = Shape<D>::kPieceRegs;
     const int mode = c.mode();
     const int lane = lane_here();
     if (mode != 0) {
@@ -586,54 +564,43 @@ __device__ __forceinline__ void decode_pieces(const Cursor &c, Rows<D, false> &R
             bp[2 * m + 1] = __builtin_amdgcn_perm(w, w, 0x0c030c02u) << 7;
         }
         uint8_t *dst = tile + (lane / NP) * TS + 32 * (lane % NP); // piece 0's place; piece k is RS k rows below
-#pragma unroll 1
-        for (int pass = 0; pass < NPASS; ++pass) {
-            if (mode == 4) {
+        if (mode == 4) {
 #pragma unroll
-                for (int k = 0; k < PP; ++k) {
-                    const uint32_t c0 = R.c[k].x, c1 = R.c[k].y;
-                    uint4 *o = reinterpret_cast<uint4 *>(dst + RS * k * TS);
-                    o[0] = octet(R.s[k], 0, c0 & 0x0F0F0F0Fu, (c0 >> 4) & 0x0F0F0F0Fu, bp, smm);
-                    o[1] = octet(R.s[k], 1, c1 & 0x0F0F0F0Fu, (c1 >> 4) & 0x0F0F0F0Fu, bp, smm);
-                }
-            } else if (mode == 2) {
+            for (int k = 0; k < NR; ++k) {
+                const uint32_t c0 = R.c[k].x, c1 = R.c[k].y;
+                uint4 *o = reinterpret_cast<uint4 *>(dst + RS * k * TS);
+                o[0] = octet(R.s[k], 0, c0 & 0x0F0F0F0Fu, (c0 >> 4) & 0x0F0F0F0Fu, bp, smm);
+                o[1] = octet(R.s[k], 1, c1 & 0x0F0F0F0Fu, (c1 >> 4) & 0x0F0F0F0Fu, bp, smm);
+            }
+        } else if (mode == 2) {
 #pragma unroll
-                for (int k = 0; k < PP; ++k) {
-                    uint4 *o = reinterpret_cast<uint4 *>(dst + RS * k * TS);
+            for (int k = 0; k < NR; ++k) {
+                uint4 *o = reinterpret_cast<uint4 *>(dst + RS * k * TS);
 #pragma unroll
-                    for (int h = 0; h < 2; ++h) {
-                        // the octet's 16 bits: byte p of lo / hi holds codes 2p / 2p + 1
-                        const uint32_t cw = R.c[k].y >> (16 * h);
-                        const uint32_t lo = (cw & 3u) | (((cw >> 4) & 3u) << 8) | (((cw >> 8) & 3u) << 16) |
-                                            (((cw >> 12) & 3u) << 24);
-                        const uint32_t hi = ((cw >> 2) & 3u) | (((cw >> 6) & 3u) << 8) | (((cw >> 10) & 3u) << 16) |
-                                            (((cw >> 14) & 3u) << 24);
-                        o[h] = octet(R.s[k], h, lo, hi, bp, smm);
-                    }
-                }
-            } else {
-                // 3-bit codes: octet h's 24 bits are bytes 2 + 3h .. 4 + 3h of
-                // c[k]; groups of two codes (6 bits) are spread to bytes first
-#pragma unroll
-                for (int k = 0; k < PP; ++k) {
-                    uint4 *o = reinterpret_cast<uint4 *>(dst + RS * k * TS);
-#pragma unroll
-                    for (int h = 0; h < 2; ++h) {
-                        const uint32_t w =
-                            h == 0 ? __builtin_amdgcn_alignbyte(R.c[k].y, R.c[k].x, 2u) : R.c[k].y >> 8;
-                        const uint32_t x =
-                            (w & 0x3Fu) | ((w << 2) & 0x3F00u) | ((w << 4) & 0x3F0000u) | ((w << 6) & 0x3F000000u);
-                        o[h] = octet(R.s[k], h, x & 0x07070707u, (x >> 3) & 0x07070707u, bp, smm);
-                    }
+                for (int h = 0; h < 2; ++h) {
+                    // the octet's 16 bits: byte p of lo / hi holds codes 2p / 2p + 1
+                    const uint32_t cw = R.c[k].y >> (16 * h);
+                    const uint32_t lo = (cw & 3u) | (((cw >> 4) & 3u) << 8) | (((cw >> 8) & 3u) << 16) |
+                                        (((cw >> 12) & 3u) << 24);
+                    const uint32_t hi = ((cw >> 2) & 3u) | (((cw >> 6) & 3u) << 8) | (((cw >> 10) & 3u) << 16) |
+                                        (((cw >> 14) & 3u) << 24);
+                    o[h] = octet(R.s[k], h, lo, hi, bp, smm);
                 }
             }
-            if constexpr (NPASS > 1) {
+        } else {
+            // 3-bit codes: octet h's 24 bits are bytes 2 + 3h .. 4 + 3h of
+            // c[k]; groups of two codes (6 bits) are spread to bytes first
 #pragma unroll
-                for (int k = 0; k < NP - PP; ++k) {
-                    R.s[k] = R.s[k + PP];
-                    R.c[k] = R.c[k + PP];
+            for (int k = 0; k < NR; ++k) {
+                uint4 *o = reinterpret_cast<uint4 *>(dst + RS * k * TS);
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const uint32_t w =
+                        h == 0 ? __builtin_amdgcn_alignbyte(R.c[k].y, R.c[k].x, 2u) : R.c[k].y >> 8;
+                    const uint32_t x =
+                        (w & 0x3Fu) | ((w << 2) & 0x3F00u) | ((w << 4) & 0x3F0000u) | ((w << 6) & 0x3F000000u);
+                    o[h] = octet(R.s[k], h, x & 0x07070707u, (x >> 3) & 0x07070707u, bp, smm);
                 }
-                dst += PP * RS * TS;
             }
         }
     } else {
@@ -641,8 +608,8 @@ __device__ __forceinline__ void decode_pieces(const Cursor &c, Rows<D, false> &R
         // the last one), to their rows; pieces of rows >= rows are overwritten below
         const int rn = 2 * D * max(1, min(c.lrows, kRawRows));
 #pragma unroll
-        for (int k = 0; k < NP; ++k) {
-            const int os = min(1024 * k + 16 * lane, rn - 16), oc = min(64 * D + 512 * k + 8 * lane, rn - 8);
+        for (int k = 0; k < NR; ++k) {
+            const int os = min(1024 * k + 16 * lane, rn - 16), oc = min(1024 * NR + 512 * k + 8 * lane, rn - 8);
             *reinterpret_cast<uint4 *>(tile + (os / (2 * D)) * TS + os % (2 * D)) = R.s[k];
             *reinterpret_cast<uint2 *>(tile + (oc / (2 * D)) * TS + oc % (2 * D)) = R.c[k];
         }
@@ -701,12 +668,10 @@ __device__ __forceinline__ bool patch_escapes(Cursor &c, int r0, int n, uint8_t 
     bool bad = false;
     int got = 0;
 #pragma unroll
-    for (int ij = 0; ij < 4 * kEscLoads<D>; ++ij) {
-        const int i = ij >> 2, j = ij & 3;
-        if (kEscLoads<D> > 1 && j == 0 && c.ecur + 256 * i >= nesc) break; // the block's records end before load i
-        const uint32_t rj = comp(c.erec[i], j);
+    for (int j = 0; j < 4; ++j) {
+        const uint32_t rj = comp(c.erec, j);
         const uint32_t pos = rj & 0xFFFFu, word = rj >> 16;
-        const bool mine = c.ecur + 256 * i + 4 * lane + j < nesc && pos < hi;
+        const bool mine = c.ecur + 4 * lane + j < nesc && pos < hi;
         if (mine) {
             const uint32_t row = pos / D - uint32_t(r0), col = pos % D;
             *reinterpret_cast<uint16_t *>(tile + row * TS + col * 2) = uint16_t(word);
@@ -894,7 +859,7 @@ __device__ __forceinline__ void scores_coded(const Rows<D, true> &R, const uint3
 template <int D>
 __device__ __forceinline__ bool rows_have_escapes(const Cursor &c, int r0, int n) {
     if (c.ecur >= c.nesc()) return false;
-    const uint32_t pos = __builtin_amdgcn_readfirstlane(c.erec[0].x) & 0xFFFFu;
+    const uint32_t pos = __builtin_amdgcn_readfirstlane(c.erec.x) & 0xFFFFu;
     return pos < uint32_t((r0 + n) * D);
 }
 
@@ -1038,12 +1003,11 @@ __device__ __forceinline__ float quad_f32(const uint2 &q) {
     else return hi_f32(q.y);
 }
 
-// Operands of the fold in flight: V of the lane's channels (lane + 64 h) for
-// the next quads of four tokens (quad Q in vq[Q % 3], requested two quads
+// Operands of the fold in flight: V of the lane's channel for the next quads
+// of four tokens (quad Q in vq[Q % 3], requested two quads
 // ahead) and e of four tokens (lane g < G: its row; the next quad's).
-template <int H>
 struct FoldIn {
-    uint2 vq[3][H];
+    uint2 vq[3];
     f4 e4[2];
 };
 
@@ -1062,20 +1026,17 @@ struct FoldIn {
 // time). V arrives by quads (load_tr) two quads ahead, e a quad ahead.
 template <int G, int D, int T, bool MOVE>
 __device__ __forceinline__ void fold_token(const WaveLds<G, D> &S, lds_f32 *eb, lds_f32 *ab, const uint8_t *trb,
-                                           const uint32_t (&am)[2], const float (&ea)[kGroups<G>][4], FoldIn<D / 64> &in,
-                                           f4 &a4, f4 (&acc)[kGroups<G>][D / 64], float &lvec) {
-    constexpr int NG = kGroups<G>, H = D / 64, TS = Shape<D>::kTileStride, Q = T / 4;
+                                           const uint32_t (&am)[2], const float (&ea)[kGroups<G>][4], FoldIn &in,
+                                           f4 &a4, f4 (&acc)[kGroups<G>], float &lvec) {
+    constexpr int NG = kGroups<G>, TS = Shape<D>::kTileStride, Q = T / 4;
     if constexpr (T % 4 == 0) {
         if constexpr (4 * (Q + 2) < kChunk) {
-#pragma unroll
-            for (int h = 0; h < H; ++h) in.vq[(Q + 2) % 3][h] = load_tr(trb + 4 * (Q + 2) * TS + 128 * h);
+            in.vq[(Q + 2) % 3] = load_tr(trb + 4 * (Q + 2) * TS);
         }
         if constexpr (4 * (Q + 1) < kChunk) in.e4[(Q + 1) & 1] = *reinterpret_cast<lds_f4 *>(eb + 4 * (Q + 1));
         if constexpr (MOVE) a4 = *reinterpret_cast<lds_f4 *>(ab + 4 * Q);
     }
-    float v[H];
-#pragma unroll
-    for (int h = 0; h < H; ++h) v[h] = quad_f32<T % 4>(in.vq[Q % 3][h]);
+    const float v = quad_f32<T % 4>(in.vq[Q % 3]);
     const f4 e4 = in.e4[Q & 1];
     const float el = (T % 4 == 0) ? e4.x : (T % 4 == 1) ? e4.y : (T % 4 == 2) ? e4.z : e4.w;
     if constexpr (MOVE) {
@@ -1085,9 +1046,7 @@ __device__ __forceinline__ void fold_token(const WaveLds<G, D> &S, lds_f32 *eb, 
 #pragma unroll
             for (int g = 0; g < G; ++g) av[g] = S.aT[g][T];
 #pragma unroll
-            for (int g = 0; g < G; ++g)
-#pragma unroll
-                for (int h = 0; h < H; ++h) acc[g / 4][h][g % 4] *= av[g];
+            for (int g = 0; g < G; ++g) acc[g / 4][g % 4] *= av[g];
         }
         const float al = (T % 4 == 0) ? a4.x : (T % 4 == 1) ? a4.y : (T % 4 == 2) ? a4.z : a4.w;
         lvec = fmaf(lvec, al, el);
@@ -1098,9 +1057,7 @@ __device__ __forceinline__ void fold_token(const WaveLds<G, D> &S, lds_f32 *eb, 
     // end of the unrolled fold with every token's operands held live)
     asm volatile("" : "+v"(lvec));
 #pragma unroll
-    for (int rg = 0; rg < NG; ++rg)
-#pragma unroll
-        for (int h = 0; h < H; ++h) acc[rg][h] = mfma_rank1<T % 16>(ea[rg][T / 16], v[h], acc[rg][h]);
+    for (int rg = 0; rg < NG; ++rg) acc[rg] = mfma_rank1<T % 16>(ea[rg][T / 16], v, acc[rg]);
 }
 
 // The chunk's fold in groups of 16 tokens: one uniform test of the group's
@@ -1109,87 +1066,11 @@ __device__ __forceinline__ void fold_token(const WaveLds<G, D> &S, lds_f32 *eb, 
 // four tokens issues its vector work (V widening, the l chain) and then its
 // eight products: a product right after a vector instruction, or the reverse,
 // stalls the SIMD, so few switches between the two pay.
-// Group J (tokens 16 J .. 16 J + 15) of the fold with a runtime quad index,
-// for a group where some token moves a running maximum at head_dim 256: there
-// the unrolled form (32 accumulator scalings per token, through the matrix
-// registers) would put the chunk loop far beyond the instruction cache. The
-// same operations in the same order as fold_token, four tokens per pass:
-// V of the quad by load_tr, e and alpha of the quad as 16-byte reads, every
-// row's alpha of a token that moves a maximum read one token ahead, and the
-// quad's A operands (e of the group's rows, lanes 16 q .. 16 q + 15 of
-// ea[rg][J]) moved to lanes 0 .. 15 by one ds_bpermute, so that token u of
-// the quad is block u. Then the next group's operands are requested as the
-// unrolled fold would have left them.
-template <int G, int D, int J>
-__device__ __forceinline__ void fold_group_dyn(const WaveLds<G, D> &S, lds_f32 *eb, lds_f32 *ab,
-                                               const uint8_t *trb, const uint32_t (&am)[2],
-                                               const float (&ea)[kGroups<G>][4], FoldIn<D / 64> &in,
-                                               f4 (&acc)[kGroups<G>][D / 64], float &lvec) {
-    constexpr int NG = kGroups<G>, H = D / 64, TS = Shape<D>::kTileStride;
-    const int lane = lane_id();
-    const uint32_t mw = am[J / 2];
-#pragma unroll 1
-    for (int q = 0; q < 4; ++q) {
-        const int T0 = 16 * J + 4 * q;
-        uint2 vq[H];
-#pragma unroll
-        for (int h = 0; h < H; ++h) vq[h] = load_tr(trb + T0 * TS + 128 * h);
-        const f4 e4 = *reinterpret_cast<lds_f4 *>(eb + T0);
-        const f4 a4 = *reinterpret_cast<lds_f4 *>(ab + T0);
-        float a[NG];
-#pragma unroll
-        for (int rg = 0; rg < NG; ++rg)
-            a[rg] = __int_as_float(__builtin_amdgcn_ds_bpermute(4 * (lane + 16 * q), __float_as_int(ea[rg][J])));
-        const uint32_t qb = (mw >> (T0 % 32)) & 15u; // the quad's tokens that move a maximum
-        // every row's alpha of the token (read one token ahead)
-        float an[G];
-        if (qb & 1u) {
-#pragma unroll
-            for (int g = 0; g < G; ++g) an[g] = S.aT[g][T0];
-        }
-        static_for<0, 4>([&](auto U) {
-            constexpr int u = decltype(U)::value;
-            float av[G];
-#pragma unroll
-            for (int g = 0; g < G; ++g) av[g] = an[g];
-            if constexpr (u < 3) {
-                if ((qb >> (u + 1)) & 1u) {
-#pragma unroll
-                    for (int g = 0; g < G; ++g) an[g] = S.aT[g][T0 + u + 1];
-                }
-            }
-            float v[H];
-#pragma unroll
-            for (int h = 0; h < H; ++h) v[h] = quad_f32<u>(vq[h]);
-            if ((qb >> u) & 1u) {
-#pragma unroll
-                for (int g = 0; g < G; ++g)
-#pragma unroll
-                    for (int h = 0; h < H; ++h) acc[g / 4][h][g % 4] *= av[g];
-            }
-            lvec = fmaf(lvec, a4[u], e4[u]);
-            asm volatile("" : "+v"(lvec));
-#pragma unroll
-            for (int rg = 0; rg < NG; ++rg)
-#pragma unroll
-                for (int h = 0; h < H; ++h) acc[rg][h] = mfma_rank1<u>(a[rg], v[h], acc[rg][h]);
-        });
-    }
-    constexpr int Q0 = 4 * (J + 1); // the next group's first quad
-    if constexpr (4 * Q0 < kChunk) {
-#pragma unroll
-        for (int k = 0; k < 2; ++k)
-#pragma unroll
-            for (int h = 0; h < H; ++h) in.vq[(Q0 + k) % 3][h] = load_tr(trb + 4 * (Q0 + k) * TS + 128 * h);
-        in.e4[Q0 & 1] = *reinterpret_cast<lds_f4 *>(eb + 4 * Q0);
-    }
-}
-
 template <int G, int D, int T>
 __device__ __forceinline__ void fold(const WaveLds<G, D> &S, lds_f32 *eb, lds_f32 *ab, const uint16_t *vb,
                                      const uint8_t *trb, const uint32_t (&am)[2], const float (&ea)[kGroups<G>][4],
-                                     FoldIn<D / 64> &in, f4 (&acc)[kGroups<G>][D / 64], float &lvec) {
-    constexpr int GS = 16, NG = kGroups<G>, H = D / 64;
+                                     FoldIn &in, f4 (&acc)[kGroups<G>], float &lvec) {
+    constexpr int GS = 16, NG = kGroups<G>;
     if constexpr (T < kChunk) {
         const uint32_t mw = am[T / 32];
         constexpr uint32_t gm = uint32_t(((1ull << GS) - 1ull) << (T % 32));
@@ -1199,11 +1080,9 @@ __device__ __forceinline__ void fold(const WaveLds<G, D> &S, lds_f32 *eb, lds_f3
                 fold_token<G, D, T + decltype(K)::value, false>(S, eb, ab, trb, am, ea, in, a4, acc, lvec);
             });
             static_for<0, GS / 4>([&](auto) {
-                __builtin_amdgcn_sched_group_barrier(0x002, 4 * (H + 1), 0);
-                __builtin_amdgcn_sched_group_barrier(0x008, 4 * NG * H, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, 4 * NG, 0);
             });
-        } else if constexpr (D == 256) {
-            fold_group_dyn<G, D, T / GS>(S, eb, ab, trb, am, ea, in, acc, lvec);
         } else {
             static_for<0, GS>([&](auto K) {
                 fold_token<G, D, T + decltype(K)::value, true>(S, eb, ab, trb, am, ea, in, a4, acc, lvec);
@@ -1239,18 +1118,21 @@ __device__ __forceinline__ void store_raw(const uint4 (&R)[D / 8], uint8_t *tile
     }
 }
 
+// Issue priority (0 to 3) of a wave with `left` tokens to go: the quarters of
+// its split (`quarter` tokens each) behind the current one.
+__device__ __forceinline__ int priority_of(int left, int quarter) {
+    return int(left > quarter) + int(left > 2 * quarter) + int(left > 3 * quarter);
+}
+
 template <bool XKV, int D> struct RegsOf { typedef Rows<D> T; };
 template <int D> struct RegsOf<false, D> { typedef uint4 T[D / 8]; };
 
-// At D = 64 the XKV instantiations with up to seven query rows are held to
-// three waves per SIMD (168 VGPRs), and LDS allows three workgroups of four
-// waves per CU; at D = 128 (the rows in flight take twice the registers) and
-// at eight query rows two waves per SIMD; at D = 256 a wave's tile of 64
-// full rows (33,792 bytes) leaves room for four one-wave workgroups per CU,
-// one wave per SIMD, which may then take all 512 registers.
+// The XKV instantiations with up to seven query rows are held to three waves
+// per SIMD (168 VGPRs; at D = 64 LDS allows three workgroups of four waves per
+// CU), the others to two.
 // ORDER 0: scalar/AVX2 score order; ORDER 1: AVX-512 BF16 order.
 template <int G, int D, bool XKV, int ORDER>
-constexpr int kWaveOcc = D == 256 ? 1 : (D == 64 && XKV && G < 8 ? 3 : 2);
+constexpr int kWaveOcc = XKV && G < 8 ? 3 : 2;
 
 template <int G, int D, bool XKV, int ORDER>
 __global__ __launch_bounds__(Shape<D>::kWaves * 64) __attribute__((amdgpu_waves_per_eu(kWaveOcc<G, D, XKV, ORDER>)))
@@ -1258,7 +1140,7 @@ void attn_wave_kernel(const HeadDev *__restrict__ heads, const WorkItem *__restr
                       int wpg, const BlockDesc *__restrict__ desc,
                       const uint16_t *__restrict__ q_all, float *__restrict__ out_all, float *__restrict__ lse_all,
                       float *__restrict__ ws) {
-    constexpr int TS = Shape<D>::kTileStride, H = D / 64;
+    constexpr int TS = Shape<D>::kTileStride;
     __shared__ WgLds<G, D> L;
     if (threadIdx.x < 64) kvexp_exp_table_to_lds(L.exptab);
     __syncthreads();
@@ -1308,11 +1190,9 @@ void attn_wave_kernel(const HeadDev *__restrict__ heads, const WorkItem *__restr
         klow = (kmin << 7) - 1u;
     }
 
-    f4 acc[NG][H];
+    f4 acc[NG];
 #pragma unroll
-    for (int rg = 0; rg < NG; ++rg)
-#pragma unroll
-        for (int h = 0; h < H; ++h) acc[rg][h] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int rg = 0; rg < NG; ++rg) acc[rg] = f4{0.0f, 0.0f, 0.0f, 0.0f};
     float msc[G]; // running maximum of each query row (wave-uniform)
 #pragma unroll
     for (int g = 0; g < G; ++g) msc[g] = -__builtin_inff();
@@ -1340,7 +1220,9 @@ void attn_wave_kernel(const HeadDev *__restrict__ heads, const WorkItem *__restr
     // instead lowers its priority as it gets through its split (3 for the
     // first quarter of its tokens, then 2, 1, 0): the waves that are behind
     // win the issue slots and all of a CU's waves finish at about the same
-    // time.
+    // time. (Quarters of the launch's longest split instead: c3's shape in the
+    // AVX-512 order 307 against 301 us.)
+    const int quarter = (wi.tok_end - wi.tok_begin + 3) / 4;
     constexpr bool TR = KVEXP_TRACE_ON(XKV, ORDER);
     unsigned long long ph[12] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     const unsigned long long tw0 = TR ? __builtin_readcyclecounter() : 0ull;
@@ -1358,15 +1240,14 @@ void attn_wave_kernel(const HeadDev *__restrict__ heads, const WorkItem *__restr
     (void)stamp;
     (void)after;
 
-    __builtin_amdgcn_s_setprio(3);
-    int prio = 3;
-    const int span = wi.tok_end - wi.tok_begin;
+    int prio = -1;
     while (t < wi.tok_end) {
         const int ln = lane_here(); // this chunk's lane index (see lane_here)
         {
-            const int want = 3 - min(3, ((t - wi.tok_begin) * 4) / max(span, 1));
+            const int want = priority_of(wi.tok_end - t, quarter);
             if (want != prio) {
-                if (want == 2) __builtin_amdgcn_s_setprio(2);
+                if (want == 3) __builtin_amdgcn_s_setprio(3);
+                else if (want == 2) __builtin_amdgcn_s_setprio(2);
                 else if (want == 1) __builtin_amdgcn_s_setprio(1);
                 else __builtin_amdgcn_s_setprio(0);
                 prio = want;
@@ -1550,19 +1431,14 @@ void attn_wave_kernel(const HeadDev *__restrict__ heads, const WorkItem *__restr
             // the loads are issued on every chunk (the last one re-reads its
             // own final row), the next K rows before the next V rows: the K
             // decode can then wait for its loads while the V loads stay in
-            // flight. At head_dim 64 and 128 the K rows are requested before
-            // this chunk's V decode (which waits only for the older V rows;
-            // c2 and c4 about 1 % faster), at 256 after it (no gain measured
-            // there, where one wave per SIMD has registers to spare).
+            // flight. The K rows are requested before this chunk's V decode
+            // (which waits only for the older V rows; c2 about 1 % faster).
             const int tp = min(tn, wi.tok_end - 1);
-            auto request_k = [&]() {
-                if (tp >= kc.t1) enter_block(kc, kc.d + 1, kc.t1);
-                stamp(7); // next K block entered
-                block_vectors<D>(kc);
-                load_rows<D>(kc, tp - kc.t0, min(kChunk, min(kc.t1, wi.tok_end) - tp), RK);
-                stamp(8); // next K rows requested
-            };
-            if constexpr (D <= 128) request_k();
+            if (tp >= kc.t1) enter_block(kc, kc.d + 1, kc.t1);
+            stamp(7); // next K block entered
+            block_vectors<D>(kc);
+            load_rows<D>(kc, tp - kc.t0, min(kChunk, min(kc.t1, wi.tok_end) - tp), RK);
+            stamp(8); // next K rows requested
             if constexpr (kWholeRows<D>) {
                 if (vc.mode() != 0) {
                     base_pairs<D>(vc, S.bp);
@@ -1574,7 +1450,6 @@ void attn_wave_kernel(const HeadDev *__restrict__ heads, const WorkItem *__restr
             stamp(5); // V rows decoded
             patch_escapes<D>(vc, t - vc.t0, n, S.tile);
             stamp(6); // V escapes written
-            if constexpr (D > 128) request_k();
             if (tp >= vc.t1) enter_block(vc, vc.d + 1, vc.t1);
             stamp(9); // next V block entered
             block_vectors<D>(vc);
@@ -1609,13 +1484,11 @@ void attn_wave_kernel(const HeadDev *__restrict__ heads, const WorkItem *__restr
             const int gl = min(ln & 7, G - 1); // lanes >= G read a row they do not use
             lds_f32 *eb = (lds_f32 *)&S.eT[gl][0];
             lds_f32 *ab = (lds_f32 *)&S.aT[gl][0];
-            FoldIn<H> in;
+            FoldIn in;
             const uint16_t *vb = reinterpret_cast<const uint16_t *>(S.tile) + ln; // channel lane of token 0
             const uint8_t *trb = S.tile + tr_lane_offset<D>(ln);                   // the lane's load_tr address
 #pragma unroll
-            for (int k = 0; k < 2; ++k)
-#pragma unroll
-                for (int h = 0; h < H; ++h) in.vq[k][h] = load_tr(trb + 4 * k * TS + 128 * h);
+            for (int k = 0; k < 2; ++k) in.vq[k] = load_tr(trb + 4 * k * TS);
             in.e4[0] = *reinterpret_cast<lds_f4 *>(eb);
             // amask as two words behind an empty asm: the group tests stay
             // 32-bit scalar compares (not a 64-bit vector compare against a
@@ -1625,7 +1498,7 @@ void attn_wave_kernel(const HeadDev *__restrict__ heads, const WorkItem *__restr
             fold<G, D, 0>(S, eb, ab, vb, trb, am, ea, in, acc, lvec);
         }
         wave_sync();
-        after(__float_as_uint(acc[0][0].x));
+        after(__float_as_uint(acc[0].x));
         stamp(11); // fold done
         t = tn;
     }
@@ -1651,9 +1524,7 @@ void attn_wave_kernel(const HeadDev *__restrict__ heads, const WorkItem *__restr
 #pragma unroll
         for (int g = 0; g < G; ++g) {
             const float l = readlane_f32(lvec, g);
-#pragma unroll
-            for (int h = 0; h < H; ++h)
-                out_all[(size_t(hd.q_row) + g) * D + 64 * h + lane] = acc[g / 4][h][g % 4] * (1.0f / l);
+            if (D == 64 || lane < D) out_all[(size_t(hd.q_row) + g) * D + lane] = acc[g / 4][g % 4] * (1.0f / l);
         }
         if (lse_all != nullptr && lane < G) lse_all[hd.q_row + lane] = mv + logf(lvec);
         return;
@@ -1665,8 +1536,7 @@ void attn_wave_kernel(const HeadDev *__restrict__ heads, const WorkItem *__restr
     }
 #pragma unroll
     for (int g = 0; g < G; ++g)
-#pragma unroll
-        for (int h = 0; h < H; ++h) slot[2 * kSlotQ + g * D + 64 * h + lane] = acc[g / 4][h][g % 4];
+        if (D == 64 || lane < D) slot[2 * kSlotQ + g * D + lane] = acc[g / 4][g % 4];
 }
 
 // Waves (merge items) per workgroup of the merge kernel: one, so that a
@@ -1676,12 +1546,14 @@ constexpr int kMergeWaves = 1;
 
 // Ordered merge of a head's split states (softmax.hpp:16-30 merge_state,
 // left to right in split order; dispatch.cpp:98-103), then out = acc * (1/l)
-// and lse = m + log l. One wave per merge item (device head, query row): lane
-// = channel (channels lane + 64 h) for the accumulators. A separate launch,
+// and lse = m + log l. One wave per merge item (device head, query row) and
+// 64 channels (blockIdx.y; lane = channel): at head_dim 256 four waves take
+// a row's channels side by side, each over 64 splits per batch, where one
+// wave for the row held 32 splits' rows at a time. A separate launch,
 // so the slots written by the split kernel are visible without fences.
 //
 // Splits go in batches of kMergeBatch. In a batch, lane j first loads m and
-// l of split s0 + j, then every lane its channels of the batch's
+// l of split s0 + j, then every lane its channel of the batch's
 // accumulator rows (all loads in flight together). While the rows arrive,
 // lane j computes the running maximum after split s0 + j (a wave scan; the
 // maximum is exact in any grouping), the two exponentials of its merge step
@@ -1690,11 +1562,13 @@ constexpr int kMergeWaves = 1;
 // read them four splits at a time (one broadcast LDS read per operand) and
 // take one fused multiply-add per split and channel, as merge_state does.
 // The first batch starts from split 0's state, as dispatch.cpp does.
+constexpr int kMergeBatch = 64;
+
 template <int D>
 __global__ __launch_bounds__(kMergeWaves * 64) void wave_merge_kernel(
     const MergeItem *__restrict__ mitems, int n_mitems, MergeItem uni, float *__restrict__ out_all,
     float *__restrict__ lse_all, const float *__restrict__ ws) {
-    constexpr int H = D / 64, B = Shape<D>::kMergeBatch, SF = Shape<D>::kSlotFloats;
+    constexpr int B = kMergeBatch, SF = Shape<D>::kSlotFloats;
     static_assert(B % 4 == 0 && B <= kWave, "one split per lane, read four at a time");
     __shared__ uint64_t tab[32];
     __shared__ float stage[kMergeWaves][3][B]; // per wave: e1, e2 and l * e2 of the batch's splits
@@ -1704,6 +1578,8 @@ __global__ __launch_bounds__(kMergeWaves * 64) void wave_merge_kernel(
     const int w = int(threadIdx.x) >> 6;
     const int mi = __builtin_amdgcn_readfirstlane(int(blockIdx.x) * kMergeWaves + w);
     if (mi >= n_mitems) return;
+    const int ch = 64 * int(blockIdx.y) + lane;   // the lane's channel
+    const int cl = D % 64 == 0 ? ch : min(ch, D - 1);
     // uni.g > 0: item i is (uni.ws_base + k uni.n_splits, uni.n_splits,
     // uni.q_row + k uni.g, i - k uni.g) with k = i / uni.g, so the slots'
     // loads need not wait for the item's
@@ -1718,19 +1594,16 @@ __global__ __launch_bounds__(kMergeWaves * 64) void wave_merge_kernel(
     const float *slots = ws + size_t(it.ws_base) * SF;
     const int n = it.n_splits;
     lds_f32 *st = (lds_f32 *)&stage[w][0][0];
-    float a[H] = {};
+    float a = 0.0f;
     float mf = 0.0f, lf = 0.0f;
     for (int s0 = 0; s0 < n; s0 += B) {
         const int cnt = min(B, n - s0);
         const float *ls = slots + size_t(s0 + min(lane, cnt - 1)) * SF;
         const float ms = lane < cnt ? ls[g] : -__builtin_inff();
         const float lb = ls[kSlotQ + g];
-        float ab[B][H];
+        float ab[B];
 #pragma unroll
-        for (int j = 0; j < B; ++j)
-#pragma unroll
-            for (int c = 0; c < H; ++c)
-                ab[j][c] = slots[size_t(s0 + min(j, cnt - 1)) * SF + 2 * kSlotQ + g * D + 64 * c + lane];
+        for (int j = 0; j < B; ++j) ab[j] = slots[size_t(s0 + min(j, cnt - 1)) * SF + 2 * kSlotQ + g * D + cl];
         const int j0 = s0 == 0 ? 1 : 0; // split 0 is the starting state
         if (s0 == 0) mf = readlane_f32(ms, 0);
         const float mm = fmaxf(wave_scan_max(ms), mf);
@@ -1746,8 +1619,7 @@ __global__ __launch_bounds__(kMergeWaves * 64) void wave_merge_kernel(
         wave_sync();
         if (s0 == 0) {
             lf = readlane_f32(lb, 0);
-#pragma unroll
-            for (int c = 0; c < H; ++c) a[c] = ab[0][c];
+            a = ab[0];
         }
 #pragma unroll
         for (int jq = 0; jq < B; jq += 4) {
@@ -1758,17 +1630,15 @@ __global__ __launch_bounds__(kMergeWaves * 64) void wave_merge_kernel(
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 if (jq + k >= j0 && jq + k < cnt) {
-#pragma unroll
-                    for (int c = 0; c < H; ++c) a[c] = fmaf(a[c], x1[k], ab[jq + k][c] * x2[k]);
+                    a = fmaf(a, x1[k], ab[jq + k] * x2[k]);
                     lf = fmaf(lf, x1[k], pl[k]);
                 }
             }
         }
         wave_sync(); // the next batch overwrites the stage
     }
-#pragma unroll
-    for (int c = 0; c < H; ++c) out_all[(size_t(it.q_row) + g) * D + 64 * c + lane] = a[c] * (1.0f / lf);
-    if (lse_all != nullptr && lane == 0) lse_all[it.q_row + g] = mf + logf(lf);
+    if (D % 64 == 0 || ch < D) out_all[(size_t(it.q_row) + g) * D + ch] = a * (1.0f / lf);
+    if (lse_all != nullptr && ch == 0) lse_all[it.q_row + g] = mf + logf(lf);
 }
 
 } // namespace wave
@@ -1815,20 +1685,20 @@ static hipError_t launch_wave_x(int G, const HeadDev *heads, const WorkItem *ite
 // In a phase-trace build each unit also exports a reader of its own copy of
 // the trace array (a file-scope device array exists once per unit).
 #if defined(KVEXP_PHASE_TRACE)
-#define KVEXP_WAVE_TRACE_READER(D, O)                                                                                \
-    hipError_t attention_wave_d##D##_o##O##_trace_read(unsigned long long *host, size_t n) {                       \
+#define KVEXP_TRACE_READER(K, D, O)                                                                                \
+    hipError_t attention_##K##_d##D##_o##O##_trace_read(unsigned long long *host, size_t n) {                       \
         return hipMemcpyFromSymbol(host, HIP_SYMBOL(kvexp_dev::wave::g_phase_trace), n * 8);                        \
     }
 #else
-#define KVEXP_WAVE_TRACE_READER(D, O)
+#define KVEXP_TRACE_READER(K, D, O)
 #endif
 #define KVEXP_WAVE_UNIT(D, O)                                                                                        \
     hipError_t attention_wave_d##D##_o##O(bool xkv, int G, const HeadDev *heads, const WorkItem *items,             \
-                                         int n_items, int wpg, const BlockDesc *desc, const uint16_t *q,           \
-                                         float *out, float *lse, float *ws, hipStream_t s) {                       \
+                                         int n_items, int wpg, const BlockDesc *desc,                  \
+                                         const uint16_t *q, float *out, float *lse, float *ws, hipStream_t s) {    \
         return xkv ? launch_wave_x<D, true, O>(G, heads, items, n_items, wpg, desc, q, out, lse, ws, s)             \
                    : launch_wave_x<D, false, O>(G, heads, items, n_items, wpg, desc, q, out, lse, ws, s);           \
     }                                                                                                                \
-    KVEXP_WAVE_TRACE_READER(D, O)
+    KVEXP_TRACE_READER(wave, D, O)
 
 } // namespace kvexp_launch

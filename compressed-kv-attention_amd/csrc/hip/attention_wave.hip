@@ -6,58 +6,91 @@
 namespace kvexp_launch {
 using namespace kvexp_dev;
 
+// The split kernel of each head_dim: the one-wave kernel (attention_wave.h) at
+// 32 and 64, the team kernel (attention_team.h) at the larger ones; the AVX-512
+// order needs a multiple of 32. X(head_dim): the sizes with a kernel.
+#define KVEXP_WAVE_DIMS(X) X(32) X(64)
+#define KVEXP_TEAM_DIMS_32(X) X(96) X(128) X(160) X(192) X(224) X(256)
+#define KVEXP_TEAM_DIMS_16(X) X(80) X(112)
+
 #define KVEXP_WAVE_DECL(D, O)                                                                                        \
     hipError_t attention_wave_d##D##_o##O(bool xkv, int G, const HeadDev *heads, const WorkItem *items,             \
-                                         int n_items, int wpg, const BlockDesc *desc, const uint16_t *q,           \
+                                         int n_items, int wpg, const BlockDesc *desc,                  \
+                                         const uint16_t *q, float *out, float *lse, float *ws, hipStream_t s);
+#define KVEXP_TEAM_DECL(D, O)                                                                                        \
+    hipError_t attention_team_d##D##_o##O(bool xkv, int G, const HeadDev *heads, const WorkItem *items,             \
+                                         int n_items, const BlockDesc *desc, const uint16_t *q,        \
                                          float *out, float *lse, float *ws, hipStream_t s);
-KVEXP_WAVE_DECL(64, 0)
-KVEXP_WAVE_DECL(64, 1)
-KVEXP_WAVE_DECL(128, 0)
-KVEXP_WAVE_DECL(128, 1)
-KVEXP_WAVE_DECL(256, 0)
-KVEXP_WAVE_DECL(256, 1)
+#define KVEXP_WAVE_DECL_BOTH(D) KVEXP_WAVE_DECL(D, 0) KVEXP_WAVE_DECL(D, 1)
+#define KVEXP_TEAM_DECL_BOTH(D) KVEXP_TEAM_DECL(D, 0) KVEXP_TEAM_DECL(D, 1)
+#define KVEXP_TEAM_DECL_0(D) KVEXP_TEAM_DECL(D, 0)
+KVEXP_WAVE_DIMS(KVEXP_WAVE_DECL_BOTH)
+KVEXP_TEAM_DIMS_32(KVEXP_TEAM_DECL_BOTH)
+KVEXP_TEAM_DIMS_16(KVEXP_TEAM_DECL_0)
 
-// head_dim 64, 128 and 256, both score orders (the host sends other sizes
-// to the general kernel).
-bool wave_supports(int dim) { return dim == 64 || dim == 128 || dim == 256; }
+#define KVEXP_DIM_CASE(D) case D:
 
-// Waves per workgroup of the split kernel (consecutive work items share a
-// workgroup).
-int wave_waves_per_wg(int dim) {
-    return dim == 64 ? wave::Shape<64>::kWaves : (dim == 128 ? wave::Shape<128>::kWaves : wave::Shape<256>::kWaves);
+// The head_dims of these kernels, both score orders where the order allows
+// the size (the host sends other sizes to the general kernel).
+bool wave_supports(int dim) {
+    switch (dim) {
+        KVEXP_WAVE_DIMS(KVEXP_DIM_CASE)
+        KVEXP_TEAM_DIMS_32(KVEXP_DIM_CASE)
+        KVEXP_TEAM_DIMS_16(KVEXP_DIM_CASE)
+        return true;
+    default: return false;
+    }
 }
+
+// Work items per workgroup of the split kernel: consecutive ones share a
+// workgroup of the one-wave kernel; a team is a workgroup.
+int wave_waves_per_wg(int dim) { return dim <= 64 ? wave::Shape<64>::kWaves : 1; }
 
 hipError_t wave_merge(int dim, const MergeItem *mitems, int n_mitems, const MergeItem &uni, float *out, float *lse,
                       const float *ws, hipStream_t s) {
     if (n_mitems <= 0) return hipSuccess;
     const int grid = (n_mitems + wave::kMergeWaves - 1) / wave::kMergeWaves;
-    if (dim == 64)
-        hipLaunchKernelGGL(wave::wave_merge_kernel<64>, dim3(grid), dim3(wave::kMergeWaves * 64), 0, s, mitems, n_mitems, uni, out,
-                           lse, ws);
-    else if (dim == 128)
-        hipLaunchKernelGGL(wave::wave_merge_kernel<128>, dim3(grid), dim3(wave::kMergeWaves * 64), 0, s, mitems, n_mitems, uni, out,
-                           lse, ws);
-    else if (dim == 256)
-        hipLaunchKernelGGL(wave::wave_merge_kernel<256>, dim3(grid), dim3(wave::kMergeWaves * 64), 0, s, mitems, n_mitems, uni, out,
-                           lse, ws);
-    else
-        return hipErrorInvalidValue;
+#define KVEXP_MERGE_CASE(D)                                                                                          \
+    case D:                                                                                                          \
+        hipLaunchKernelGGL(wave::wave_merge_kernel<D>, dim3(grid, (D + 63) / 64), dim3(wave::kMergeWaves * 64), 0, s, \
+                           mitems, n_mitems, uni, out, lse, ws);                                                             \
+        break;
+    switch (dim) {
+        KVEXP_WAVE_DIMS(KVEXP_MERGE_CASE)
+        KVEXP_TEAM_DIMS_32(KVEXP_MERGE_CASE)
+        KVEXP_TEAM_DIMS_16(KVEXP_MERGE_CASE)
+    default: return hipErrorInvalidValue;
+    }
+#undef KVEXP_MERGE_CASE
     return hipGetLastError();
 }
 
 hipError_t attention_wave(bool xkv, int order, int G, int dim, const HeadDev *heads, const WorkItem *items,
-                          int n_items, int wpg, const BlockDesc *desc, const uint16_t *q, float *out, float *lse,
-                          float *ws, hipStream_t s) {
+                          int n_items, int wpg, const BlockDesc *desc, const uint16_t *q, float *out,
+                          float *lse, float *ws, hipStream_t s) {
     if (n_items <= 0) return hipSuccess;
     if (order != 0 && order != 1) return hipErrorInvalidValue;
 #define KVEXP_WAVE_CASE(D)                                                                                           \
-    if (dim == D)                                                                                                    \
+    case D:                                                                                                          \
         return order == 0 ? attention_wave_d##D##_o0(xkv, G, heads, items, n_items, wpg, desc, q, out, lse, ws, s)   \
                           : attention_wave_d##D##_o1(xkv, G, heads, items, n_items, wpg, desc, q, out, lse, ws, s);
-    KVEXP_WAVE_CASE(64)
-    KVEXP_WAVE_CASE(128)
-    KVEXP_WAVE_CASE(256)
+#define KVEXP_TEAM_CASE_32(D)                                                                                        \
+    case D:                                                                                                          \
+        return order == 0 ? attention_team_d##D##_o0(xkv, G, heads, items, n_items, desc, q, out, lse, ws, s)        \
+                          : attention_team_d##D##_o1(xkv, G, heads, items, n_items, desc, q, out, lse, ws, s);
+#define KVEXP_TEAM_CASE_16(D)                                                                                        \
+    case D:                                                                                                          \
+        if (order != 0) break;                                                                                       \
+        return attention_team_d##D##_o0(xkv, G, heads, items, n_items, desc, q, out, lse, ws, s);
+    switch (dim) {
+        KVEXP_WAVE_DIMS(KVEXP_WAVE_CASE)
+        KVEXP_TEAM_DIMS_32(KVEXP_TEAM_CASE_32)
+        KVEXP_TEAM_DIMS_16(KVEXP_TEAM_CASE_16)
+    default: break;
+    }
 #undef KVEXP_WAVE_CASE
+#undef KVEXP_TEAM_CASE_32
+#undef KVEXP_TEAM_CASE_16
     return hipErrorInvalidValue;
 }
 
@@ -66,16 +99,16 @@ hipError_t attention_wave(bool xkv, int order, int G, int dim, const HeadDev *he
 #if defined(KVEXP_PHASE_TRACE)
 namespace kvexp_launch {
 hipError_t attention_wave_d64_o0_trace_read(unsigned long long *host, size_t n);
-hipError_t attention_wave_d128_o0_trace_read(unsigned long long *host, size_t n);
-hipError_t attention_wave_d256_o0_trace_read(unsigned long long *host, size_t n);
+hipError_t attention_team_d128_o0_trace_read(unsigned long long *host, size_t n);
+hipError_t attention_team_d256_o0_trace_read(unsigned long long *host, size_t n);
 } // namespace kvexp_launch
 // Copies the phase trace of the last traced launch at head_dim `dim` (n
 // words) to the host (trace builds only).
 extern "C" int kvexp_hip_phase_trace_read(unsigned long long *host, size_t n, int dim) {
     using namespace kvexp_launch;
     if (dim == 64) return int(attention_wave_d64_o0_trace_read(host, n));
-    if (dim == 128) return int(attention_wave_d128_o0_trace_read(host, n));
-    if (dim == 256) return int(attention_wave_d256_o0_trace_read(host, n));
+    if (dim == 128) return int(attention_team_d128_o0_trace_read(host, n));
+    if (dim == 256) return int(attention_team_d256_o0_trace_read(host, n));
     return int(hipErrorInvalidValue);
 }
 #endif
