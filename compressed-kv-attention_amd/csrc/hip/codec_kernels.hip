@@ -4,8 +4,8 @@
 // include/kvexp/scan.hpp:125-155): one workgroup per block. A coded element
 // is bf16_from_delta(base[d], code, sm) unless its code is the all-ones
 // sentinel, in which case it is the next escape word of the block in scan
-// order; the escape rank of each element comes from a workgroup prefix sum
-// of per-thread sentinel counts.
+// order; the escape rank of each element comes from prefix sums of per-lane
+// sentinel counts.
 //
 // Encode (reference src/codec.cpp:18-164), three launches:
 //   1. per block: exponent histogram per channel, the smallest base that
@@ -29,12 +29,179 @@ constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / kWave;
 
 // ----------------------------------------------------------------- decode --
+// Whether the containers' index covers `need` tokens (0: not asked); if not,
+// nothing is decoded and kStShort is raised.
+__device__ __forceinline__ bool decode_covers(const int32_t *first, int n_blocks, int need, uint32_t *status) {
+    if (need == 0 || first[n_blocks] >= need) return true;
+    if (threadIdx.x == 0) atomicOr(status, kStShort);
+    return false;
+}
+
+// head_dim a multiple of 8: a block in segments of 16,384 elements, a quarter
+// of a segment's octets (8 channels of one row) to each wave, lane-strided,
+// so that all of a segment's codes and sign/mantissa bytes are in flight
+// before the first is used (24 registers per lane), and one octet is one
+// 16-byte store. The ranks need one barrier per segment (the waves' totals);
+// only a wave step that holds a sentinel scans its lanes. The work is a
+// streaming copy (1.5 bytes in, 2 out per element), so the aim is bytes in
+// flight and whole-line accesses; two barriers and a scan per 1,024 elements,
+// with byte loads, took 66 us for one head_dim-128 tensor of 131,072 tokens.
+constexpr int kDecSteps = 8;                              // octets per lane per segment
+constexpr int kDecSegment = 8 * kDecSteps * kThreads;     // elements
+
+typedef uint32_t dec_u32 __attribute__((aligned(1)));
+typedef uint16_t dec_u16 __attribute__((aligned(1)));
+typedef uint32_t dec_u32x2 __attribute__((ext_vector_type(2), aligned(1)));
+typedef uint32_t dec_u32x4 __attribute__((ext_vector_type(4), aligned(1)));
+
+// Two BF16 from sign/mantissa bytes lb, lb + 1 of sm, codes k, k + 1 of cw
+// (`mode` bits each) and base bytes lb, lb + 1 of b (see bf16_join).
+__device__ __forceinline__ uint32_t dec_pair(uint32_t sm, uint32_t b, int lb, uint32_t c0, uint32_t c1) {
+    const uint32_t e0 = ((b >> (8 * lb)) & 0xFFu) + c0, e1 = ((b >> (8 * lb + 8)) & 0xFFu) + c1;
+    const uint32_t e = ((e0 & 0xFFu) << 7) | ((e1 & 0xFFu) << 23);
+    const uint32_t hb = uint32_t(lb + 1), l = uint32_t(lb);
+    const uint32_t s = __builtin_amdgcn_perm(sm, sm, (hb << 24) | (hb << 16) | (l << 8) | l);
+    return (s & 0x807F807Fu) | e;
+}
+
+template <int MODE>
+__device__ __forceinline__ uint32_t dec_codes(const uint8_t *codes, int o) {
+    if (MODE == 4) return *reinterpret_cast<const dec_u32 *>(codes + 4 * size_t(o));
+    if (MODE == 2) return *reinterpret_cast<const dec_u16 *>(codes + 2 * size_t(o));
+    const uint8_t *p = codes + 3 * size_t(o);
+    return uint32_t(*reinterpret_cast<const dec_u16 *>(p)) | (uint32_t(p[2]) << 16);
+}
+
+// One coded block: `octets` of its octets (the rows asked for) to out; every
+// thread of the workgroup calls it. tmp: kWaves ints in LDS.
+template <int MODE>
+__device__ __forceinline__ uint32_t decode_coded(const uint8_t *p, const BlockHdr &h, int dim, int octets, uint16_t *out,
+                                                 int *tmp) {
+    constexpr uint32_t sentinel = (1u << MODE) - 1u;
+    const uint8_t *sm = p + dim;
+    const uint8_t *codes = sm + size_t(h.n_tokens) * size_t(dim);
+    const uint8_t *esc = codes + exp_payload_bytes(h.n_tokens, dim, MODE);
+    const int lane = lane_id(), w = int(threadIdx.x) >> 6, cpr = dim / 8;
+    uint32_t bad = 0;
+    int carry = 0; // sentinels of earlier segments
+    for (int seg = 0; seg < octets; seg += kDecSegment / 8) {
+        const int o0 = seg + w * (kDecSteps * kWave) + lane; // the lane's first octet
+        uint32_t cw[kDecSteps];
+        uint2 s8[kDecSteps], b8[kDecSteps];
+        int col = o0 % cpr;
+        const int step = kWave % cpr;
+#pragma unroll
+        for (int k = 0; k < kDecSteps; ++k) {
+            const int o = min(o0 + kWave * k, octets - 1);
+            cw[k] = dec_codes<MODE>(codes, o);
+            const dec_u32x2 x = *reinterpret_cast<const dec_u32x2 *>(sm + 8 * size_t(o));
+            s8[k] = make_uint2(x.x, x.y);
+        }
+#pragma unroll
+        for (int k = 0; k < kDecSteps; ++k) {
+            const dec_u32x2 x = *reinterpret_cast<const dec_u32x2 *>(p + 8 * col);
+            b8[k] = make_uint2(x.x, x.y);
+            col += step;
+            if (col >= cpr) col -= cpr;
+        }
+        // ranks: the wave's first one from the earlier waves' totals
+        int rank = carry;
+        if (h.n_escape > 0) {
+            int mine = 0;
+#pragma unroll
+            for (int k = 0; k < kDecSteps; ++k)
+                mine += o0 + kWave * k < octets ? unit_sentinels(cw[k], MODE) : 0;
+            const int total = wave_sum_i32(mine);
+            __syncthreads(); // the last segment's totals are read
+            if (lane == 0) tmp[w] = total;
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < kWaves; ++i) {
+                rank += i < w ? tmp[i] : 0;
+                carry += tmp[i];
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < kDecSteps; ++k) {
+            const int o = o0 + kWave * k;
+            const bool in = o < octets;
+            const uint32_t c = cw[k];
+            auto code = [&](int i) { return (c >> (MODE * i)) & sentinel; };
+            uint4 v;
+            v.x = dec_pair(s8[k].x, b8[k].x, 0, code(0), code(1));
+            v.y = dec_pair(s8[k].x, b8[k].x, 2, code(2), code(3));
+            v.z = dec_pair(s8[k].y, b8[k].y, 0, code(4), code(5));
+            v.w = dec_pair(s8[k].y, b8[k].y, 2, code(6), code(7));
+            const int n = in ? unit_sentinels(c, MODE) : 0;
+            if (__ballot(n != 0) != 0) {
+                const int incl = wave_scan_add(n);
+                int r = rank + incl - n;
+                rank += __builtin_amdgcn_readlane(incl, kWave - 1);
+                if (n != 0) {
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) {
+                        if (code(i) != sentinel) continue;
+                        uint32_t word = 0;
+                        if (r < h.n_escape) word = *reinterpret_cast<const dec_u16 *>(esc + 2 * size_t(r));
+                        else bad = kStEscape;
+                        ++r;
+                        uint32_t &d = i < 2 ? v.x : (i < 4 ? v.y : (i < 6 ? v.z : v.w));
+                        d = (i & 1) ? (d & 0xFFFFu) | (word << 16) : (d & 0xFFFF0000u) | word;
+                    }
+                }
+            }
+            if (in) *reinterpret_cast<dec_u32x4 *>(out + 8 * size_t(o)) = dec_u32x4{v.x, v.y, v.z, v.w};
+        }
+    }
+    return bad;
+}
+
+__global__ __launch_bounds__(kThreads) void decode_octets_kernel(const uint8_t *__restrict__ blob, uint64_t bytes,
+                                                                const int64_t *__restrict__ offs,
+                                                                const int32_t *__restrict__ first, int n_blocks,
+                                                                int need, int seq, int dim,
+                                                                uint16_t *__restrict__ out,
+                                                                uint32_t *__restrict__ status) {
+    __shared__ int tmp[kWaves];
+    const int b = int(blockIdx.x);
+    const int t0 = first[b], want = first[b + 1] - t0;
+    const int64_t off = offs[b];
+    if (!decode_covers(first, n_blocks, need, status)) return;
+    BlockHdr h;
+    const uint32_t st = check_block(blob, bytes, off, dim, want, &h);
+    if (st != 0u) {
+        if (threadIdx.x == 0) atomicOr(status, st);
+        return;
+    }
+    const int rows = min(want, seq - t0);
+    if (rows <= 0) return;
+    const uint8_t *p = blob + off + 8;
+    uint16_t *o = out + size_t(t0) * size_t(dim);
+    const int octets = rows * dim / 8;
+    uint32_t bad = 0;
+    if (h.mode == 0) {
+        for (int i = int(threadIdx.x); i < octets; i += kThreads)
+            *reinterpret_cast<dec_u32x4 *>(o + 8 * size_t(i)) =
+                *reinterpret_cast<const dec_u32x4 *>(p + 16 * size_t(i));
+    } else if (h.mode == 4) {
+        bad = decode_coded<4>(p, h, dim, octets, o, tmp);
+    } else if (h.mode == 2) {
+        bad = decode_coded<2>(p, h, dim, octets, o, tmp);
+    } else {
+        bad = decode_coded<3>(p, h, dim, octets, o, tmp);
+    }
+    if (bad) atomicOr(status, bad);
+}
+
+// The other head_dims (multiples of 4): four elements per thread and step.
 __global__ __launch_bounds__(kThreads) void decode_blocks_kernel(const uint8_t *__restrict__ blob, uint64_t bytes,
                                                                 const int64_t *__restrict__ offs,
-                                                                const int32_t *__restrict__ first, int seq, int dim,
+                                                                const int32_t *__restrict__ first, int n_blocks,
+                                                                int need, int seq, int dim,
                                                                 uint16_t *__restrict__ out,
                                                                 uint32_t *__restrict__ status) {
     __shared__ int scan_tmp[kWaves];
+    if (!decode_covers(first, n_blocks, need, status)) return;
     const int b = int(blockIdx.x);
     const int t0 = first[b];
     const int want = first[b + 1] - t0;
@@ -54,14 +221,13 @@ __global__ __launch_bounds__(kThreads) void decode_blocks_kernel(const uint8_t *
         for (int i = int(threadIdx.x); i < total; i += kThreads) o[i] = uint16_t(load_u16_any(p + 2 * i));
         return;
     }
-    const int mode = h.mode;
-    const int U = code_unit(mode);
+    const int mode = h.mode; // 2 or 4 (3-bit blocks have head_dim % 8 == 0)
     const uint32_t sentinel = (1u << mode) - 1u;
     const uint8_t *base = p;
     const uint8_t *sm = p + dim;
     const uint8_t *codes = sm + size_t(h.n_tokens) * size_t(dim);
     const uint8_t *esc = codes + exp_payload_bytes(h.n_tokens, dim, mode);
-    const int units = total / U; // dim % 4 == 0 (dim % 8 == 0 for 3-bit codes)
+    const int units = total / 4;
     int carry = 0;
     uint32_t bad = 0;
     for (int r = 0; r < units; r += kThreads) {
@@ -80,12 +246,11 @@ __global__ __launch_bounds__(kThreads) void decode_blocks_kernel(const uint8_t *
             carry += tot;
         }
         if (act) {
-            const int e0 = U * u;
+            const int e0 = 4 * u;
             const int d0 = e0 % dim;
-            uint32_t v[8];
+            uint32_t v[4];
 #pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                if (k >= U) break;
+            for (int k = 0; k < 4; ++k) {
                 const uint32_t code = unit_code(cw, mode, k);
                 if (code == sentinel) {
                     if (rank < h.n_escape) {
@@ -99,12 +264,10 @@ __global__ __launch_bounds__(kThreads) void decode_blocks_kernel(const uint8_t *
                     v[k] = bf16_join(uint32_t(base[d0 + k]) + code, load_u8(sm + e0 + k));
                 }
             }
-            for (int k = 0; k < U; k += 4) {
-                uint2 w;
-                w.x = v[k] | (v[k + 1] << 16);
-                w.y = v[k + 2] | (v[k + 3] << 16);
-                *reinterpret_cast<uint2 *>(o + e0 + k) = w;
-            }
+            uint2 w;
+            w.x = v[0] | (v[1] << 16);
+            w.y = v[2] | (v[3] << 16);
+            *reinterpret_cast<uint2 *>(o + e0) = w;
         }
     }
     if (bad) atomicOr(status, bad);
@@ -1358,11 +1521,12 @@ __global__ __launch_bounds__(256) void expf_kernel(const float *__restrict__ x, 
 namespace kvexp_launch {
 using namespace kvexp_dev;
 
+// need: tokens that the index must cover for anything to be decoded (0: any)
 hipError_t decode(const uint8_t *blob, uint64_t bytes, const int64_t *offs, const int32_t *first, int n_blocks,
-                  int seq, int dim, uint16_t *out, uint32_t *status, hipStream_t s) {
+                  int need, int seq, int dim, uint16_t *out, uint32_t *status, hipStream_t s) {
     if (n_blocks <= 0) return hipSuccess;
-    hipLaunchKernelGGL(decode_blocks_kernel, dim3(n_blocks), dim3(kThreads), 0, s, blob, bytes, offs, first, seq,
-                       dim, out, status);
+    hipLaunchKernelGGL(dim % 8 == 0 ? decode_octets_kernel : decode_blocks_kernel, dim3(n_blocks), dim3(kThreads), 0,
+                       s, blob, bytes, offs, first, n_blocks, need, seq, dim, out, status);
     return hipGetLastError();
 }
 

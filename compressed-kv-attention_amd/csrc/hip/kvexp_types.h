@@ -13,6 +13,7 @@ enum : uint32_t {
     kStEscape = 1u << 3,    // more sentinels than n_escape
     kStIndex = 1u << 4,     // block index disagrees with the headers
     kStLookback = 1u << 5,  // the fused encoder's wait for an earlier block's size ran out
+    kStShort = 1u << 6,     // the block index covers fewer tokens than a checked decode asks for
 };
 
 

@@ -27,7 +27,7 @@ using kvexp_dev::WorkItem;
 
 namespace kvexp_launch {
 hipError_t decode(const uint8_t *blob, uint64_t bytes, const int64_t *offs, const int32_t *first, int n_blocks,
-                  int seq, int dim, uint16_t *out, uint32_t *status, hipStream_t s);
+                  int need, int seq, int dim, uint16_t *out, uint32_t *status, hipStream_t s);
 bool encode_fused_supported(int dim, int bt);
 hipError_t encode(const uint16_t *kv, int seq, int dim, int bt, int n_blocks, EncBlockMeta *meta, uint8_t *bases,
                   int64_t *offs, int32_t *first, uint8_t *out, uint32_t *status, hipStream_t s, bool rebase,
@@ -194,6 +194,7 @@ struct DevBuf {
 
 std::string status_message(uint32_t st) {
     using namespace kvexp_dev;
+    if (st & kStShort) return "xkv decode ran out of blocks";
     if (st & kStHeader) return "xkv block dimension or length mismatch";
     if (st & kStMode) return "unknown xkv block mode";
     if (st & kStTruncated) return "truncated coded xkv block";
@@ -841,14 +842,14 @@ int kvexp_hip_decode(kvexp_hip_ctx *ctx, const uint8_t *d_blob, size_t bytes, co
             fail(KVEXP_HIP_INVALID_ARGUMENT, "kvexp_hip_decode: null argument");
         DeviceGuard g(ctx->device);
         hipStream_t s = static_cast<hipStream_t>(stream);
-        if (check) {
+        if (check && n_blocks == 0) { // no block to launch for: the index's one entry is read here
             int32_t have = 0;
-            HIPX(hipMemcpyAsync(&have, d_first_token + n_blocks, sizeof have, hipMemcpyDeviceToHost, s));
+            HIPX(hipMemcpyAsync(&have, d_first_token, sizeof have, hipMemcpyDeviceToHost, s));
             HIPX(hipStreamSynchronize(s));
             if (have < seq) fail(KVEXP_HIP_FORMAT_ERROR, "xkv decode ran out of blocks");
         }
         scratch_acquire(ctx, s); // the status word is shared with the encoders
-        HIPX(kvexp_launch::decode(d_blob, bytes, d_offsets, d_first_token, n_blocks, seq, dim, d_out,
+        HIPX(kvexp_launch::decode(d_blob, bytes, d_offsets, d_first_token, n_blocks, check ? seq : 0, seq, dim, d_out,
                                   ctx->status.as<uint32_t>(), s));
         scratch_used(ctx, s);
         if (check) check_status_word(ctx->status.as<uint32_t>(), s);
