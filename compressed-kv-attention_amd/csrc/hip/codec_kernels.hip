@@ -329,6 +329,54 @@ __host__ __device__ constexpr size_t stats_lds_bytes(int dim) {
            (3 * kWaves + 2 * stats_cols(dim)) * sizeof(int);
 }
 
+// best_base (codec.cpp:18-35) of one channel column for the 2-, 3- and 4-bit
+// windows (3, 7 and 15 exponents) over the bases of words [j0, j1] (base 4 j +
+// i): the largest key coverage * 256 + 255 - base, so the most covered
+// exponents and then the smallest base. hw: the column's 64 words of byte
+// counters and a zero word after them. A block holds at most 255 tokens, so
+// the coverages of four bases fit the bytes of a word, and a window's sum is
+// built from sums of 2, 4 and 8 exponents shared by all windows:
+//   s2(b) = h(b) + h(b+1), s4(b) = s2(b) + s2(b+2),
+//   s3 = s2(b) + h(b+2), s7 = s4(b) + s2(b+4) + h(b+6),
+//   s15 = s4(b) + s4(b+4) + s4(b+8) + s2(b+12) + h(b+14),
+// about 22 instructions and one LDS read per four bases (sliding each window
+// by one exponent took two byte reads and five instructions per base and
+// window). Bases past 256 - width are no candidates of best_base; they need
+// no test, since the window at 256 - width covers all that theirs do at a
+// smaller base. Words 64 and up read as the zero word.
+__device__ __forceinline__ void window_keys(const uint32_t *hw, int j0, int j1, bool three, uint32_t (&key)[3]) {
+    typedef unsigned short pk16 __attribute__((ext_vector_type(2)));
+    pk16 best[3] = {{0, 0}, {0, 0}, {0, 0}};
+    auto word = [&](int j) { return hw[min(j, 64)]; };
+    auto al = [](uint32_t hi, uint32_t lo, uint32_t n) { return __builtin_amdgcn_alignbyte(hi, lo, n); };
+    // per word j: w, h2 = h(b + 2), s2, s4; s4(j) needs w(j .. j + 2)
+    uint32_t w1 = word(j0 + 1), w2 = word(j0 + 2), w3 = word(j0 + 3), w4 = word(j0 + 4);
+    uint32_t w0 = word(j0);
+    uint32_t s2a = w0 + al(w1, w0, 1), s2b = w1 + al(w2, w1, 1), s2c = w2 + al(w3, w2, 1), s2d = w3 + al(w4, w3, 1);
+    uint32_t h2a = al(w1, w0, 2), h2b = al(w2, w1, 2), h2c = al(w3, w2, 2), h2d = al(w4, w3, 2);
+    uint32_t s4a = s2a + al(s2b, s2a, 2), s4b = s2b + al(s2c, s2b, 2), s4c = s2c + al(s2d, s2c, 2);
+    uint32_t ce = uint32_t(255 - 4 * j0) | (uint32_t(253 - 4 * j0) << 16); // 255 - base of bases 4j and 4j + 2
+    auto take = [&](int i, uint32_t cov) {
+        const uint32_t e = __builtin_amdgcn_perm(cov, ce, 0x06020400u);
+        const uint32_t o = __builtin_amdgcn_perm(cov, ce - 0x00010001u, 0x07020500u);
+        best[i] = __builtin_elementwise_max(best[i], __builtin_bit_cast(pk16, e));
+        best[i] = __builtin_elementwise_max(best[i], __builtin_bit_cast(pk16, o));
+    };
+    for (int j = j0; j <= j1; ++j) {
+        take(0, s2a + h2a);
+        if (three) take(1, s4a + s2b + h2b);
+        take(2, s4a + s4b + s4c + s2d + h2d);
+        const uint32_t w5 = word(j + 5);
+        const uint32_t s2e = w4 + al(w5, w4, 1), h2e = al(w5, w4, 2);
+        s2a = s2b, s2b = s2c, s2c = s2d, h2a = h2b, h2b = h2c, h2c = h2d;
+        s4a = s4b, s4b = s4c, s4c = s2c + al(s2e, s2c, 2);
+        s2d = s2e, h2d = h2e, w4 = w5;
+        ce -= 0x00040004u;
+    }
+#pragma unroll
+    for (int i = 0; i < 3; ++i) key[i] = max(uint32_t(best[i].x), uint32_t(best[i].y));
+}
+
 // The block's mode from the escape counts of the 2-, 3- and 4-bit windows
 // (codec.cpp:94-103): raw, then the coded modes by width; replace when
 // smaller, or on a tie when the best is not raw and has more escapes (or
@@ -379,7 +427,7 @@ __device__ __forceinline__ void encode_stats_block(uint32_t *hist, int *esc_part
         const bool has = d < dim;
         if (slice == 0 && has) {
 #pragma unroll 16
-            for (int k = 0; k < 64; ++k) h[k] = 0u;
+            for (int k = 0; k < kHistStride; ++k) h[k] = 0u;
             lohi[own] = 255;
             lohi[nthr + own] = 0;
         }
@@ -410,24 +458,13 @@ __device__ __forceinline__ void encode_stats_block(uint32_t *hist, int *esc_part
         __syncthreads();
         if (slice == 0 && has) {
             const int e_lo = lohi[own], e_hi = lohi[nthr + own];
-            auto count = [&](int b) { return int((h[b >> 2] >> (8 * (b & 3))) & 0xFFu); };
-            for (int wi = 0; wi < nwin; ++wi) {
-                const int bi = wi == 0 ? 0 : (wi == 1 && nwin == 2 ? 2 : wi); // 2-, (3-,) 4-bit
-                const int width = (4 << bi) - 1; // codes 0..2^bits-2
-                const int lo = min(max(0, e_lo - width + 1), 256 - width);
-                const int hi = min(e_hi, 256 - width);
-                int cov = 0;
-                for (int b = lo; b < lo + width; ++b) cov += count(b);
-                int best = cov, best_base = lo;
-                for (int b = lo + 1; b <= hi; ++b) {
-                    cov += count(b + width - 1) - count(b - 1);
-                    if (cov > best) {
-                        best = cov;
-                        best_base = b;
-                    }
-                }
-                bases[size_t(bi) * size_t(dim) + size_t(d)] = uint8_t(best_base);
-                esc[bi] += n - best;
+            uint32_t key[3];
+            window_keys(h, max(0, e_lo - 14) >> 2, e_hi >> 2, nwin == 3, key);
+#pragma unroll
+            for (int bi = 0; bi < 3; ++bi) {
+                if (bi == 1 && nwin != 3) continue;
+                bases[size_t(bi) * size_t(dim) + size_t(d)] = uint8_t(255u - (key[bi] & 255u));
+                esc[bi] += n - int(key[bi] >> 8);
             }
         }
         __syncthreads(); // the columns are cleared again for the next channels
@@ -838,10 +875,10 @@ encode_fused_kernel(const AppendJobDev *__restrict__ jobs, AppendJobDev one, int
     __shared__ uint32_t s_ticket, s_next;
     __shared__ int s_lo[kWaves], s_hi[kWaves], s_esc[kWaves][3];
     __shared__ __align__(16) uint8_t s_base[3][kMaxDim]; // window bases of the 2-, 3- and 4-bit codes
-    __shared__ uint16_t s_key[3 * kMaxDim];               // best (coverage, base) of the upper half of each range
+    __shared__ uint16_t s_key[3][kThreads];               // best (coverage, base) of each window, segment and channel
     __shared__ uint32_t s_scan[kWaves * EscRanks<NL>::NP];
     __shared__ long long s_excl;
-    const int tid = int(threadIdx.x), lane = lane_id(), w = tid >> 6;
+    const int tid = int(threadIdx.x);
     const int jx = int(blockIdx.y);
     uint32_t polls = 0; // look-back reads that found a nearer block unpublished
 #if defined(KVEXP_PHASE_TRACE)
@@ -989,77 +1026,33 @@ encode_fused_kernel(const AppendJobDev *__restrict__ jobs, AppendJobDev one, int
             if (bn < j.nb) load_tokens(bn, xn);
         }
 
-        // ---- best_base of each (window, channel) (codec.cpp:18-35): the most
-        // covered exponents, then the smallest base; bases outside
-        // [blk_lo - width + 1, blk_hi] cover nothing. Each range is split in two
-        // halves taken by different waves (tasks [0, pairs) the lower halves,
-        // [pairs, 2 pairs) the upper); a half's best is the key
-        // coverage * 256 + 255 - base, so the larger key is the better base.
+        // ---- best_base of each channel and window (window_keys) over the bases
+        // whose windows reach the block's exponents, in segments of words when
+        // there are threads for more than one per channel
         const int nwin = (modes & 8) ? 3 : 2;
-        const int pairs = nwin * dim;
-        int key_lo[3] = {0, 0, 0}; // this thread's lower-half results (tasks tid, tid + 256, tid + 512)
+        const int nseg = dim <= 64 ? 4 : (dim <= 128 ? 2 : 1);
+        if (tid < nseg * dim) {
+            const int seg = dim == 64 ? w : (tid >= dim) + (tid >= 2 * dim) + (tid >= 3 * dim);
+            const int d = tid - seg * dim;
+            const int jlo = max(0, blk_lo - 14) >> 2, jn = (blk_hi >> 2) - jlo + 1;
+            const int per = (jn + nseg - 1) / nseg; // (a power of two)
+            uint32_t key[3];
+            window_keys(fz_hist + d * kHistStride, jlo + seg * per, min(jlo + jn, jlo + (seg + 1) * per) - 1, nwin == 3,
+                        key);
 #pragma unroll
-        for (int r = 0; r < 6; ++r) {
-            const int t = tid + r * kThreads;
-            if (t >= 2 * pairs) break;
-            const int half = int(t >= pairs);
-            const int pt = t - half * pairs;
-            const int wi = int(pt >= dim) + int(pt >= 2 * dim);
-            const int d = pt - wi * dim;
-            const int bi = wi == 0 ? 0 : (nwin == 2 ? 2 : wi);
-            const int width = (4 << bi) - 1;
-            const int lo0 = min(max(0, blk_lo - width + 1), 256 - width);
-            const int hi0 = min(blk_hi, 256 - width);
-            const int mid = (lo0 + hi0 + 1) >> 1;
-            const int lo = half ? mid : lo0, hi = half ? hi0 : mid - 1;
-            int key = 0;
-            if (lo <= hi) {
-                const uint8_t *hb = reinterpret_cast<const uint8_t *>(fz_hist + d * kHistStride);
-                // the first window's coverage: the byte counters of bins [lo,
-                // lo + width) summed a word (four bins) at a time with
-                // v_sad_u8, the bins outside masked off (lo is the same in
-                // every lane of the wave, so is the loop)
-                int cov = 0;
-                {
-                    const uint32_t *hw = fz_hist + d * kHistStride;
-                    const int w0 = lo >> 2, w1 = (lo + width - 1) >> 2;
-                    const uint32_t m0 = 0xFFFFFFFFu << (8 * (lo & 3));
-                    const uint32_t m1 = 0xFFFFFFFFu >> (8 * (3 - ((lo + width - 1) & 3)));
-                    uint32_t acc = 0;
-                    for (int wi = w0; wi <= w1; ++wi) {
-                        uint32_t m = 0xFFFFFFFFu;
-                        if (wi == w0) m &= m0;
-                        if (wi == w1) m &= m1;
-                        acc = __builtin_amdgcn_sad_u8(hw[wi] & m, 0u, acc);
-                    }
-                    cov = int(acc);
-                }
-                int best = cov, best_b = lo;
-#pragma unroll 4
-                for (int base = lo + 1; base <= hi; ++base) {
-                    cov += int(hb[base + width - 1]) - int(hb[base - 1]);
-                    if (cov > best) {
-                        best = cov;
-                        best_b = base;
-                    }
-                }
-                key = best * 256 + 255 - best_b;
-            }
-            if (half) s_key[pt] = uint16_t(key);
-            else if (r < 3) key_lo[r] = key;
+            for (int bi = 0; bi < 3; ++bi) s_key[bi][tid] = uint16_t(key[bi]);
         }
         __syncthreads();
         int esc[3] = {0, 0, 0};
+        if (tid < dim) {
 #pragma unroll
-        for (int r = 0; r < 3; ++r) {
-            const int pt = tid + r * kThreads;
-            if (pt >= pairs) break;
-            const int wi = int(pt >= dim) + int(pt >= 2 * dim);
-            const int d = pt - wi * dim;
-            const int bi = wi == 0 ? 0 : (nwin == 2 ? 2 : wi);
-            const int key = max(key_lo[r], int(s_key[pt]));
-            s_base[bi][d] = uint8_t(255 - (key & 255));
-            esc[bi] += n - (key >> 8);
+            for (int bi = 0; bi < 3; ++bi) {
+                if (bi == 1 && nwin != 3) continue;
+                uint32_t key = s_key[bi][tid];
+                for (int i = 1; i < nseg; ++i) key = max(key, uint32_t(s_key[bi][tid + i * dim]));
+                s_base[bi][tid] = uint8_t(255u - (key & 255u));
+                esc[bi] = n - int(key >> 8);
+            }
         }
 #pragma unroll
         for (int bi = 0; bi < 3; ++bi) esc[bi] = wave_sum_i32(esc[bi]);
