@@ -332,8 +332,8 @@ __host__ __device__ constexpr size_t stats_lds_bytes(int dim) {
 // best_base (codec.cpp:18-35) of one channel column for the 2-, 3- and 4-bit
 // windows (3, 7 and 15 exponents) over the bases of words [j0, j1] (base 4 j +
 // i): the largest key coverage * 256 + 255 - base, so the most covered
-// exponents and then the smallest base. hw: the column's 64 words of byte
-// counters and a zero word after them. A block holds at most 255 tokens, so
+// exponents and then the smallest base. word(j): word j of the column's byte
+// counters, 0 from word 64 on. A block holds at most 255 tokens, so
 // the coverages of four bases fit the bytes of a word, and a window's sum is
 // built from sums of 2, 4 and 8 exponents shared by all windows:
 //   s2(b) = h(b) + h(b+1), s4(b) = s2(b) + s2(b+2),
@@ -343,11 +343,11 @@ __host__ __device__ constexpr size_t stats_lds_bytes(int dim) {
 // by one exponent took two byte reads and five instructions per base and
 // window). Bases past 256 - width are no candidates of best_base; they need
 // no test, since the window at 256 - width covers all that theirs do at a
-// smaller base. Words 64 and up read as the zero word.
-__device__ __forceinline__ void window_keys(const uint32_t *hw, int j0, int j1, bool three, uint32_t (&key)[3]) {
+// smaller base.
+template <class Word>
+__device__ __forceinline__ void window_keys(Word &&word, int j0, int j1, bool three, uint32_t (&key)[3]) {
     typedef unsigned short pk16 __attribute__((ext_vector_type(2)));
     pk16 best[3] = {{0, 0}, {0, 0}, {0, 0}};
-    auto word = [&](int j) { return hw[min(j, 64)]; };
     auto al = [](uint32_t hi, uint32_t lo, uint32_t n) { return __builtin_amdgcn_alignbyte(hi, lo, n); };
     // per word j: w, h2 = h(b + 2), s2, s4; s4(j) needs w(j .. j + 2)
     uint32_t w1 = word(j0 + 1), w2 = word(j0 + 2), w3 = word(j0 + 3), w4 = word(j0 + 4);
@@ -459,7 +459,8 @@ __device__ __forceinline__ void encode_stats_block(uint32_t *hist, int *esc_part
         if (slice == 0 && has) {
             const int e_lo = lohi[own], e_hi = lohi[nthr + own];
             uint32_t key[3];
-            window_keys(h, max(0, e_lo - 14) >> 2, e_hi >> 2, nwin == 3, key);
+            // (the word after the column's 64 stays zero)
+            window_keys([&](int j) { return h[min(j, 64)]; }, max(0, e_lo - 14) >> 2, e_hi >> 2, nwin == 3, key);
 #pragma unroll
             for (int bi = 0; bi < 3; ++bi) {
                 if (bi == 1 && nwin != 3) continue;
@@ -695,8 +696,23 @@ __global__ __launch_bounds__(kThreads) void append_write_kernel(const AppendJobD
                        bases + size_t(g) * 3 * size_t(dim), j.out + j.offs[b], status);
 }
 
-// The raw rows of each job's new trailing partial block that are not in
-// its tail buffer yet, copied there (after the write kernel has read it).
+// The raw rows of a job's new trailing partial block that are not in its tail
+// buffer yet, copied there: 16 bytes per thread and step where source, tail
+// and row size allow it (32 tails of 86 rows of head_dim 256: 21.8 us with
+// 2-byte copies).
+__device__ __forceinline__ void copy_rows(const AppendJobDev &j, int dim) {
+    const int total = j.copy_rows * dim;
+    const uint16_t *from = j.src + size_t(j.copy_from) * size_t(dim);
+    uint16_t *to = j.tail + size_t(j.copy_to) * size_t(dim);
+    if (dim % 8 == 0 && ((reinterpret_cast<uintptr_t>(from) | reinterpret_cast<uintptr_t>(to)) & 15u) == 0) {
+        for (int i = int(threadIdx.x); i < total / 8; i += int(blockDim.x))
+            reinterpret_cast<uint4 *>(to)[i] = reinterpret_cast<const uint4 *>(from)[i];
+        return;
+    }
+    for (int i = int(threadIdx.x); i < total; i += int(blockDim.x)) to[i] = from[i];
+}
+
+// Each job's rows of copy_rows (after the write kernel has read it).
 // With `terminal` set (after the fused encoder, which writes the index of
 // the jobs with blocks), also the index entry of an empty container.
 __global__ __launch_bounds__(kThreads) void append_tail_kernel(const AppendJobDev *__restrict__ jobs, int dim,
@@ -706,10 +722,7 @@ __global__ __launch_bounds__(kThreads) void append_tail_kernel(const AppendJobDe
         j.offs[0] = j.rebase ? j.offs[0] : 0;
         j.first[0] = j.tok0;
     }
-    const int total = j.copy_rows * dim;
-    const uint16_t *from = j.src + size_t(j.copy_from) * size_t(dim);
-    uint16_t *to = j.tail + size_t(j.copy_to) * size_t(dim);
-    for (int i = int(threadIdx.x); i < total; i += kThreads) to[i] = from[i];
+    copy_rows(j, dim);
 }
 
 // ------------------------------------------------ encode: one fused pass --
@@ -725,19 +738,24 @@ __global__ __launch_bounds__(kThreads) void append_tail_kernel(const AppendJobDe
 // neither round trip stands on a block's path but the first one's. It stops
 // at its first ticket past the job's blocks (the one that draws the job's
 // last ticket, number n_blocks + P - 1, resets the counter). A block: it
-// holds the block's tokens in
-// registers (chunks of 8 elements of one row, 16 bytes, NL chunks per
-// thread), counts each channel's exponents into LDS byte counters, slides the
-// code windows (one (window, channel) pair per thread, so that every wave
-// works), chooses the mode, and finds its place in the container by a
+// holds the block's tokens in registers (chunks of 8 elements of one row, 16
+// bytes, NL chunks per thread), counts each channel's exponents into LDS byte
+// counters, sums the code windows over them (a channel per thread, or a half
+// of its range), chooses the mode, and finds its place in the container by a
 // decoupled look-back over the sizes of its job's earlier blocks: each block
 // publishes its own size as soon as its mode is known, and the job-relative
 // end of its bytes once its place is known; wave 0 reads up to 64 earlier
 // entries at a time and sums back to the nearest end, after the block's codes
 // and escape ranks are computed (so that the earlier blocks have had that
 // long to publish). Then the block is written from the registers.
-// head_dim % 8 == 0, at most kFusedMaxElems elements per block, sources
-// 16-byte aligned (the host checks; otherwise it uses the three launches).
+// Bound: vector instructions (about 1,000 per wave and block at head_dim 64;
+// the pipe is busy about 80 % of the launch) and the block's chain of
+// barriers, which eight workgroups per CU overlap. Per prefill call: 96
+// containers x 32,768 tokens of head_dim 64, 264 -> 224 us (2.7 -> 3.2 TB/s);
+// 32 x 8,150 tokens of head_dim 256 (blocks of 32,768 elements, which took the
+// three launches before), 211 -> 104 us.
+// head_dim % 8 == 0 and sources 16-byte aligned (the host checks; otherwise it
+// uses the three launches).
 //
 // Look-back state: one ticket counter per job (reset to 0 by the workgroup
 // that takes the job's last ticket) and, in an array of its own, one entry
@@ -776,10 +794,10 @@ typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 typedef const __attribute__((address_space(1))) u32x4_t g_cu32x4; // 16-byte global loads
 
-// Exclusive prefix over the workgroup, in chunk order (chunk k * kThreads +
-// thread), of the sentinel counts packed two to a 32-bit word (16 bits
-// each: at most 8 per chunk, 2048 per chunk row of the workgroup, so no
-// field carries into the next). tmp: [kWaves][NP] words in LDS. Leaves in
+// Exclusive prefix over the workgroup of TH threads, in chunk order (chunk k *
+// TH + thread), of the sentinel counts packed two to a 32-bit word (16 bits
+// each: at most 8 per chunk, 8,192 per chunk row of the workgroup, so no
+// field carries into the next). tmp: [TH / 64][NP] words in LDS. Leaves in
 // excl[q] the thread's exclusive prefix within each chunk row and in
 // total[q] the rows' totals (field k % 2 of word k / 2 for chunk row k);
 // EscRanks::rank gives a chunk's first rank.
@@ -805,7 +823,7 @@ struct EscRanks {
     }
 };
 
-template <int NL>
+template <int NL, int TH>
 __device__ __forceinline__ EscRanks<NL> fused_escape_ranks(const uint32_t (&v)[EscRanks<NL>::NP], uint32_t *tmp) {
     constexpr int NP = EscRanks<NL>::NP;
     const int lane = lane_id(), w = int(threadIdx.x) >> 6;
@@ -821,7 +839,7 @@ __device__ __forceinline__ EscRanks<NL> fused_escape_ranks(const uint32_t (&v)[E
     for (int q = 0; q < NP; ++q) {
         uint32_t before = 0, total = 0;
 #pragma unroll
-        for (int x = 0; x < kWaves; ++x) {
+        for (int x = 0; x < TH / kWave; ++x) {
             const uint32_t t = tmp[x * NP + q];
             before += x < w ? t : 0;
             total += t;
@@ -832,6 +850,9 @@ __device__ __forceinline__ EscRanks<NL> fused_escape_ranks(const uint32_t (&v)[E
     return r;
 }
 
+// Workgroups have TH threads: 256 for blocks of up to 16,384 elements, 512 and
+// 1,024 above (a CU's LDS then holds two blocks, or one, and the threads keep
+// four waves per SIMD).
 // Waves per SIMD the one-pass encoder is compiled for (its registers fit
 // 512 / waves without spilling): 8 with up to four chunk rows per thread.
 template <int NL>
@@ -840,8 +861,8 @@ constexpr int kFusedWaves = NL <= 4 ? 8 : 4;
 // thread, one block's tokens fit in registers beside the next block's (NL
 // 16-byte loads each) at eight waves; at four rows the next block's tokens
 // are loaded only once this block's are dead (kFusedNextEarly), which keeps
-// the kernel at 64 registers and eight waves (eight workgroups per CU: the
-// c2 prefill 2.6 % faster than six with both sets in registers). At NL 8 the
+// the kernel at 64 registers and eight waves (eight workgroups per CU: c2's
+// prefill call 224 us, 229 with seven, 232 with six). At NL 8 the
 // budget stays at four (128 registers): three would let a head_dim-128
 // tensor's 1,024 blocks fill only 768 workgroups at once.
 template <int NL>
@@ -851,32 +872,79 @@ constexpr int kFusedWavesMin = NL <= 4 ? 8 : 4;
 template <int NL>
 constexpr bool kFusedNextEarly = NL <= 2;
 
+// The histograms: channel d's 64 words of byte counters (four exponents each)
+// lie at word 64 d, word j of them at place j ^ (d % 64). So the 64 lanes of
+// an add or of a window read, on 64 channels at about the same exponents, use
+// different banks, and the place of an element's counter is a few XORs of
+// bit fields that do not overlap.
+constexpr int kFusedCol = 64; // words per channel
+
 // Dynamic LDS of the one-pass encoder: the histogram columns, or the
 // largest block (raw: header + 2 bytes per element) staged for its copy,
-// whichever is larger. At most 66,560 bytes (head_dim 256, 64-token blocks).
+// whichever is larger. At most 130,584 bytes (head_dim 256, 255-token blocks).
 __host__ __device__ constexpr size_t fused_lds_bytes(int dim, int bt) {
-    const size_t hist = size_t(dim) * kHistStride * sizeof(uint32_t);
+    const size_t hist = size_t(dim) * kFusedCol * sizeof(uint32_t);
     const size_t raw = (8u + 2u * size_t(bt) * size_t(dim) + 15u) & ~size_t(15);
     return hist > raw ? hist : raw;
 }
 
+typedef unsigned short u16x2_t __attribute__((ext_vector_type(2)));
+
+// The exponent fields of a dword's two BF16, 16 bits apart.
+__device__ __forceinline__ uint32_t exponent_pair(uint32_t x) { return (x >> 7) & 0x00FF00FFu; }
+
+// The codes (`mode` bits each) of a chunk's 8 elements v against the bases of
+// their channels (16 bits each): exponent - base where that is below 2^mode -
+// 1, else (wrapped below 0 included) the sentinel, two elements at a time.
+__device__ __forceinline__ uint32_t chunk_codes(const u32x4_t &v, const uint4 &bases, int mode) {
+    const uint32_t width = (1u << mode) - 1u;
+    const u16x2_t top = {uint16_t(width), uint16_t(width)};
+    const uint32_t b[4] = {bases.x, bases.y, bases.z, bases.w};
+    uint32_t c[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const u16x2_t d = __builtin_bit_cast(u16x2_t, exponent_pair(v[i])) - __builtin_bit_cast(u16x2_t, b[i]);
+        c[i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_min(d, top));
+    }
+    if (mode == 4) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) c[i] |= c[i] >> 12; // the pair's byte
+        return __builtin_amdgcn_perm(c[1], c[0], 0x0c0c0400u) | __builtin_amdgcn_perm(c[3], c[2], 0x04000c0cu);
+    }
+    uint32_t cw = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) cw |= ((c[i] | (c[i] >> (16 - mode))) & ((1u << (2 * mode)) - 1u)) << (2 * mode * i);
+    return cw;
+}
+
+// The sentinels of a chunk's code word: bit mode * h for element h.
+__device__ __forceinline__ uint32_t sentinel_bits(uint32_t cw, int mode) {
+    if (mode == 4) {
+        const uint32_t a = cw & (cw >> 1);
+        return a & (a >> 2) & 0x11111111u;
+    }
+    if (mode == 2) return cw & (cw >> 1) & 0x5555u;
+    return cw & (cw >> 1) & (cw >> 2) & 0x249249u;
+}
+
 // JOBS: the jobs are in device memory (appends); else the one job is a
 // kernel argument (an encode), read from the argument segment.
-template <int NL, bool JOBS>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kFusedWavesMin<NL>, kFusedWaves<NL>))) void
+template <int NL, int TH, bool JOBS>
+__global__ __launch_bounds__(TH) __attribute__((amdgpu_waves_per_eu(kFusedWavesMin<NL>, kFusedWaves<NL>))) void
 encode_fused_kernel(const AppendJobDev *__restrict__ jobs, AppendJobDev one, int dim, int bt, int modes,
                     uint64_t *__restrict__ state, uint32_t *__restrict__ tickets, uint32_t epoch,
                     uint32_t *__restrict__ status) {
-    // dynamic LDS: the exponent byte counters [dim][kHistStride], then the
+    constexpr int NW = TH / kWave;
+    // dynamic LDS: the exponent byte counters [dim][kFusedCol], then the
     // block's bytes staged for the copy to the container (fused_lds_bytes)
     extern __shared__ __align__(16) uint32_t fz_lds[];
     uint32_t *fz_hist = fz_lds;
     uint8_t *stage = reinterpret_cast<uint8_t *>(fz_lds);
     __shared__ uint32_t s_ticket, s_next;
-    __shared__ int s_lo[kWaves], s_hi[kWaves], s_esc[kWaves][3];
-    __shared__ __align__(16) uint8_t s_base[3][kMaxDim]; // window bases of the 2-, 3- and 4-bit codes
-    __shared__ uint16_t s_key[3][kThreads];               // best (coverage, base) of each window, segment and channel
-    __shared__ uint32_t s_scan[kWaves * EscRanks<NL>::NP];
+    __shared__ int s_lo[NW], s_hi[NW], s_esc[NW][3];
+    __shared__ __align__(16) uint16_t s_base[3][kMaxDim]; // window bases of the 2-, 3- and 4-bit codes
+    __shared__ uint16_t s_key[3][TH];                     // best (coverage, base) of each window, segment and channel
+    __shared__ uint32_t s_scan[NW * EscRanks<NL>::NP];
     __shared__ long long s_excl;
     const int tid = int(threadIdx.x);
     const int jx = int(blockIdx.y);
@@ -900,9 +968,12 @@ encode_fused_kernel(const AppendJobDev *__restrict__ jobs, AppendJobDev one, int
         s_ticket = t;
     }
     // first channel of chunk c (8 * (c mod dim / 8); the float quotient is
-    // exact to far below its distance from an integer, c < 4096)
+    // exact to far below its distance from an integer, c < 8192)
     const int cpr = dim / 8;
     const float inv_cpr = __builtin_amdgcn_rcpf(float(cpr));
+    // a thread's chunks all lie in one chunk column, 8 (or a multiple) rows
+    // apart (head_dim 32, 64, 128, 256)
+    const bool same_rows = TH % cpr == 0 && (TH / cpr) % 8 == 0;
     auto chunk_d0 = [&](int c) {
         const int row = int((float(c) + 0.5f) * inv_cpr);
         return 8 * (c - row * cpr);
@@ -913,9 +984,15 @@ encode_fused_kernel(const AppendJobDev *__restrict__ jobs, AppendJobDev one, int
     auto load_tokens = [&](int bb, u32x4_t (&dst)[NL]) {
         const EncRows sr = job_rows(j, bb, bt, dim);
         const int nch = min(bt, j.seq - bb * bt) * dim / 8, spl = sr.split / 8;
+        if (nch == NL * TH && spl == 0) { // the full block of one source: no chunk to pick or clamp
+            const uint8_t *p = reinterpret_cast<const uint8_t *>(sr.b);
+#pragma unroll
+            for (int k = 0; k < NL; ++k) dst[k] = *(g_cu32x4 *)(p + 16 * TH * k + uint32_t(16 * tid));
+            return;
+        }
 #pragma unroll
         for (int k = 0; k < NL; ++k) {
-            const int c = k * kThreads + tid < nch ? k * kThreads + tid : 0;
+            const int c = k * TH + tid < nch ? k * TH + tid : 0;
             const uint16_t *p = c < spl ? sr.a + 8 * size_t(c) : sr.b + 8 * size_t(c - spl);
             dst[k] = *(g_cu32x4 *)(p);
         }
@@ -943,9 +1020,8 @@ encode_fused_kernel(const AppendJobDev *__restrict__ jobs, AppendJobDev one, int
         // the next ticket, consumed after the histograms
         uint32_t tn = uint32_t(j.nb);
         if (tid == 0 && !one_shot) tn = atomicAdd(tickets + jx, 1u);
-        // (dim * kHistStride is a multiple of 8: 16-byte stores)
 #pragma unroll 1
-        for (int i = 4 * tid; i < dim * kHistStride; i += 4 * kThreads)
+        for (int i = 4 * tid; i < dim * kFusedCol; i += 4 * TH)
             *reinterpret_cast<uint4 *>(fz_hist + i) = make_uint4(0u, 0u, 0u, 0u);
         __syncthreads();
         polls = 0;
@@ -959,49 +1035,71 @@ encode_fused_kernel(const AppendJobDev *__restrict__ jobs, AppendJobDev one, int
         const int chunks = n * dim / 8;
 
         // ---- channel histograms of the block's tokens (in registers)
-        // exponent fields (bits 14..7 of each BF16) of the thread's elements,
-        // smallest and largest, both halves at once (v_pk_min_u16 /
-        // v_pk_max_u16); 0xFFFF: no element
-        typedef unsigned short u16x2_t __attribute__((ext_vector_type(2)));
+        // exponents of the thread's elements, smallest and largest, two at a time
+        // (v_pk_min_u16 / v_pk_max_u16); 0xFFFF: no element
         u16x2_t lo2 = {0xFFFF, 0xFFFF}, hi2 = {0, 0};
 #if defined(KVEXP_PHASE_TRACE)
         asm volatile("" ::"v"(x[NL - 1][0]), "v"(x[0][0]));
 #endif
         KVEXP_ENC_MARK(3);
         // Lanes that share a chunk column (the rows of one chunk position) count
-        // their 8 elements in an order rotated by the row (step h takes element
-        // (h + row) % 8), so that the 64 lanes of an LDS add hit different
-        // channel columns rather than 8 lanes one counter.
+        // their 8 elements in an order XORed with the row (step h takes element
+        // h ^ (row % 8)), so that the 64 lanes of an LDS add hit different
+        // channel columns rather than 8 lanes one counter. Element h ^ r of the
+        // chunk at column q is channel 8 q + (h ^ r); the place of its counter
+        // is bytes (2048 q + 32 (q % 8)) ^ 260 (h ^ r) ^ 4 (e / 4), and 260 (h ^ r)
+        // = 260 h ^ 260 r. (An order rotated by the row took an add, a mask and
+        // a product per element: the kernel was bound by its vector
+        // instructions, 40 per element, of which these were a third.)
+        uint32_t m4 = 0, m2 = 0, sw = 0, at[8] = {}; // of the chunk's row and column
+        const uint32_t wmask = [] {
+            uint32_t m = 0xFCu;
+            asm volatile("" : "+v"(m));
+            return m;
+        }();
 #pragma unroll
         for (int k = 0; k < NL; ++k) {
-            const int c = k * kThreads + tid;
+            const int c = k * TH + tid;
             if (c < chunks) {
-                const int row = int((float(c) + 0.5f) * inv_cpr);
-                const int rot = row & 7;
-                uint32_t *col = fz_hist + 8 * (c - row * cpr) * kHistStride;
-                // the chunk rotated right by 16 * rot bits: element h of v is element (h + rot) % 8
-                u32x4_t v = x[k];
-                if (rot & 4) v = u32x4_t{v[2], v[3], v[0], v[1]};
-                if (rot & 2) v = u32x4_t{v[1], v[2], v[3], v[0]};
-                if (rot & 1)
-                    v = u32x4_t{__builtin_amdgcn_alignbit(v[1], v[0], 16), __builtin_amdgcn_alignbit(v[2], v[1], 16),
-                                __builtin_amdgcn_alignbit(v[3], v[2], 16), __builtin_amdgcn_alignbit(v[0], v[3], 16)};
+                if (k == 0 || !same_rows) {
+                    const int row = int((float(c) + 0.5f) * inv_cpr);
+                    const uint32_t q = uint32_t(c - row * cpr), r = uint32_t(row) & 7u;
+                    m4 = 0u - (r >> 2), m2 = 0u - ((r >> 1) & 1u), sw = 16u * (r & 1u);
+                    const uint32_t at0 = (2048u * q | 32u * (q & 7u)) ^ (260u * r);
 #pragma unroll
-                for (int h = 0; h < 8; ++h) {
-                    const uint32_t e = (v[h >> 1] >> (16 * (h & 1) + 7)) & 0xFFu;
-                    atomicAdd(col + ((h + rot) & 7) * kHistStride + int(e >> 2), 1u << (8u * (e & 3u)));
+                    for (int h = 0; h < 8; ++h) at[h] = at0 ^ (260u * uint32_t(h));
                 }
+                uint32_t t[4];
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    const u16x2_t ef = __builtin_bit_cast(u16x2_t, x[k][i] & 0x7F807F80u);
-                    lo2 = __builtin_elementwise_min(lo2, ef);
-                    hi2 = __builtin_elementwise_max(hi2, ef);
+                    t[i] = exponent_pair(x[k][i]);
+                    lo2 = __builtin_elementwise_min(lo2, __builtin_bit_cast(u16x2_t, t[i]));
+                    hi2 = __builtin_elementwise_max(hi2, __builtin_bit_cast(u16x2_t, t[i]));
+                }
+                // element h of t becomes element h ^ r (swaps by all-lane masks)
+                auto pick = [](uint32_t m, uint32_t a, uint32_t b) -> uint32_t {
+                    return __builtin_amdgcn_bitop3_b32(a, b, m, 0xE4);
+                };
+                const uint32_t u0 = pick(m4, t[2], t[0]), u1 = pick(m4, t[3], t[1]), u2 = pick(m4, t[0], t[2]),
+                               u3 = pick(m4, t[1], t[3]);
+                const uint32_t v[4] = {pick(m2, u1, u0), pick(m2, u0, u1), pick(m2, u3, u2), pick(m2, u2, u3)};
+#pragma unroll
+                for (int h = 0; h < 8; ++h) {
+                    // the element's exponent in bits 7:0, its bits above exponent
+                    // bit 4 of no effect on the mask and the shift below
+                    const uint32_t p = __builtin_amdgcn_alignbit(v[h >> 1], v[h >> 1], sw);
+                    const uint32_t e = (h & 1) ? p >> 16 : p;
+                    // (e & 0xFC) ^ place: S0 & S1 ^ S2
+                    const uint32_t byte = __builtin_amdgcn_bitop3_b32(e, wmask, at[h], 0x6A);
+                    const uint32_t one = 1u << (((h & 1) ? p >> 13 : p << 3) & 31u);
+                    atomicAdd(reinterpret_cast<uint32_t *>(reinterpret_cast<uint8_t *>(fz_hist) + byte), one);
                 }
             }
+            __builtin_amdgcn_sched_barrier(0); // chunk by chunk (interleaved, they spill)
         }
         const uint32_t pk_lo = min(uint32_t(lo2.x), uint32_t(lo2.y)), pk_hi = max(uint32_t(hi2.x), uint32_t(hi2.y));
-        const int e_lo = wave_min_i32(pk_lo == 0xFFFFu ? 255 : int(pk_lo >> 7));
-        const int e_hi = wave_max_i32(int(pk_hi >> 7));
+        const int e_lo = wave_min_i32(int(min(pk_lo, 255u)));
+        const int e_hi = wave_max_i32(int(pk_hi));
         if (lane == 0) {
             s_lo[w] = e_lo;
             s_hi[w] = e_hi;
@@ -1014,7 +1112,7 @@ encode_fused_kernel(const AppendJobDev *__restrict__ jobs, AppendJobDev one, int
         KVEXP_ENC_MARK(4);
         int blk_lo = 255, blk_hi = 0;
 #pragma unroll
-        for (int i = 0; i < kWaves; ++i) {
+        for (int i = 0; i < NW; ++i) {
             blk_lo = min(blk_lo, s_lo[i]);
             blk_hi = max(blk_hi, s_hi[i]);
         }
@@ -1027,18 +1125,21 @@ encode_fused_kernel(const AppendJobDev *__restrict__ jobs, AppendJobDev one, int
         }
 
         // ---- best_base of each channel and window (window_keys) over the bases
-        // whose windows reach the block's exponents, in segments of words when
-        // there are threads for more than one per channel
+        // whose windows reach the block's exponents, in two segments of words
+        // where there are threads for them (four would repeat the sums at
+        // their starts more than they gain: 232.5 against 233.4 us per c2
+        // prefill call, and the kernel then spills at eight waves per SIMD)
         const int nwin = (modes & 8) ? 3 : 2;
-        const int nseg = dim <= 64 ? 4 : (dim <= 128 ? 2 : 1);
+        const int lseg = dim <= TH / 2 ? 1 : 0, nseg = 1 << lseg;
         if (tid < nseg * dim) {
-            const int seg = dim == 64 ? w : (tid >= dim) + (tid >= 2 * dim) + (tid >= 3 * dim);
+            const int seg = int(tid >= dim);
             const int d = tid - seg * dim;
             const int jlo = max(0, blk_lo - 14) >> 2, jn = (blk_hi >> 2) - jlo + 1;
-            const int per = (jn + nseg - 1) / nseg; // (a power of two)
+            const int per = (jn + nseg - 1) >> lseg;
             uint32_t key[3];
-            window_keys(fz_hist + d * kHistStride, jlo + seg * per, min(jlo + jn, jlo + (seg + 1) * per) - 1, nwin == 3,
-                        key);
+            const uint32_t *hw = fz_hist + d * kFusedCol;
+            window_keys([&](int jj) { return jj < kFusedCol ? hw[jj ^ (d & 63)] : 0u; }, jlo + seg * per,
+                        min(jlo + jn, jlo + (seg + 1) * per) - 1, nwin == 3, key);
 #pragma unroll
             for (int bi = 0; bi < 3; ++bi) s_key[bi][tid] = uint16_t(key[bi]);
         }
@@ -1050,7 +1151,7 @@ encode_fused_kernel(const AppendJobDev *__restrict__ jobs, AppendJobDev one, int
                 if (bi == 1 && nwin != 3) continue;
                 uint32_t key = s_key[bi][tid];
                 for (int i = 1; i < nseg; ++i) key = max(key, uint32_t(s_key[bi][tid + i * dim]));
-                s_base[bi][tid] = uint8_t(255u - (key & 255u));
+                s_base[bi][tid] = uint16_t(255u - (key & 255u));
                 esc[bi] = n - int(key >> 8);
             }
         }
@@ -1063,10 +1164,12 @@ encode_fused_kernel(const AppendJobDev *__restrict__ jobs, AppendJobDev one, int
         __syncthreads();
         int cand[3] = {0, 0, 0};
 #pragma unroll
-        for (int i = 0; i < kWaves; ++i) {
+        for (int i = 0; i < NW; ++i) {
 #pragma unroll
             for (int bi = 0; bi < 3; ++bi) cand[bi] += s_esc[i][bi];
         }
+#pragma unroll
+        for (int bi = 0; bi < 3; ++bi) cand[bi] = __builtin_amdgcn_readfirstlane(cand[bi]); // (uniform: scalar code)
         const EncBlockMeta m = choose_mode(cand, n, dim, modes, nwin);
         KVEXP_ENC_MARK(5);
 
@@ -1077,30 +1180,23 @@ encode_fused_kernel(const AppendJobDev *__restrict__ jobs, AppendJobDev one, int
 
         // ---- codes and sentinel counts
         const int mode = m.mode;
-        const uint32_t width = (1u << mode) - 1u;
         uint32_t cw[NL];
         uint32_t cnt_pk[EscRanks<NL>::NP] = {}; // sentinels per chunk, 16 bits each
+        uint4 bb = make_uint4(0u, 0u, 0u, 0u);  // the bases of the chunk's channels
 #pragma unroll
         for (int k = 0; k < NL; ++k) {
             cw[k] = 0u;
-            if (mode != 0 && k * kThreads + tid < chunks) {
-                int cnt = 0;
-                const uint2 bb = *reinterpret_cast<const uint2 *>(&s_base[mode - 2][chunk_d0(k * kThreads + tid)]);
-#pragma unroll
-                for (int h = 0; h < 8; ++h) {
-                    const uint32_t e = (x[k][h >> 1] >> (16 * (h & 1) + 7)) & 0xFFu;
-                    const uint32_t base = ((h < 4 ? bb.x : bb.y) >> (8 * (h & 3))) & 0xFFu;
-                    const uint32_t delta = e - base; // wraps when e < base
-                    const bool hit = delta < width;
-                    cw[k] |= (hit ? delta : width) << (mode * h);
-                    cnt += hit ? 0 : 1;
-                }
-                cnt_pk[k / 2] |= uint32_t(cnt) << (16 * (k % 2));
+            if (mode != 0 && k * TH + tid < chunks) {
+                if (k == 0 || !same_rows)
+                    bb = *reinterpret_cast<const uint4 *>(&s_base[mode - 2][chunk_d0(k * TH + tid)]);
+                cw[k] = chunk_codes(x[k], bb, mode);
+                cnt_pk[k / 2] |= uint32_t(__builtin_popcount(sentinel_bits(cw[k], mode))) << (16 * (k % 2));
             }
+            __builtin_amdgcn_sched_barrier(0);
         }
         // the escape ranks; the barrier in it also ends every read of the
         // histograms, whose LDS now takes the staged block
-        const EscRanks<NL> er = fused_escape_ranks<NL>(cnt_pk, s_scan);
+        const EscRanks<NL> er = fused_escape_ranks<NL, TH>(cnt_pk, s_scan);
         KVEXP_ENC_MARK(6);
 
         // ---- the block's bytes, staged in LDS in their final order
@@ -1114,31 +1210,28 @@ encode_fused_kernel(const AppendJobDev *__restrict__ jobs, AppendJobDev one, int
         if (mode == 0) {
 #pragma unroll
             for (int k = 0; k < NL; ++k) {
-                const int c = k * kThreads + tid;
+                const int c = k * TH + tid;
                 typedef u32x4_t __attribute__((aligned(8))) u32x4_a8;
                 if (c < chunks) *reinterpret_cast<u32x4_a8 *>(body + 16 * c) = x[k]; // 8 + 16c: 8-byte aligned
             }
         } else {
-            if (2 * tid < dim) // dim <= 256 = kThreads: one pair of bases per thread
-                *reinterpret_cast<uint16_t *>(body + 2 * tid) =
-                    *reinterpret_cast<const uint16_t *>(&s_base[mode - 2][2 * tid]);
+            if (tid < dim) body[tid] = uint8_t(s_base[mode - 2][tid]);
             uint8_t *sm = body + dim;
             uint8_t *codes = sm + n * dim;
             uint8_t *escw = codes + exp_payload_bytes(n, dim, mode);
 #pragma unroll
             for (int k = 0; k < NL; ++k) {
-                const int c = k * kThreads + tid;
+                const int c = k * TH + tid;
                 if (c >= chunks) continue;
-                // sign and mantissa bytes of the 8 elements: (h >> 8 & 0x80) | (h & 0x7F)
-                uint32_t s4[4];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const uint32_t mm = x[k][i] & 0x807F807Fu;
-                    s4[i] = mm | (mm >> 8); // bytes 0 and 2 hold the two elements' sm bytes
-                }
+                // sign and mantissa bytes of the 8 elements: (h >> 8 & 0x80) | (h & 0x7F),
+                // the four elements of two dwords from their low and high bytes
+                auto sm4 = [](uint32_t hi, uint32_t lo) -> uint32_t {
+                    return __builtin_amdgcn_bitop3_b32(__builtin_amdgcn_perm(hi, lo, 0x07050301u),
+                                                       __builtin_amdgcn_perm(hi, lo, 0x06040200u), 0x80808080u, 0xE4);
+                };
                 u32x2_t smv;
-                smv.x = __builtin_amdgcn_perm(s4[1], s4[0], 0x06040200u);
-                smv.y = __builtin_amdgcn_perm(s4[3], s4[2], 0x06040200u);
+                smv.x = sm4(x[k][1], x[k][0]);
+                smv.y = sm4(x[k][3], x[k][2]);
                 *reinterpret_cast<u32x2_t *>(sm + 8 * c) = smv; // 8 + dim + 8c: 8-byte aligned
                 if (mode == 4) {
                     *reinterpret_cast<uint32_t *>(codes + 4 * c) = cw[k];
@@ -1150,19 +1243,22 @@ encode_fused_kernel(const AppendJobDev *__restrict__ jobs, AppendJobDev one, int
                     q[1] = uint8_t(cw[k] >> 8);
                     q[2] = uint8_t(cw[k] >> 16);
                 }
-                if (((cnt_pk[k / 2] >> (16 * (k % 2))) & 0xFFFFu) != 0) {
+                // its escapes, one per step of the wave's lane with the most
+                uint32_t left = sentinel_bits(cw[k], mode);
+                if (left != 0) {
                     int r = er.rank(k);
-#pragma unroll
-                    for (int h = 0; h < 8; ++h) {
-                        if (((cw[k] >> (mode * h)) & width) == width) {
-                            if (r < m.n_escape) { // escape words may sit at odd offsets (3-bit codes): bytes
-                                const uint32_t v = x[k][h >> 1] >> (16 * (h & 1));
-                                escw[2 * r] = uint8_t(v);
-                                escw[2 * r + 1] = uint8_t(v >> 8);
-                            }
-                            ++r;
+                    do {
+                        const int bit = __builtin_ctz(left);
+                        const int h = mode == 4 ? bit >> 2 : (mode == 2 ? bit >> 1 : (bit * 11) >> 5);
+                        left &= left - 1u;
+                        if (r < m.n_escape) { // escape words may sit at odd offsets (3-bit codes): bytes
+                            const uint32_t lo = h & 2 ? x[k][1] : x[k][0], hi = h & 2 ? x[k][3] : x[k][2];
+                            const uint32_t v = (h & 4 ? hi : lo) >> (16 * (h & 1));
+                            escw[2 * r] = uint8_t(v);
+                            escw[2 * r + 1] = uint8_t(v >> 8);
                         }
-                    }
+                        ++r;
+                    } while (left != 0);
                 }
             }
         }
@@ -1220,7 +1316,7 @@ encode_fused_kernel(const AppendJobDev *__restrict__ jobs, AppendJobDev one, int
         const int head = min(nbytes, int((16u - (uint32_t(reinterpret_cast<uintptr_t>(p)) & 15u)) & 15u));
         const int n16 = (nbytes - head) >> 4;
         const int tail0 = head + 16 * n16;
-        for (int i = tid; i < n16; i += kThreads) {
+        for (int i = tid; i < n16; i += TH) {
             typedef const u32x4_t __attribute__((aligned(1))) u32x4_a1;
             *(__attribute__((address_space(1))) u32x4_t *)(p + head + 16 * i) =
                 *reinterpret_cast<u32x4_a1 *>(stage + head + 16 * i);
@@ -1310,10 +1406,7 @@ __global__ __launch_bounds__(kThreads) void append_one_kernel(const AppendJobDev
     }
     encode_write_block(scan_tmp, rows, j.seq, dim, m, bases_s, j.out + base, status);
     __syncthreads();
-    const int total = j.copy_rows * dim;
-    const uint16_t *from = j.src + size_t(j.copy_from) * size_t(dim);
-    uint16_t *to = j.tail + size_t(j.copy_to) * size_t(dim);
-    for (int i = int(threadIdx.x); i < total; i += kThreads) to[i] = from[i];
+    copy_rows(j, dim);
 }
 
 // ------------------------------------------------------------ escape records --
@@ -1524,18 +1617,18 @@ hipError_t decode(const uint8_t *blob, uint64_t bytes, const int64_t *offs, cons
 }
 
 bool encode_fused_supported(int dim, int bt) {
-    return dim >= 8 && dim % 8 == 0 && dim <= kMaxDim && bt >= 1 && int64_t(bt) * dim <= kFusedMaxElems;
+    return dim >= 8 && dim % 8 == 0 && dim <= kMaxDim && bt >= 1 && int64_t(bt) * dim <= 65535;
 }
 
 namespace {
-template <int NL, bool JOBS>
+template <int NL, int TH, bool JOBS>
 hipError_t launch_fused_j(const AppendJobDev *jobs, int n_jobs, const AppendJobDev &one, int max_job_blocks, int dim,
                           int bt, int modes, const EncLookback &lb, uint32_t *status, hipStream_t s) {
-    // head_dim 256 needs 66,560 bytes of histogram columns, past the default
-    // 64 KiB of dynamic LDS (set once per instantiation)
+    // past the default 64 KiB of dynamic LDS: the largest block this
+    // instantiation stages (set once per instantiation)
     static const hipError_t configured =
-        hipFuncSetAttribute(reinterpret_cast<const void *>(encode_fused_kernel<NL, JOBS>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, int(fused_lds_bytes(kMaxDim, 64)));
+        hipFuncSetAttribute(reinterpret_cast<const void *>(encode_fused_kernel<NL, TH, JOBS>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, int(fused_lds_bytes(kMaxDim, NL * TH * 8 / kMaxDim)));
     if (configured != hipSuccess) return configured;
     const size_t lds = fused_lds_bytes(dim, bt);
     // P workgroups per job: as many as are resident together over all jobs
@@ -1545,21 +1638,21 @@ hipError_t launch_fused_j(const AppendJobDev *jobs, int n_jobs, const AppendJobD
     if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
     if (e == hipSuccess)
         e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &per_cu, reinterpret_cast<const void *>(encode_fused_kernel<NL, JOBS>), kThreads, lds);
+            &per_cu, reinterpret_cast<const void *>(encode_fused_kernel<NL, TH, JOBS>), TH, lds);
     if (e != hipSuccess) return e;
     const int64_t resident = std::max<int64_t>(1, int64_t(cus) * std::max(per_cu, 1));
     const int per_job = int(std::max<int64_t>(1, std::min<int64_t>(max_job_blocks, resident / std::max(n_jobs, 1))));
-    hipLaunchKernelGGL((encode_fused_kernel<NL, JOBS>), dim3(unsigned(per_job), unsigned(n_jobs)),
-                       dim3(kThreads), lds, s, jobs, one, dim, bt, modes, lb.words, lb.tickets, lb.epoch, status);
+    hipLaunchKernelGGL((encode_fused_kernel<NL, TH, JOBS>), dim3(unsigned(per_job), unsigned(n_jobs)),
+                       dim3(TH), lds, s, jobs, one, dim, bt, modes, lb.words, lb.tickets, lb.epoch, status);
     return hipGetLastError();
 }
 
-template <int NL>
+template <int NL, int TH>
 hipError_t launch_fused(const AppendJobDev *jobs, int n_jobs, const AppendJobDev &one, int max_job_blocks, int dim,
                         int bt, int modes, const EncLookback &lb, uint32_t *status, hipStream_t s) {
     return jobs != nullptr
-               ? launch_fused_j<NL, true>(jobs, n_jobs, one, max_job_blocks, dim, bt, modes, lb, status, s)
-               : launch_fused_j<NL, false>(jobs, n_jobs, one, max_job_blocks, dim, bt, modes, lb, status, s);
+               ? launch_fused_j<NL, TH, true>(jobs, n_jobs, one, max_job_blocks, dim, bt, modes, lb, status, s)
+               : launch_fused_j<NL, TH, false>(jobs, n_jobs, one, max_job_blocks, dim, bt, modes, lb, status, s);
 }
 
 // The fused encoder over the blocks of `jobs` (device; n_jobs of them, the
@@ -1572,12 +1665,17 @@ hipError_t encode_fused(const AppendJobDev *jobs, int n_jobs, const AppendJobDev
         hipLaunchKernelGGL(clear_lookback_kernel, dim3(unsigned((nclear + 255) / 256)), dim3(256), 0, s, lb.words,
                            lb.clear_words, lb.tickets, lb.clear_tickets);
     const int chunks = (bt * dim) / 8;
-    if (chunks <= kThreads) return launch_fused<1>(jobs, n_jobs, one, max_job_blocks, dim, bt, modes, lb, status, s);
+    if (chunks <= kThreads)
+        return launch_fused<1, 256>(jobs, n_jobs, one, max_job_blocks, dim, bt, modes, lb, status, s);
     if (chunks <= 2 * kThreads)
-        return launch_fused<2>(jobs, n_jobs, one, max_job_blocks, dim, bt, modes, lb, status, s);
+        return launch_fused<2, 256>(jobs, n_jobs, one, max_job_blocks, dim, bt, modes, lb, status, s);
     if (chunks <= 4 * kThreads)
-        return launch_fused<4>(jobs, n_jobs, one, max_job_blocks, dim, bt, modes, lb, status, s);
-    return launch_fused<8>(jobs, n_jobs, one, max_job_blocks, dim, bt, modes, lb, status, s);
+        return launch_fused<4, 256>(jobs, n_jobs, one, max_job_blocks, dim, bt, modes, lb, status, s);
+    if (chunks <= 8 * kThreads)
+        return launch_fused<8, 256>(jobs, n_jobs, one, max_job_blocks, dim, bt, modes, lb, status, s);
+    if (chunks <= 16 * kThreads)
+        return launch_fused<8, 512>(jobs, n_jobs, one, max_job_blocks, dim, bt, modes, lb, status, s);
+    return launch_fused<8, 1024>(jobs, n_jobs, one, max_job_blocks, dim, bt, modes, lb, status, s);
 }
 } // namespace
 

@@ -118,8 +118,10 @@ struct EncLookback {
     size_t clear_tickets;
 };
 
-// The fused encoder holds a block in registers: at most this many elements.
-constexpr int kFusedMaxElems = 16384;
+// Blocks of up to this many elements count as the one-pass encoder's in the
+// no-allocation entry's scratch rule (a larger block's call is held to the
+// three-launch encoder's scratch, whichever encodes it).
+constexpr int kNoAllocFusedElems = 16384;
 
 // Job of a batched append, as the kernels read it (built by the host API).
 struct AppendJobDev {

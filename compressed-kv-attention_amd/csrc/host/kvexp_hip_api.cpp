@@ -657,10 +657,12 @@ int kvexp_hip_encode_noalloc(kvexp_hip_ctx *ctx, const uint16_t *d_kv, int seq, 
         const int nb = kvexp_hip_block_count(seq, bt);
         auto up = [](size_t n) { return (n + 255u) & ~size_t(255); };
         // one pass: a look-back word per block and the ticket; else block
-        // metadata and base-exponent candidates
+        // metadata and base-exponent candidates (which hold a one-pass call's
+        // look-back words as well)
         const bool fused = kvexp_launch::encode_fused_supported(dim, bt) && aligned16(d_kv);
-        const size_t meta_bytes = fused ? 256u + up(size_t(nb) * sizeof(uint64_t)) : up(size_t(nb) * sizeof(EncBlockMeta));
-        const size_t base_bytes = fused ? 0 : up(size_t(nb) * 3u * size_t(dim));
+        const bool small = fused && int64_t(bt) * dim <= kvexp_dev::kNoAllocFusedElems;
+        const size_t meta_bytes = small ? 256u + up(size_t(nb) * sizeof(uint64_t)) : up(size_t(nb) * sizeof(EncBlockMeta));
+        const size_t base_bytes = small ? 0 : up(size_t(nb) * 3u * size_t(dim));
         const size_t need = meta_bytes + base_bytes + 256u; // + a status word when d_status is NULL
         if (need > kvexp_dev::kNoAllocScratchBytes)
             fail(KVEXP_HIP_CAPACITY, "kvexp_hip_encode_noalloc: " + std::to_string(nb) + " blocks of head_dim " +
