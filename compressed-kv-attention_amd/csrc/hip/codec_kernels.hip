@@ -712,17 +712,9 @@ __device__ __forceinline__ void copy_rows(const AppendJobDev &j, int dim) {
     for (int i = int(threadIdx.x); i < total; i += int(blockDim.x)) to[i] = from[i];
 }
 
-// Each job's rows of copy_rows (after the write kernel has read it).
-// With `terminal` set (after the fused encoder, which writes the index of
-// the jobs with blocks), also the index entry of an empty container.
-__global__ __launch_bounds__(kThreads) void append_tail_kernel(const AppendJobDev *__restrict__ jobs, int dim,
-                                                              int terminal) {
-    const AppendJobDev j = jobs[blockIdx.x];
-    if (terminal && j.nb == 0 && threadIdx.x == 0) {
-        j.offs[0] = j.rebase ? j.offs[0] : 0;
-        j.first[0] = j.tok0;
-    }
-    copy_rows(j, dim);
+// Each job's rows of copy_rows (after the write kernel has read the tail).
+__global__ __launch_bounds__(kThreads) void append_tail_kernel(const AppendJobDev *__restrict__ jobs, int dim) {
+    copy_rows(jobs[blockIdx.x], dim);
 }
 
 // ------------------------------------------------ encode: one fused pass --
@@ -962,9 +954,20 @@ encode_fused_kernel(const AppendJobDev *__restrict__ jobs, AppendJobDev one, int
     // prefetch (the job's draws number P)
     const bool one_shot = gridDim.x >= uint32_t(j.nb);
     const uint32_t last_draw = (one_shot ? 0u : uint32_t(j.nb)) + gridDim.x - 1u;
+    if (j.nb == 0) { // an empty container: its terminal index entry
+        if (tid == 0 && blockIdx.x == 0) {
+            j.offs[0] = j.rebase ? j.offs[0] : 0;
+            j.first[0] = j.tok0;
+        }
+        return;
+    }
     if (tid == 0) {
-        const uint32_t t = atomicAdd(tickets + jx, 1u);
-        if (t == last_draw) atomicExch(tickets + jx, 0u);
+        // (a decode step's append: one workgroup and one block per job, no draw)
+        uint32_t t = 0;
+        if (last_draw != 0) {
+            t = atomicAdd(tickets + jx, 1u);
+            if (t == last_draw) atomicExch(tickets + jx, 0u);
+        }
         s_ticket = t;
     }
     // first channel of chunk c (8 * (c mod dim / 8); the float quotient is
@@ -1307,6 +1310,16 @@ encode_fused_kernel(const AppendJobDev *__restrict__ jobs, AppendJobDev one, int
         }
         __syncthreads();
         KVEXP_ENC_MARK(7);
+        // the job's raw tail for the next append, by its last block's workgroup:
+        // the look-back has shown that every earlier block published its size,
+        // so the first block, which alone reads the old tail, has its tokens
+        // (source and tail are 16-byte aligned here)
+        if (JOBS && b == j.nb - 1) {
+            const uint4 *from = reinterpret_cast<const uint4 *>(j.src) + size_t(j.copy_from) * size_t(cpr);
+            uint4 *to = reinterpret_cast<uint4 *>(j.tail) + j.copy_to * cpr;
+#pragma unroll 1
+            for (int i = tid; i < j.copy_rows * cpr; i += TH) to[i] = from[i];
+        }
 
         // ---- the staged bytes to the container: 16-byte aligned stores, the
         // bytes before the first aligned address and after the last one alone
@@ -1373,7 +1386,8 @@ __global__ __launch_bounds__(256) void clear_lookback_kernel(uint64_t *__restric
 }
 
 // Append jobs that encode one block each (a decode step: the trailing block
-// plus one token never exceeds a block), fused in one launch: one workgroup
+// plus one token never exceeds a block) of shapes that the one-pass encoder
+// does not take, fused in one launch: one workgroup
 // (kThreads) per job computes the block's statistics, its place (the
 // container's trailing-block offset, which no other job touches), writes it
 // and the index entries around it, then stores the raw rows kept for the
@@ -1416,36 +1430,89 @@ __global__ __launch_bounds__(kThreads) void append_one_kernel(const AppendJobDev
 // takes the i-th escape word, which the format stores after the codes; a
 // sentinel count other than n_escape raises kStEscape. All threads of the
 // workgroup call it.
+// octets (total % 8 == 0, as head_dim is a multiple of 8): a segment of 16,384
+// codes at a time, all of its code words in flight together and one barrier
+// for the waves' counts, as in decode_coded (c2's plan update: 8.2 us per
+// launch with a scan and its two barriers every 1,024 codes).
+template <int MODE>
+__device__ __forceinline__ int escape_octets(const uint8_t *codes, int octets, int n_escape,
+                                             uint32_t *__restrict__ pos, int *tmp) {
+    constexpr uint32_t sentinel = (1u << MODE) - 1u;
+    const uint8_t *words = codes + MODE * size_t(octets);
+    const int lane = lane_id(), w = int(threadIdx.x) >> 6;
+    int carry = 0;
+    for (int seg = 0; seg < octets; seg += kDecSegment / 8) {
+        const int o0 = seg + w * (kDecSteps * kWave) + lane;
+        uint32_t cw[kDecSteps];
+        int cnt[kDecSteps], mine = 0;
+#pragma unroll
+        for (int k = 0; k < kDecSteps; ++k) cw[k] = dec_codes<MODE>(codes, min(o0 + kWave * k, octets - 1));
+#pragma unroll
+        for (int k = 0; k < kDecSteps; ++k) {
+            cnt[k] = o0 + kWave * k < octets ? unit_sentinels(cw[k], MODE) : 0;
+            mine += cnt[k];
+        }
+        const int sum = wave_sum_i32(mine);
+        __syncthreads(); // the last segment's totals are read
+        if (lane == 0) tmp[w] = sum;
+        __syncthreads();
+        int rank = carry;
+#pragma unroll
+        for (int i = 0; i < kWaves; ++i) {
+            rank += i < w ? tmp[i] : 0;
+            carry += tmp[i];
+        }
+#pragma unroll
+        for (int k = 0; k < kDecSteps; ++k) {
+            if (__ballot(cnt[k] != 0) == 0) continue;
+            const int incl = wave_scan_add(cnt[k]);
+            int r = rank + incl - cnt[k];
+            rank += __builtin_amdgcn_readlane(incl, kWave - 1);
+            if (cnt[k] == 0) continue;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                if (((cw[k] >> (MODE * i)) & sentinel) != sentinel) continue;
+                if (r < n_escape)
+                    pos[r] = uint32_t(8 * (o0 + kWave * k) + i) |
+                             (uint32_t(*reinterpret_cast<const dec_u16 *>(words + 2 * size_t(r))) << 16);
+                ++r;
+            }
+        }
+    }
+    return carry;
+}
+
 __device__ __forceinline__ void escape_positions(const uint8_t *codes, int mode, int total, int n_escape,
                                                  uint32_t *__restrict__ pos, int *scan_tmp,
                                                  uint32_t *__restrict__ status) {
-    const uint8_t *words = codes + (total * mode + 7) / 8;
-    const int U = code_unit(mode);
-    const uint32_t sentinel = (1u << mode) - 1u;
-    const int units = total / U;
     int carry = 0;
-    for (int r = 0; r < units; r += kThreads) {
-        const int u = r + int(threadIdx.x);
-        const bool act = u < units;
-        uint32_t cw = 0;
-        int cnt = 0;
-        if (act) {
-            cw = load_codes(codes, mode, u);
-            cnt = unit_sentinels(cw, mode);
-        }
-        int tot = 0;
-        int rank = carry + block_excl_scan<kWaves>(cnt, scan_tmp, &tot);
-        carry += tot;
-        if (act && cnt) {
+    if (total % 8 == 0) {
+        carry = mode == 4   ? escape_octets<4>(codes, total / 8, n_escape, pos, scan_tmp)
+                : mode == 2 ? escape_octets<2>(codes, total / 8, n_escape, pos, scan_tmp)
+                            : escape_octets<3>(codes, total / 8, n_escape, pos, scan_tmp);
+    } else { // 2- and 4-bit codes, four elements per thread and step
+        const uint8_t *words = codes + (total * mode + 7) / 8;
+        const uint32_t sentinel = (1u << mode) - 1u;
+        const int units = total / 4;
+        for (int r = 0; r < units; r += kThreads) {
+            const int u = r + int(threadIdx.x);
+            const bool act = u < units;
+            uint32_t cw = 0;
+            int cnt = 0;
+            if (act) {
+                cw = load_codes(codes, mode, u);
+                cnt = unit_sentinels(cw, mode);
+            }
+            int tot = 0;
+            int rank = carry + block_excl_scan<kWaves>(cnt, scan_tmp, &tot);
+            carry += tot;
+            if (act && cnt) {
 #pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                if (k >= U) break;
-                if (unit_code(cw, mode, k) == sentinel) {
-                    if (rank < n_escape) {
-                        const uint32_t w = uint32_t(words[2 * rank]) | (uint32_t(words[2 * rank + 1]) << 8);
-                        pos[rank] = uint32_t(U * u + k) | (w << 16);
+                for (int k = 0; k < 4; ++k) {
+                    if (unit_code(cw, mode, k) == sentinel) {
+                        if (rank < n_escape) pos[rank] = uint32_t(4 * u + k) | (load_u16_any(words + 2 * rank) << 16);
+                        ++rank;
                     }
-                    ++rank;
                 }
             }
         }
@@ -1498,6 +1565,25 @@ __global__ __launch_bounds__(kThreads) void esc_start_kernel(const EscJob *__res
     if (threadIdx.x == 0) j.esc0[j.n_blocks] = carry;
 }
 
+// The block first tokens of every tensor of a plan, one after another in
+// `out` (one workgroup per tensor): the host then reads them with one copy
+// (c2's 96 tensors took 96 copies, about 0.9 ms of a plan's 1.25).
+__global__ __launch_bounds__(kThreads) void gather_first_kernel(const FirstJob *__restrict__ jobs,
+                                                               int32_t *__restrict__ out) {
+    const FirstJob j = jobs[blockIdx.x];
+    for (int i = int(threadIdx.x); i < j.n; i += kThreads) out[j.at + i] = j.first[i];
+}
+
+// A 64-bit word (nullable) and the status word to host memory that the GPU can
+// write (the caller then synchronises the stream): one small launch in place
+// of two copies to pageable memory.
+__global__ void result_kernel(const int64_t *__restrict__ value, const uint32_t *__restrict__ status,
+                              int64_t *__restrict__ host) {
+    host[0] = value != nullptr ? *value : 0;
+    host[1] = int64_t(*status);
+    __threadfence_system();
+}
+
 // Element index of every escape of one block (one workgroup per block;
 // `blocks` lists (job, block) pairs).
 __global__ __launch_bounds__(kThreads) void esc_pos_kernel(const EscJob *__restrict__ jobs,
@@ -1529,25 +1615,29 @@ __global__ __launch_bounds__(kThreads) void esc_pos_kernel(const EscJob *__restr
 // attended tokens raises kStIndex. The workgroups after them set each device
 // head's length and byte counts and the end of each head's last split from
 // the jobs (tensors 2h and 2h + 1 are the K and V of head h, which owns
-// device heads [h * per_head, (h + 1) * per_head)).
+// device heads [h * per_head, (h + 1) * per_head)). The lengths come as a
+// kernel argument where lens.n is not 0 (the byte counts are then those of the
+// last update), else from the jobs.
 __global__ __launch_bounds__(kThreads) void plan_refresh_kernel(const EscJob *__restrict__ jobs, int n_jobs,
                                                                HeadDev *__restrict__ heads, int n_dev_heads,
                                                                WorkItem *__restrict__ items, int n_items,
-                                                               int per_head, uint32_t *__restrict__ status) {
+                                                               int per_head, uint32_t *__restrict__ status,
+                                                               PlanLens lens) {
     __shared__ int scan_tmp[kWaves];
     __shared__ int ok_s;
+    auto seq_of = [&](int h) { return lens.n > 0 ? lens.seq[h] : jobs[2 * h].seq; };
     if (int(blockIdx.x) >= n_jobs) {
         const int i = (int(blockIdx.x) - n_jobs) * kThreads + int(threadIdx.x);
         if (i < n_dev_heads) {
             const int h = i / per_head;
-            heads[i].seq = jobs[2 * h].seq;
+            heads[i].seq = seq_of(h);
             heads[i].kbytes = jobs[2 * h].bytes;
             heads[i].vbytes = jobs[2 * h + 1].bytes;
         }
         if (i < n_items) {
             WorkItem &w = items[i];
             const int h = w.head / per_head;
-            if (w.split == heads[w.head].n_splits - 1) w.tok_end = jobs[2 * h].seq;
+            if (w.split == heads[w.head].n_splits - 1) w.tok_end = seq_of(h);
         }
         return;
     }
@@ -1561,7 +1651,7 @@ __global__ __launch_bounds__(kThreads) void plan_refresh_kernel(const EscJob *__
         uint32_t st = check_block(j.blob, j.bytes, off, dim, j.first[b + 1] - j.first[b], &h);
         const int ne = st != 0u || h.mode == 0 ? 0 : h.n_escape;
         if (st == 0u && e0 + ne > j.pos_cap) st = kStEscape;
-        if (j.first[j.n_blocks] < j.seq) st |= kStIndex;
+        if (j.first[j.n_blocks] < seq_of(int(blockIdx.x) / 2)) st |= kStIndex;
         BlockDesc d{};
         d.data = j.blob + off;
         d.esc = j.pos + e0;
@@ -1707,18 +1797,11 @@ hipError_t append(const AppendJobDev *jobs, int n_jobs, int total_blocks, int di
                   uint8_t *bases, uint32_t *status, hipStream_t s, bool one_block, int modes, const EncLookback *lb,
                   int max_job_blocks) {
     if (n_jobs <= 0) return hipSuccess;
+    if (lb != nullptr) // one pass, which also writes the index of empty containers and keeps the tails
+        return encode_fused(jobs, n_jobs, AppendJobDev{}, max_job_blocks, dim, bt, modes, *lb, status, s);
     if (one_block) {
         const size_t lds = stats_lds_bytes(dim) + 3 * size_t(dim);
         hipLaunchKernelGGL(append_one_kernel, dim3(n_jobs), dim3(kThreads), lds, s, jobs, dim, bt, status, modes);
-        return hipGetLastError();
-    }
-    if (lb != nullptr) { // one pass, then the tails (and the index of empty containers)
-        if (total_blocks > 0) {
-            const hipError_t e =
-                encode_fused(jobs, n_jobs, AppendJobDev{}, max_job_blocks, dim, bt, modes, *lb, status, s);
-            if (e != hipSuccess) return e;
-        }
-        hipLaunchKernelGGL(append_tail_kernel, dim3(n_jobs), dim3(kThreads), 0, s, jobs, dim, 1);
         return hipGetLastError();
     }
     if (total_blocks > 0)
@@ -1728,7 +1811,7 @@ hipError_t append(const AppendJobDev *jobs, int n_jobs, int total_blocks, int di
     if (total_blocks > 0)
         hipLaunchKernelGGL(append_write_kernel, dim3(total_blocks), dim3(kThreads), 0, s, jobs, n_jobs, dim, bt, meta,
                            bases, status);
-    hipLaunchKernelGGL(append_tail_kernel, dim3(n_jobs), dim3(kThreads), 0, s, jobs, dim, 0);
+    hipLaunchKernelGGL(append_tail_kernel, dim3(n_jobs), dim3(kThreads), 0, s, jobs, dim);
     return hipGetLastError();
 }
 
@@ -1739,11 +1822,22 @@ hipError_t esc_start(const EscJob *jobs, int n_jobs, uint32_t *status, hipStream
 }
 
 hipError_t plan_refresh(const EscJob *jobs, int n_jobs, HeadDev *heads, int n_dev_heads, WorkItem *items,
-                        int n_items, int per_head, uint32_t *status, hipStream_t s) {
+                        int n_items, int per_head, uint32_t *status, const PlanLens &lens, hipStream_t s) {
     const int extra = (std::max(n_dev_heads, n_items) + kThreads - 1) / kThreads;
     if (n_jobs + extra <= 0) return hipSuccess;
     hipLaunchKernelGGL(plan_refresh_kernel, dim3(n_jobs + extra), dim3(kThreads), 0, s, jobs, n_jobs, heads,
-                       n_dev_heads, items, n_items, per_head, status);
+                       n_dev_heads, items, n_items, per_head, status, lens);
+    return hipGetLastError();
+}
+
+hipError_t result(const int64_t *value, const uint32_t *status, int64_t *host, hipStream_t s) {
+    hipLaunchKernelGGL(result_kernel, dim3(1), dim3(1), 0, s, value, status, host);
+    return hipGetLastError();
+}
+
+hipError_t gather_first(const FirstJob *jobs, int n_jobs, int32_t *out, hipStream_t s) {
+    if (n_jobs <= 0) return hipSuccess;
+    hipLaunchKernelGGL(gather_first_kernel, dim3(n_jobs), dim3(kThreads), 0, s, jobs, out);
     return hipGetLastError();
 }
 

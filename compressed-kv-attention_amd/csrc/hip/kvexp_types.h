@@ -71,6 +71,20 @@ struct EscJob {
     int32_t seq;          // tokens a plan update attends (esc_tail_kernel checks the index covers them)
 };
 
+// One tensor's block first tokens for gather_first_kernel: n entries to out[at].
+struct FirstJob {
+    const int32_t *first;
+    int32_t n, at;
+};
+
+// Lengths of a plan's heads as a kernel argument (a plan update then uploads
+// nothing); n 0: not used.
+constexpr int kPlanLens = 512;
+struct PlanLens {
+    int32_t n;
+    int32_t seq[kPlanLens];
+};
+
 // One split: tokens [tok_begin, tok_end) of a head; for XKV the blocks that
 // hold tok_begin in K and V, as block indexes of the head's tensors and (one-
 // wave kernel plans) as indexes into the plan's descriptor array (-1

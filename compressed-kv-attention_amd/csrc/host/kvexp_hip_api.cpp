@@ -43,7 +43,9 @@ hipError_t expf(const float *x, float *y, size_t n, hipStream_t s);
 hipError_t esc_start(const kvexp_dev::EscJob *jobs, int n_jobs, uint32_t *status, hipStream_t s);
 hipError_t esc_pos(const kvexp_dev::EscJob *jobs, const int2 *blocks, int n_blocks, uint32_t *status, hipStream_t s);
 hipError_t plan_refresh(const kvexp_dev::EscJob *jobs, int n_jobs, HeadDev *heads, int n_dev_heads, WorkItem *items,
-                        int n_items, int per_head, uint32_t *status, hipStream_t s);
+                        int n_items, int per_head, uint32_t *status, const kvexp_dev::PlanLens &lens, hipStream_t s);
+hipError_t result(const int64_t *value, const uint32_t *status, int64_t *host, hipStream_t s);
+hipError_t gather_first(const kvexp_dev::FirstJob *jobs, int n_jobs, int32_t *out, hipStream_t s);
 bool wave_supports(int dim);
 hipError_t attention_wave(bool xkv, int order, int G, int dim, const HeadDev *heads, const WorkItem *items,
                           int n_items, int wpg, const kvexp_dev::BlockDesc *desc, const uint16_t *q, float *out,
@@ -163,6 +165,7 @@ struct DevBuf {
     void *p = nullptr;
     DevPool *pool = nullptr;
     size_t cap = 0;
+    bool part = false;
     DevBuf() = default;
     explicit DevBuf(size_t n) {
         if (n) HIPX(hipMalloc(&p, n));
@@ -177,15 +180,23 @@ struct DevBuf {
     }
     DevBuf(const DevBuf &) = delete;
     DevBuf &operator=(const DevBuf &) = delete;
-    DevBuf(DevBuf &&o) noexcept : p(o.p), pool(o.pool), cap(o.cap) { o.p = nullptr; }
+    DevBuf(DevBuf &&o) noexcept : p(o.p), pool(o.pool), cap(o.cap), part(o.part) { o.p = nullptr; }
     DevBuf &operator=(DevBuf &&o) noexcept {
         std::swap(p, o.p);
         std::swap(pool, o.pool);
         std::swap(cap, o.cap);
+        std::swap(part, o.part);
         return *this;
     }
+    // A part of another allocation, which outlives it.
+    static DevBuf part_of(void *at) {
+        DevBuf b;
+        b.p = at;
+        b.part = true;
+        return b;
+    }
     ~DevBuf() {
-        if (p == nullptr) return;
+        if (p == nullptr || part) return;
         if (pool) pool->put(p, cap);
         else (void)hipFree(p);
     }
@@ -239,10 +250,17 @@ struct kvexp_hip_ctx {
     // pinned host staging for the plan builder's reads of block indexes
     void *pinned = nullptr;
     size_t pinned_cap = 0;
+    // pinned result slots (two words each, written by result_kernel): leased
+    // per call, since plans of one context may be checked from several threads
+    static constexpr int kResultSlots = 64;
+    std::mutex result_mu;
+    int64_t *results = nullptr;
+    uint64_t results_used = 0;
     ~kvexp_hip_ctx() {
         if (stream) (void)hipStreamSynchronize(stream);
         if (scratch_done) (void)hipEventSynchronize(scratch_done);
         if (pinned) (void)hipHostFree(pinned);
+        if (results) (void)hipHostFree(results);
         if (scratch_done) (void)hipEventDestroy(scratch_done);
         if (stream) (void)hipStreamDestroy(stream);
     }
@@ -253,7 +271,21 @@ struct kvexp_hip_plan {
     // buffers from the context's pool (plans of the host-pointer entry, which
     // synchronises its stream before destroying them); others are freed
     bool pooled = false;
-    DevBuf alloc(size_t n) const { return DevBuf(pooled ? &ctx->pool : nullptr, n); }
+    // The plan's device arrays lie in one allocation (plan_build sizes it before
+    // the first of them is taken; an allocation takes about 30 us, so eleven of
+    // them were a quarter of a rebuild), an array past its end in one of its own.
+    static size_t padded(size_t n) { return (n + 255u) & ~size_t(255); }
+    void reserve(size_t n) {
+        arena = DevBuf(pooled ? &ctx->pool : nullptr, n);
+        arena_size = n;
+        arena_used = 0;
+    }
+    DevBuf alloc(size_t n) {
+        if (arena_used + padded(n) > arena_size) return DevBuf(pooled ? &ctx->pool : nullptr, n);
+        void *at = arena.as<uint8_t>() + arena_used;
+        arena_used += padded(n);
+        return DevBuf::part_of(at);
+    }
     int n_heads = 0, n_q = 0, dim = 0, order = 0, split_tokens = 0;
     // set when kvexp_hip_plan_update failed after the containers changed: the
     // plan's descriptors no longer describe them, so runs are refused until
@@ -268,8 +300,11 @@ struct kvexp_hip_plan {
     std::vector<kvexp_dev::EscJob> jobs;
     std::vector<int32_t> esc_prefix; // per tensor (jobs order): escapes before each block, n_blocks + 1 entries
     std::vector<size_t> esc_prefix_at;
+    DevBuf arena; // declared before its parts
+    size_t arena_size = 0, arena_used = 0;
     DevBuf djobs;
-    bool wave = false; // one-wave-per-split kernel (dim 64 or 128)
+    bool jobs_uploaded = false; // djobs holds `jobs` but for the lengths
+    bool wave = false; // the one-wave or team split kernels (kvexp_launch::wave_supports)
     DevBuf heads, items, merge_ids, ws, status;
     // wave kernel: merge work (head, row), escape records, block descriptors
     DevBuf mitems, esc0, escpos, desc;
@@ -357,10 +392,67 @@ void scratch_used(kvexp_hip_ctx *ctx, hipStream_t s) {
     HIPX(hipEventRecord(ctx->scratch_done, s));
 }
 
-void check_status_word(uint32_t *d_status, hipStream_t s) {
-    uint32_t st = 0;
-    HIPX(hipMemcpyAsync(&st, d_status, sizeof st, hipMemcpyDeviceToHost, s));
+// The context's pinned staging buffer, at least n bytes (its last use is over:
+// every user synchronises its stream before it returns). It grows by half more
+// than asked for: a decode loop's rebuilds each need a little more.
+void *pinned_staging(kvexp_hip_ctx *ctx, size_t n) {
+    if (n > ctx->pinned_cap) {
+        n += n / 2;
+        if (ctx->pinned) HIPX(hipHostFree(ctx->pinned));
+        ctx->pinned = nullptr;
+        ctx->pinned_cap = 0;
+        HIPX(hipHostMalloc(&ctx->pinned, n, hipHostMallocDefault));
+        ctx->pinned_cap = n;
+    }
+    return ctx->pinned;
+}
+
+// A leased pinned result slot (p null when all are leased).
+struct ResultSlot {
+    kvexp_hip_ctx *ctx;
+    volatile int64_t *p = nullptr;
+    int i = -1;
+    explicit ResultSlot(kvexp_hip_ctx *c) : ctx(c) {
+        std::lock_guard<std::mutex> lock(c->result_mu);
+        if (c->results == nullptr)
+            HIPX(hipHostMalloc(reinterpret_cast<void **>(&c->results), kvexp_hip_ctx::kResultSlots * 16,
+                               hipHostMallocDefault));
+        if (c->results_used == ~uint64_t(0)) return;
+        i = __builtin_ctzll(~c->results_used);
+        c->results_used |= uint64_t(1) << i;
+        p = c->results + 2 * i;
+    }
+    ResultSlot(const ResultSlot &) = delete;
+    ~ResultSlot() {
+        if (i < 0) return;
+        std::lock_guard<std::mutex> lock(ctx->result_mu);
+        ctx->results_used &= ~(uint64_t(1) << i);
+    }
+};
+
+// Synchronises `s` and returns the status word; *value (nullable) receives
+// the device word d_value. Through a pinned slot that the GPU writes (one
+// tensor's encode call: 49 us with two copies to pageable memory, 32 so).
+uint32_t read_result(kvexp_hip_ctx *ctx, const int64_t *d_value, const uint32_t *d_status, int64_t *value,
+                     hipStream_t s) {
+    ResultSlot slot(ctx);
+    if (slot.p == nullptr) { // every slot leased
+        int64_t v = 0;
+        uint32_t st = 0;
+        if (d_value != nullptr) HIPX(hipMemcpyAsync(&v, d_value, sizeof v, hipMemcpyDeviceToHost, s));
+        HIPX(hipMemcpyAsync(&st, d_status, sizeof st, hipMemcpyDeviceToHost, s));
+        HIPX(hipStreamSynchronize(s));
+        if (value != nullptr) *value = v;
+        return st;
+    }
+    HIPX(kvexp_launch::result(d_value, d_status, const_cast<int64_t *>(slot.p), s));
     HIPX(hipStreamSynchronize(s));
+    if (value != nullptr) *value = slot.p[0];
+    return uint32_t(slot.p[1]);
+}
+
+void check_status_word(kvexp_hip_ctx *ctx, uint32_t *d_status, hipStream_t s) {
+    const uint32_t st = read_result(ctx, nullptr, d_status, nullptr, s);
     if (st != 0u) {
         HIPX(hipMemsetAsync(d_status, 0, sizeof(uint32_t), s));
         HIPX(hipStreamSynchronize(s));
@@ -408,10 +500,13 @@ void build_escape_index(kvexp_hip_plan &p, const kvexp_hip_head *heads, int n_he
     for (auto &j : jobs1) j.desc = nullptr;
     HIPX(hipMemcpyAsync(djobs.p, jobs1.data(), jobs1.size() * sizeof(kvexp_dev::EscJob), hipMemcpyHostToDevice, s));
     HIPX(kvexp_launch::esc_start(djobs.as<kvexp_dev::EscJob>(), int(jobs.size()), st, s));
-    check_status_word(st, s);
-    std::vector<int32_t> e0(e0_total);
-    HIPX(hipMemcpyAsync(e0.data(), p.esc0.p, e0_total * sizeof(int32_t), hipMemcpyDeviceToHost, s));
+    // the status word and the escape counts with one synchronisation
+    auto *host = static_cast<int32_t *>(pinned_staging(p.ctx, (e0_total + 1) * sizeof(int32_t)));
+    HIPX(hipMemcpyAsync(host, st, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+    HIPX(hipMemcpyAsync(host + 1, p.esc0.p, e0_total * sizeof(int32_t), hipMemcpyDeviceToHost, s));
     HIPX(hipStreamSynchronize(s));
+    if (host[0] != 0) check_status_word(p.ctx, st, s); // clears the word and reports it
+    std::vector<int32_t> e0(host + 1, host + 1 + e0_total);
     p.esc_prefix = e0;
     p.esc_prefix_at = e0_at;
     // each tensor's positions, then room for its last block to grow to the
@@ -437,9 +532,10 @@ void build_escape_index(kvexp_hip_plan &p, const kvexp_hip_head *heads, int n_he
     DevBuf dblocks = p.alloc(std::max<size_t>(blocks.size(), 1) * sizeof(int2));
     HIPX(hipMemcpyAsync(dblocks.p, blocks.data(), blocks.size() * sizeof(int2), hipMemcpyHostToDevice, s));
     HIPX(kvexp_launch::esc_pos(djobs.as<kvexp_dev::EscJob>(), dblocks.as<int2>(), int(blocks.size()), st, s));
-    check_status_word(st, s); // synchronises s: the host vectors above may go
+    check_status_word(p.ctx, st, s); // synchronises s: the host vectors above may go
     p.jobs = jobs;
     p.djobs = std::move(djobs);
+    p.jobs_uploaded = true;
     const int per_head = (n_q + kMaxQPerLaunch - 1) / kMaxQPerLaunch;
     for (int h = 0; h < n_heads; ++h) {
         for (int c = 0; c < per_head; ++c) {
@@ -603,10 +699,7 @@ int kvexp_hip_encode(kvexp_hip_ctx *ctx, const uint16_t *d_kv, int seq, int dim,
         scratch_used(ctx, s);
         if (bytes_out != nullptr) {
             int64_t total = 0;
-            uint32_t st = 0;
-            HIPX(hipMemcpyAsync(&total, offs + nb, sizeof total, hipMemcpyDeviceToHost, s));
-            HIPX(hipMemcpyAsync(&st, ctx->status.p, sizeof st, hipMemcpyDeviceToHost, s));
-            HIPX(hipStreamSynchronize(s));
+            const uint32_t st = read_result(ctx, offs + nb, ctx->status.as<uint32_t>(), &total, s);
             if (st != 0u) {
                 HIPX(hipMemsetAsync(ctx->status.p, 0, sizeof(uint32_t), s));
                 HIPX(hipStreamSynchronize(s));
@@ -744,14 +837,14 @@ void run_append(kvexp_hip_ctx *ctx, const kvexp_hip_append_job *jobs, int n_jobs
     int blocks = 0;
     for (int i = 0; i < n_jobs; ++i) blocks += add_append_job(jobs[i], dim, bt, blocks, dj);
     if (dj.empty()) return;
-    // every job encodes at most one block (a decode step): one fused launch
+    // every job encodes at most one block (a decode step)
     const bool one_block = std::all_of(dj.begin(), dj.end(), [](const AppendJobDev &j) { return j.nb <= 1; });
-    // several blocks: one pass when the shape fits it and every source is
-    // 16-byte aligned (the tails are allocated so; the new tokens' rows are
-    // then aligned too, since dim % 8 == 0)
+    // one launch of the one-pass encoder when the shape fits it and every
+    // source is 16-byte aligned (the tails are allocated so; the new tokens'
+    // rows are then aligned too, since dim % 8 == 0)
     int max_nb = 0;
     for (const AppendJobDev &j : dj) max_nb = std::max(max_nb, j.nb);
-    const bool fused = !one_block && kvexp_launch::encode_fused_supported(dim, bt) && dj.size() <= 65535u &&
+    const bool fused = kvexp_launch::encode_fused_supported(dim, bt) && dj.size() <= 65535u &&
                        std::all_of(dj.begin(), dj.end(), [](const AppendJobDev &j) {
                            return aligned16(j.src) && aligned16(j.tail);
                        });
@@ -774,10 +867,10 @@ void run_append(kvexp_hip_ctx *ctx, const kvexp_hip_append_job *jobs, int n_jobs
     scratch_used(ctx, s);
 }
 
-void check_encoder_status(kvexp_hip_ctx *ctx, hipStream_t s) {
-    uint32_t st = 0;
-    HIPX(hipMemcpyAsync(&st, ctx->status.p, sizeof st, hipMemcpyDeviceToHost, s));
-    HIPX(hipStreamSynchronize(s));
+// Synchronises `s`; *value (nullable) receives the device word d_value.
+void check_encoder_status(kvexp_hip_ctx *ctx, hipStream_t s, const int64_t *d_value = nullptr,
+                          int64_t *value = nullptr) {
+    const uint32_t st = read_result(ctx, d_value, ctx->status.as<uint32_t>(), value, s);
     if (st != 0u) {
         HIPX(hipMemsetAsync(ctx->status.p, 0, sizeof(uint32_t), s));
         HIPX(hipStreamSynchronize(s));
@@ -810,8 +903,7 @@ int kvexp_hip_append(kvexp_hip_ctx *ctx, const uint16_t *d_new, int n_new, int n
         if (bytes_out != nullptr) {
             const int nb_all = kvexp_hip_block_count(n_tokens + n_new, bt);
             int64_t bytes = 0;
-            HIPX(hipMemcpyAsync(&bytes, d_offsets + nb_all, sizeof bytes, hipMemcpyDeviceToHost, s));
-            check_encoder_status(ctx, s);
+            check_encoder_status(ctx, s, d_offsets + nb_all, &bytes);
             *bytes_out = size_t(bytes);
         }
     });
@@ -854,7 +946,7 @@ int kvexp_hip_decode(kvexp_hip_ctx *ctx, const uint8_t *d_blob, size_t bytes, co
         HIPX(kvexp_launch::decode(d_blob, bytes, d_offsets, d_first_token, n_blocks, check ? seq : 0, seq, dim, d_out,
                                   ctx->status.as<uint32_t>(), s));
         scratch_used(ctx, s);
-        if (check) check_status_word(ctx->status.as<uint32_t>(), s);
+        if (check) check_status_word(ctx, ctx->status.as<uint32_t>(), s);
     });
 }
 
@@ -909,6 +1001,14 @@ int kvexp_hip_suggest_splits_batch(kvexp_hip_ctx *ctx, int n_heads, const int *s
 
 namespace {
 
+// std::lower_bound(f, f + n, tok) on a tensor's block first tokens (ascending),
+// tried first where blocks of `bt` tokens would put it.
+int first_block_at(const int32_t *f, int n, int tok, int bt) {
+    const int g = (tok + bt - 1) / bt;
+    if (g >= 0 && g < n && f[g] >= tok && (g == 0 || f[g - 1] < tok)) return g;
+    return int(std::lower_bound(f, f + n, tok) - f);
+}
+
 // Orders each query-row group's work items so that the waves sharing a SIMD
 // carry similar work. The dispatcher places workgroup g on XCD g % 8 and the
 // workgroups g, g + C, g + 2C, ... (C = CU count) on the same CU, one wave
@@ -935,7 +1035,7 @@ void balance_items(kvexp_hip_plan &p, std::vector<WorkItem> &items, bool xkv, co
             const int32_t *f0 = first_all + first_at[t];
             const int nb = p.jobs[t].n_blocks;
             const int b0 = kv ? w.vblk : w.kblk;
-            const int b1 = int(std::lower_bound(f0, f0 + nb, w.tok_end) - f0);
+            const int b1 = first_block_at(f0, nb, w.tok_end, p.split_tokens);
             const int32_t *e = p.esc_prefix.data() + p.esc_prefix_at[t];
             c += double(e[b1] - e[b0]) / 15.0;
         }
@@ -974,8 +1074,6 @@ void balance_items(kvexp_hip_plan &p, std::vector<WorkItem> &items, bool xkv, co
 // indexes it reads) and synchronises only `s`. Status words: the plan's own.
 void plan_build(kvexp_hip_plan *p, const kvexp_hip_head *heads, int n_heads, hipStream_t s) {
     kvexp_hip_ctx *ctx = p->ctx;
-    p->status = p->alloc(sizeof(uint32_t));
-    HIPX(hipMemsetAsync(p->status.p, 0, sizeof(uint32_t), s));
     const int n_q = p->n_q, dim = p->dim, split_tokens = p->split_tokens;
     const bool xkv = heads[0].k_xkv != nullptr;
     std::vector<HeadDev> hv;
@@ -998,25 +1096,29 @@ void plan_build(kvexp_hip_plan *p, const kvexp_hip_head *heads, int n_heads, hip
             first_at[size_t(2 * h + 1)] = total;
             total += size_t(H.v_n_blocks) + 1;
         }
-        if (total * 4 > ctx->pinned_cap) {
-            if (ctx->pinned) HIPX(hipHostFree(ctx->pinned));
-            ctx->pinned = nullptr;
-            ctx->pinned_cap = 0;
-            HIPX(hipHostMalloc(&ctx->pinned, total * 4, hipHostMallocDefault));
-            ctx->pinned_cap = total * 4;
-        }
-        int32_t *host = static_cast<int32_t *>(ctx->pinned);
+        std::vector<kvexp_dev::FirstJob> fj;
         for (int h = 0; h < n_heads; ++h) {
             const kvexp_hip_head &H = heads[h];
             if (H.k_xkv == nullptr || H.k_offsets == nullptr || H.v_offsets == nullptr ||
                 H.k_first_token == nullptr || H.v_first_token == nullptr || H.k_n_blocks <= 0 || H.v_n_blocks <= 0)
                 break;
-            HIPX(hipMemcpyAsync(host + first_at[size_t(2 * h)], H.k_first_token, (size_t(H.k_n_blocks) + 1) * 4,
-                                hipMemcpyDeviceToHost, s));
-            HIPX(hipMemcpyAsync(host + first_at[size_t(2 * h + 1)], H.v_first_token, (size_t(H.v_n_blocks) + 1) * 4,
-                                hipMemcpyDeviceToHost, s));
+            fj.push_back({H.k_first_token, H.k_n_blocks + 1, int32_t(first_at[size_t(2 * h)])});
+            fj.push_back({H.v_first_token, H.v_n_blocks + 1, int32_t(first_at[size_t(2 * h + 1)])});
         }
-        HIPX(hipStreamSynchronize(s));
+        auto *host = static_cast<int32_t *>(pinned_staging(ctx, total * sizeof(int32_t)));
+        if (total > size_t(INT32_MAX)) fail(KVEXP_HIP_UNSUPPORTED, "kvexp_hip_plan_create: too many blocks in one plan");
+        if (!fj.empty()) {
+            // from the context's pool: their use ends with the synchronisation below
+            DevBuf dj(&ctx->pool, fj.size() * sizeof(kvexp_dev::FirstJob)), out(&ctx->pool, total * sizeof(int32_t));
+            struct SyncOnExit { // (also when a call below fails: before the buffers go back)
+                hipStream_t s;
+                ~SyncOnExit() { (void)hipStreamSynchronize(s); }
+            } sync_on_exit{s};
+            HIPX(hipMemcpyAsync(dj.p, fj.data(), fj.size() * sizeof(kvexp_dev::FirstJob), hipMemcpyHostToDevice, s));
+            HIPX(kvexp_launch::gather_first(dj.as<kvexp_dev::FirstJob>(), int(fj.size()), out.as<int32_t>(), s));
+            HIPX(hipMemcpyAsync(host, out.p, total * sizeof(int32_t), hipMemcpyDeviceToHost, s));
+            HIPX(hipStreamSynchronize(s));
+        }
         firsts.assign(host, host + total);
         first_all = firsts.data();
     }
@@ -1066,8 +1168,8 @@ void plan_build(kvexp_hip_plan *p, const kvexp_hip_head *heads, int n_heads, hip
                 wi.kblk = wi.vblk = -1;
                 wi.kdi = wi.vdi = -1;
                 if (x) {
-                    const int32_t *kit = std::lower_bound(kf0, kf1, wi.tok_begin);
-                    const int32_t *vit = std::lower_bound(vf0, vf1, wi.tok_begin);
+                    const int32_t *kit = kf0 + first_block_at(kf0, H.k_n_blocks, wi.tok_begin, split_tokens);
+                    const int32_t *vit = vf0 + first_block_at(vf0, H.v_n_blocks, wi.tok_begin, split_tokens);
                     if (kit == kf1 || *kit != wi.tok_begin || vit == vf1 || *vit != wi.tok_begin)
                         fail(KVEXP_HIP_FORMAT_ERROR, "token split is not aligned to an encoded block");
                     wi.kblk = int(kit - kf0);
@@ -1084,18 +1186,39 @@ void plan_build(kvexp_hip_plan *p, const kvexp_hip_head *heads, int n_heads, hip
     }
     p->xkv = xkv;
     p->wave = kvexp_launch::wave_supports(dim);
+    const size_t slot_floats = size_t(kMaxQPerLaunch) * size_t(dim + 2);
+    {
+        using P = kvexp_hip_plan;
+        size_t n = P::padded(sizeof(uint32_t)) + P::padded(hv.size() * sizeof(HeadDev)) +
+                   P::padded(items.size() * sizeof(WorkItem)) +
+                   P::padded(std::max<size_t>(1, merge.size()) * sizeof(int32_t)) +
+                   P::padded(std::max<size_t>(1, size_t(ws_slots)) * slot_floats * sizeof(float)) +
+                   P::padded(size_t(2 * n_heads) * sizeof(kvexp_dev::EscJob));
+        if (p->wave) {
+            n += P::padded(std::max<size_t>(1, merge.size() * size_t(kMaxQPerLaunch)) * sizeof(kvexp_dev::MergeItem));
+            // per block: first escape, descriptor and the position builder's work list
+            const size_t e = firsts.size();
+            if (xkv)
+                n += P::padded(e * sizeof(int32_t)) + P::padded(e * sizeof(kvexp_dev::BlockDesc)) +
+                     P::padded(std::max<size_t>(1, e) * sizeof(int2));
+        }
+        p->reserve(n);
+    }
+    p->status = p->alloc(sizeof(uint32_t));
+    HIPX(hipMemsetAsync(p->status.p, 0, sizeof(uint32_t), s));
     p->n_dev_heads = int(hv.size());
     p->n_items = int(items.size());
     p->n_merge = int(merge.size());
     if (p->wave) {
         // items grouped by G (one launch per distinct G)
-        std::stable_sort(items.begin(), items.end(), [&](const WorkItem &a, const WorkItem &b) {
+        const auto fewer_rows = [&](const WorkItem &a, const WorkItem &b) {
             return hv[size_t(a.head)].n_q < hv[size_t(b.head)].n_q;
-        });
-        for (int G = 0; G <= 8; ++G)
-            p->group_start[G + 1] =
-                int(std::count_if(items.begin(), items.end(),
-                                  [&](const WorkItem &w) { return hv[size_t(w.head)].n_q <= G; }));
+        };
+        if (!std::is_sorted(items.begin(), items.end(), fewer_rows))
+            std::stable_sort(items.begin(), items.end(), fewer_rows);
+        for (int G = 0; G < 10; ++G) p->group_start[G] = 0;
+        for (const WorkItem &w : items) ++p->group_start[hv[size_t(w.head)].n_q + 1];
+        for (int G = 1; G < 10; ++G) p->group_start[G] += p->group_start[G - 1];
         std::vector<kvexp_dev::MergeItem> mi;
         for (int32_t dh : merge) {
             const HeadDev &d = hv[size_t(dh)];
@@ -1139,7 +1262,6 @@ void plan_build(kvexp_hip_plan *p, const kvexp_hip_head *heads, int n_heads, hip
     p->heads = p->alloc(hv.size() * sizeof(HeadDev));
     p->items = p->alloc(items.size() * sizeof(WorkItem));
     p->merge_ids = p->alloc(std::max<size_t>(1, merge.size()) * sizeof(int32_t));
-    const size_t slot_floats = size_t(kMaxQPerLaunch) * size_t(dim + 2);
     p->ws = p->alloc(std::max<size_t>(1, size_t(ws_slots)) * slot_floats * sizeof(float));
     HIPX(hipMemcpyAsync(p->heads.p, hv.data(), hv.size() * sizeof(HeadDev), hipMemcpyHostToDevice, s));
     HIPX(hipMemcpyAsync(p->items.p, items.data(), items.size() * sizeof(WorkItem), hipMemcpyHostToDevice, s));
@@ -1162,7 +1284,11 @@ void swap_built(kvexp_hip_plan &dst, kvexp_hip_plan &src) {
     swap(dst.jobs, src.jobs);
     swap(dst.esc_prefix, src.esc_prefix);
     swap(dst.esc_prefix_at, src.esc_prefix_at);
+    swap(dst.arena, src.arena);
+    swap(dst.arena_size, src.arena_size);
+    swap(dst.arena_used, src.arena_used);
     swap(dst.djobs, src.djobs);
+    swap(dst.jobs_uploaded, src.jobs_uploaded);
     swap(dst.wave, src.wave);
     swap(dst.heads, src.heads);
     swap(dst.items, src.items);
@@ -1277,18 +1403,30 @@ int kvexp_hip_plan_update(kvexp_hip_plan *plan, const kvexp_hip_head *heads, int
             // the device heads' lengths and byte counts and the last splits' ends
             // are set on the GPU from the jobs, with the last blocks' descriptors
             const int per_head = (plan->n_q + kMaxQPerLaunch - 1) / kMaxQPerLaunch;
+            kvexp_dev::PlanLens lens;
+            // lengths as a kernel argument while nothing else of the job table
+            // changes (a decode loop's steps give the buffers' capacities)
+            lens.n = n_heads <= kvexp_dev::kPlanLens && plan->jobs_uploaded ? n_heads : 0;
             for (int h = 0; h < n_heads; ++h)
                 for (int kv = 0; kv < 2; ++kv) {
                     kvexp_dev::EscJob &j = plan->jobs[size_t(2 * h + kv)];
-                    j.bytes = kv ? heads[h].v_bytes : heads[h].k_bytes;
+                    const uint64_t bytes = kv ? heads[h].v_bytes : heads[h].k_bytes;
+                    if (j.bytes != bytes) lens.n = 0;
+                    j.bytes = bytes;
                     j.seq = heads[h].seq;
                 }
-            HIPX(hipMemcpyAsync(plan->djobs.p, plan->jobs.data(), plan->jobs.size() * sizeof(kvexp_dev::EscJob),
-                                hipMemcpyHostToDevice, s));
+            if (lens.n > 0) {
+                for (int h = 0; h < n_heads; ++h) lens.seq[h] = heads[h].seq;
+            } else {
+                plan->jobs_uploaded = false;
+                HIPX(hipMemcpyAsync(plan->djobs.p, plan->jobs.data(), plan->jobs.size() * sizeof(kvexp_dev::EscJob),
+                                    hipMemcpyHostToDevice, s));
+                plan->jobs_uploaded = true;
+            }
             HIPX(kvexp_launch::plan_refresh(plan->djobs.as<kvexp_dev::EscJob>(),
                                             plan->xkv ? int(plan->jobs.size()) : 0, plan->heads.as<HeadDev>(),
                                             plan->n_dev_heads, plan->items.as<WorkItem>(), plan->n_items, per_head,
-                                            plan->status.as<uint32_t>(), s));
+                                            plan->status.as<uint32_t>(), lens, s));
             plan->src.assign(heads, heads + n_heads);
             plan->invalid = false;
             plan->invalid_msg.clear();
@@ -1362,7 +1500,7 @@ int kvexp_hip_attention_run(kvexp_hip_plan *plan, const uint16_t *d_q, float *d_
                                          plan->status.as<uint32_t>(), s));
             if (ev1) HIPX(hipEventRecord(ev1, s));
         }
-        if (check) check_status_word(plan->status.as<uint32_t>(), s);
+        if (check) check_status_word(plan->ctx, plan->status.as<uint32_t>(), s);
     });
 }
 
@@ -1396,7 +1534,7 @@ int kvexp_hip_plan_status(kvexp_hip_plan *plan, void *stream) {
     return guarded([&] {
         if (plan == nullptr) fail(KVEXP_HIP_INVALID_ARGUMENT, "kvexp_hip_plan_status: null plan");
         DeviceGuard g(plan->ctx->device);
-        check_status_word(plan->status.as<uint32_t>(), static_cast<hipStream_t>(stream));
+        check_status_word(plan->ctx, plan->status.as<uint32_t>(), static_cast<hipStream_t>(stream));
     });
 }
 

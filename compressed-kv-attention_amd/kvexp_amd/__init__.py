@@ -462,6 +462,7 @@ def _head_dtype():
 class Plan:
     def __init__(self, ctx: Context, h, n_heads: int, n_q: int, dim: int, keep):
         self.ctx, self.h, self.n_heads, self.n_q, self.dim, self._keep = ctx, h, n_heads, n_q, dim, keep
+        self._table = None
 
     def update(self, heads: list, stream=None) -> None:
         """kvexp_hip_plan_update: the plan's heads (same dicts as for Context.plan)
@@ -479,14 +480,18 @@ class Plan:
         import numpy as np
 
         n = self.n_heads
-        v = np.frombuffer(self._arr, dtype=_head_dtype(), count=n)
-        seqs = np.full(n, int(seq), np.int64) if np.isscalar(seq) else np.asarray(seq, np.int64)
-        nb = (seqs + block - 1) // block
-        v["seq"] = seqs
-        if self._caps and self._caps[0][0]:
+        if self._table is None or self._table[0] is not self._arr:  # the head table as numpy fields, made once
+            v = np.frombuffer(self._arr, dtype=_head_dtype(), count=n)
             caps = np.asarray(self._caps, dtype=np.uint64)
-            v["k_bytes"], v["v_bytes"] = caps[:, 0], caps[:, 1]
-            v["k_n_blocks"], v["v_n_blocks"] = nb, nb
+            self._table = (self._arr, v["seq"], v["k_n_blocks"], v["v_n_blocks"], v["k_bytes"], v["v_bytes"],
+                           caps[:, 0], caps[:, 1], bool(self._caps and self._caps[0][0]))
+        _, v_seq, v_knb, v_vnb, v_kb, v_vb, k_cap, v_cap, xkv = self._table
+        seqs = np.full(n, int(seq), np.int64) if np.isscalar(seq) else np.asarray(seq, np.int64)
+        v_seq[:] = seqs
+        if xkv:
+            nb = (seqs + block - 1) // block
+            v_kb[:], v_vb[:] = k_cap, v_cap
+            v_knb[:], v_vnb[:] = nb, nb
         check(lib().kvexp_hip_plan_update(self.h, self._arr, n, _stream(stream)))
 
     def update_heads(self, seqs, k_bytes=None, v_bytes=None, k_blocks=None, v_blocks=None, stream=None) -> None:

@@ -231,10 +231,7 @@ def decode_attention_kv(q: Tensor, kv: int, seqs: list[int]) -> Tensor:
         e["plan"] = ctx.plan(heads, n_q, dim, e["split"], e["order"], stream=stream)
         e["seqs"] = seqs
     elif seqs != e["seqs"]:
-        bt = e["split"]
-        nb = [(s + bt - 1) // bt for s in seqs]
-        neg = [-1] * n_heads
-        e["plan"].update_heads(seqs, neg, neg, nb, nb, stream=stream)
+        e["plan"].update_lengths(seqs, e["split"], stream=stream)
         e["seqs"] = seqs
     out = torch.empty((n_heads, n_q, dim), dtype=torch.float32, device=q.device)
     e["plan"].run(q.contiguous(), out, stream=stream)
