@@ -1432,24 +1432,38 @@ __global__ __launch_bounds__(kThreads) void append_one_kernel(const AppendJobDev
 // workgroup call it.
 // octets (total % 8 == 0, as head_dim is a multiple of 8): a segment of 16,384
 // codes at a time, all of its code words in flight together and one barrier
-// for the waves' counts, as in decode_coded (c2's plan update: 8.2 us per
-// launch with a scan and its two barriers every 1,024 codes).
+// for the waves' counts, as in decode_coded; a segment that is not full is
+// spread over all waves. The sentinels' element indexes go to LDS by rank and
+// the records are put together at the end, a record per thread with the words
+// read in order. Bound: the chain of dependent reads (job, index, header,
+// codes, words), about 1 us each. Storing every record where its sentinel is
+// found put a read of its word into the chain for each: a plan update of 96
+// tensors of head_dim 64 took 11.2 us (up to 13 as the last blocks fill), 6.7
+// so; the records of 65,536 blocks of head_dim 128 took 268 us, 240 so.
+// Ranks past the LDS window (8 KB; only blocks of more than 8,192 elements
+// can hold so many escapes) store theirs directly.
+constexpr int kRecWin = 4096;
 template <int MODE>
 __device__ __forceinline__ int escape_octets(const uint8_t *codes, int octets, int n_escape,
-                                             uint32_t *__restrict__ pos, int *tmp) {
+                                             uint32_t *__restrict__ pos, int *tmp, uint16_t *at) {
     constexpr uint32_t sentinel = (1u << MODE) - 1u;
     const uint8_t *words = codes + MODE * size_t(octets);
     const int lane = lane_id(), w = int(threadIdx.x) >> 6;
+    auto word = [&](int r) { return uint32_t(*reinterpret_cast<const dec_u16 *>(words + 2 * size_t(r))) << 16; };
+    // the thread's first word arrives with the codes
+    const uint32_t word0 = int(threadIdx.x) < n_escape ? word(int(threadIdx.x)) : 0u;
     int carry = 0;
     for (int seg = 0; seg < octets; seg += kDecSegment / 8) {
-        const int o0 = seg + w * (kDecSteps * kWave) + lane;
+        const int per_wave = (min(octets - seg, kDecSegment / 8) + kThreads - 1) / kThreads * kWave;
+        const int o0 = seg + w * per_wave + lane;
+        const int o1 = min(octets, seg + (w + 1) * per_wave);
         uint32_t cw[kDecSteps];
         int cnt[kDecSteps], mine = 0;
 #pragma unroll
         for (int k = 0; k < kDecSteps; ++k) cw[k] = dec_codes<MODE>(codes, min(o0 + kWave * k, octets - 1));
 #pragma unroll
         for (int k = 0; k < kDecSteps; ++k) {
-            cnt[k] = o0 + kWave * k < octets ? unit_sentinels(cw[k], MODE) : 0;
+            cnt[k] = o0 + kWave * k < o1 ? unit_sentinels(cw[k], MODE) : 0;
             mine += cnt[k];
         }
         const int sum = wave_sum_i32(mine);
@@ -1472,24 +1486,29 @@ __device__ __forceinline__ int escape_octets(const uint8_t *codes, int octets, i
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 if (((cw[k] >> (MODE * i)) & sentinel) != sentinel) continue;
-                if (r < n_escape)
-                    pos[r] = uint32_t(8 * (o0 + kWave * k) + i) |
-                             (uint32_t(*reinterpret_cast<const dec_u16 *>(words + 2 * size_t(r))) << 16);
+                const uint32_t e = uint32_t(8 * (o0 + kWave * k) + i);
+                if (r < kRecWin) at[r] = uint16_t(e);
+                else if (r < n_escape) pos[r] = e | word(r);
                 ++r;
             }
         }
     }
+    __syncthreads();
+    const int n = min(min(carry, n_escape), kRecWin);
+    for (int r = int(threadIdx.x); r < n; r += kThreads)
+        pos[r] = uint32_t(at[r]) | (r < kThreads ? word0 : word(r));
     return carry;
 }
 
 __device__ __forceinline__ void escape_positions(const uint8_t *codes, int mode, int total, int n_escape,
                                                  uint32_t *__restrict__ pos, int *scan_tmp,
                                                  uint32_t *__restrict__ status) {
+    __shared__ uint16_t at[kRecWin];
     int carry = 0;
     if (total % 8 == 0) {
-        carry = mode == 4   ? escape_octets<4>(codes, total / 8, n_escape, pos, scan_tmp)
-                : mode == 2 ? escape_octets<2>(codes, total / 8, n_escape, pos, scan_tmp)
-                            : escape_octets<3>(codes, total / 8, n_escape, pos, scan_tmp);
+        carry = mode == 4   ? escape_octets<4>(codes, total / 8, n_escape, pos, scan_tmp, at)
+                : mode == 2 ? escape_octets<2>(codes, total / 8, n_escape, pos, scan_tmp, at)
+                            : escape_octets<3>(codes, total / 8, n_escape, pos, scan_tmp, at);
     } else { // 2- and 4-bit codes, four elements per thread and step
         const uint8_t *words = codes + (total * mode + 7) / 8;
         const uint32_t sentinel = (1u << mode) - 1u;
@@ -1624,7 +1643,6 @@ __global__ __launch_bounds__(kThreads) void plan_refresh_kernel(const EscJob *__
                                                                int per_head, uint32_t *__restrict__ status,
                                                                PlanLens lens) {
     __shared__ int scan_tmp[kWaves];
-    __shared__ int ok_s;
     auto seq_of = [&](int h) { return lens.n > 0 ? lens.seq[h] : jobs[2 * h].seq; };
     if (int(blockIdx.x) >= n_jobs) {
         const int i = (int(blockIdx.x) - n_jobs) * kThreads + int(threadIdx.x);
@@ -1646,12 +1664,13 @@ __global__ __launch_bounds__(kThreads) void plan_refresh_kernel(const EscJob *__
     const int dim = j.dim;
     const int64_t off = j.offs[b];
     const int e0 = j.esc0[b];
+    // every thread checks the header for itself: no barrier, one read of it
+    BlockHdr h{};
+    uint32_t st = check_block(j.blob, j.bytes, off, dim, j.first[b + 1] - j.first[b], &h);
+    const int ne = st != 0u || h.mode == 0 ? 0 : h.n_escape;
+    if (st == 0u && e0 + ne > j.pos_cap) st = kStEscape;
+    if (j.first[j.n_blocks] < seq_of(int(blockIdx.x) / 2)) st |= kStIndex;
     if (threadIdx.x == 0) {
-        BlockHdr h{};
-        uint32_t st = check_block(j.blob, j.bytes, off, dim, j.first[b + 1] - j.first[b], &h);
-        const int ne = st != 0u || h.mode == 0 ? 0 : h.n_escape;
-        if (st == 0u && e0 + ne > j.pos_cap) st = kStEscape;
-        if (j.first[j.n_blocks] < seq_of(int(blockIdx.x) / 2)) st |= kStIndex;
         BlockDesc d{};
         d.data = j.blob + off;
         d.esc = j.pos + e0;
@@ -1663,11 +1682,8 @@ __global__ __launch_bounds__(kThreads) void plan_refresh_kernel(const EscJob *__
         j.desc[b + 1] = z;
         j.esc0[b + 1] = e0 + ne;
         if (st != 0u) atomicOr(status, st);
-        ok_s = st == 0u && ne > 0;
     }
-    __syncthreads();
-    if (!ok_s) return;
-    const BlockHdr h = read_hdr(j.blob + off);
+    if (st != 0u || ne == 0) return;
     const uint8_t *codes = j.blob + off + 8 + dim + size_t(h.n_tokens) * size_t(dim);
     escape_positions(codes, h.mode, h.n_tokens * dim, h.n_escape, j.pos + e0, scan_tmp, status);
 }
