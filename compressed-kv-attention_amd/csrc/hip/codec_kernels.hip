@@ -844,7 +844,10 @@ __device__ __forceinline__ EscRanks<NL> fused_escape_ranks(const uint32_t (&v)[E
 
 // Workgroups have TH threads: 256 for blocks of up to 16,384 elements, 512 and
 // 1,024 above (a CU's LDS then holds two blocks, or one, and the threads keep
-// four waves per SIMD).
+// four waves per SIMD). Twice the threads with four chunk rows each (512 and
+// 1,024 for blocks of 8,193 to 32,768 elements) are slower: what a thread does
+// once per block outweighs the waves gained (prefill of 48 x 16,384 tokens of
+// head_dim 128: 129 -> 180 us, 32 x 8,150 of 256: 96 -> 122 us).
 // Waves per SIMD the one-pass encoder is compiled for (its registers fit
 // 512 / waves without spilling): 8 with up to four chunk rows per thread.
 template <int NL>

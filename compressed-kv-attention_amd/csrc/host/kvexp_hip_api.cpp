@@ -957,9 +957,9 @@ int kvexp_hip_suggest_splits(kvexp_hip_ctx *ctx, int n_heads, int seq, int split
 
 namespace {
 
-// One round of the split kernel's resident waves: three single-wave splits
-// per SIMD at head_dim 64 (two for 8 query rows, and for the AVX-512 order
-// with 6 or more), two at head_dim 128. The uniform count is the largest one
+// One round of the split kernel's resident splits: three single waves per
+// SIMD at head_dim 64 (two for 8 query rows), two two-wave teams at 128, one
+// four-wave team at 256 (per SIMD, four waves either way). The uniform count is the largest one
 // whose longest split is no longer than the mean split of one round
 // (total tokens / resident waves): for equal lengths that is one full round,
 // with no second, partly filled one; for ragged lengths the long heads are
@@ -970,7 +970,7 @@ int suggest_core(const kvexp_hip_ctx *ctx, int64_t total_tokens, int max_seq, in
     if (ctx == nullptr || total_tokens <= 0 || max_seq <= 0 || split_tokens <= 0) return 1;
     const int tiles = (max_seq + split_tokens - 1) / split_tokens;
     const int g = std::min(std::max(1, n_q), kMaxQPerLaunch);
-    const int per_simd = dim == 256 ? 1 : (dim == 64 && g < 8 ? 3 : 2); // the wave kernel's occupancy (kWaveOcc)
+    const int per_simd = dim == 256 ? 1 : (dim == 64 && g < 8 ? 3 : 2); // splits resident per SIMD
     (void)order;
     const int64_t groups = (std::max(1, n_q) + kMaxQPerLaunch - 1) / kMaxQPerLaunch; // device heads per head
     const int64_t slots = int64_t(4) * per_simd * std::max(1, ctx->cu_count);
