@@ -1221,8 +1221,11 @@ void attn_wave_kernel(const HeadDev *__restrict__ heads, const WorkItem *__restr
     // first quarter of its tokens, then 2, 1, 0): the waves that are behind
     // win the issue slots and all of a CU's waves finish at about the same
     // time. (Quarters of the launch's longest split instead: c3's shape in the
-    // AVX-512 order 307 against 301 us.)
-    const int quarter = (wi.tok_end - wi.tok_begin + 3) / 4;
+    // AVX-512 order 307 against 301 us.) A launch of one or two waves per
+    // workgroup has one wave per SIMD and stays at priority 0, where waves
+    // start: changing it took 0.09-0.15 us of a call (one head x 8,192 tokens
+    // 14.19 -> 14.04 us, 32 plain heads x 1,000 tokens 11.79 -> 11.72).
+    const int quarter = wpg <= 2 ? INT_MAX / 4 : (wi.tok_end - wi.tok_begin + 3) / 4;
     constexpr bool TR = KVEXP_TRACE_ON(XKV, ORDER);
     unsigned long long ph[12] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     const unsigned long long tw0 = TR ? __builtin_readcyclecounter() : 0ull;
@@ -1240,7 +1243,7 @@ void attn_wave_kernel(const HeadDev *__restrict__ heads, const WorkItem *__restr
     (void)stamp;
     (void)after;
 
-    int prio = -1;
+    int prio = 0;
     while (t < wi.tok_end) {
         const int ln = lane_here(); // this chunk's lane index (see lane_here)
         {
@@ -1578,7 +1581,7 @@ __global__ __launch_bounds__(kMergeWaves * 64) void wave_merge_kernel(
     const int w = int(threadIdx.x) >> 6;
     const int mi = __builtin_amdgcn_readfirstlane(int(blockIdx.x) * kMergeWaves + w);
     if (mi >= n_mitems) return;
-    const int ch = 64 * int(blockIdx.y) + lane;   // the lane's channel
+    const int ch = D > 64 ? 64 * int(blockIdx.y) + lane : lane; // the lane's channel
     const int cl = D % 64 == 0 ? ch : min(ch, D - 1);
     // uni.g > 0: item i is (uni.ws_base + k uni.n_splits, uni.n_splits,
     // uni.q_row + k uni.g, i - k uni.g) with k = i / uni.g, so the slots'
