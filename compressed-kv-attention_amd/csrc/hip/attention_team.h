@@ -513,6 +513,9 @@ __device__ __forceinline__ void team_scores_dp(const uint8_t *row, int w, const 
                         ch[rg][J] = mfma_rank1<(i0 + e) % 16>(qa[rg][(i0 + e) / 16], k, ch[rg][J]);
                 });
             });
+            // octet by octet (all octets read ahead spilled above four rows)
+            __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 8 * NG, 0);
         });
 #pragma unroll
         for (int rg = 0; rg < NG; ++rg) {
@@ -586,6 +589,9 @@ __device__ __forceinline__ void team_fold_token(const TeamLds<G, D> &S, lds_f32 
     const float v = quad_f32<T % 4>(in.vq[Q % 3]);
     if constexpr (MOVE) {
         if ((am[T / 32] & (1u << (T % 32))) != 0) {
+            // (the empty asm keeps this a branch: at two rows the compiler read
+            // and selected the alphas of all 64 tokens instead, and spilled)
+            if constexpr (G == 2) asm volatile("");
             float av[G];
 #pragma unroll
             for (int g = 0; g < G; ++g) av[g] = S.aT[g][T];
@@ -622,6 +628,8 @@ __device__ __forceinline__ void team_fold(const TeamLds<G, D> &S, lds_f32 *eb, l
         } else {
             static_for<0, GS>([&](auto K) {
                 team_fold_token<G, D, T + decltype(K)::value, true, L>(S, eb, ab, trb, am, ea, in, a4, acc, lvec);
+                // (two rows: quad by quad, or registers of the rows in flight are moved and spilled)
+                if constexpr (G == 2 && decltype(K)::value % 4 == 3) asm volatile("" : "+v"(acc[0]));
             });
         }
         team_fold<G, D, T + GS, L>(S, eb, ab, trb, am, ea, in, acc, lvec);
@@ -670,7 +678,12 @@ template <bool XKV, int D> struct TRegsOf { typedef TRows<D> T; };
 template <int D> struct TRegsOf<false, D> { typedef uint4 T[kTeamRawRegs<D>]; };
 
 // Four waves per SIMD (128 registers); three (168) at more than four query
-// rows, whose second row group would spill.
+// rows, whose second row group would spill 14 to 84 registers at four (64
+// plain heads x 24,000 tokens of head_dim 128, five rows: 171 -> 207 us). A
+// spill or a move of a register that a row in flight is loaded into waits for
+// the load, which cost two rows at head_dim 128 a quarter of the call (plain
+// 186 -> 146 us, AVX-512 XKV 171 -> 129 without them). Left: two registers at
+// four plain rows of head_dim 256.
 template <int G>
 constexpr int kTeamOcc = G > 4 ? 3 : 4;
 
