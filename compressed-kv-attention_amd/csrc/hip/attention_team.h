@@ -7,7 +7,8 @@
 // a chunk's rows, every row group's accumulators of every channel and a tile
 // of 64 whole rows in one wave, which at these sizes leaves one or two waves
 // per SIMD. Here W waves (2 up to head_dim 128, 4 above) share the chunk's
-// tile and split its work, so that four waves fit a SIMD at every size:
+// tile and split its work, so that three or four waves fit a SIMD at every size
+// (kTeamOcc):
 //   1. wave w decodes rows [64 w / W, 64 (w + 1) / W) of the chunk's K rows
 //      from registers into the tile and writes the escapes of its rows over
 //      them, then requests its rows of the next chunk's K;
@@ -679,16 +680,17 @@ template <int D> struct TRegsOf<false, D> { typedef uint4 T[kTeamRawRegs<D>]; };
 
 // Four waves per SIMD (128 registers); three (168) at more than four query
 // rows, whose second row group would spill 14 to 84 registers at four (64
-// plain heads x 24,000 tokens of head_dim 128, five rows: 171 -> 207 us). A
-// spill or a move of a register that a row in flight is loaded into waits for
-// the load, which cost two rows at head_dim 128 a quarter of the call (plain
-// 186 -> 146 us, AVX-512 XKV 171 -> 129 without them). Left: two registers at
-// four plain rows of head_dim 256.
-template <int G>
-constexpr int kTeamOcc = G > 4 ? 3 : 4;
+// plain heads x 24,000 tokens of head_dim 128, five rows: 171 -> 207 us),
+// except at the sizes whose rows take three registers per stream and wave
+// instead of four (80 and 160). A spill or a move of a register that a row in
+// flight is loaded into waits for the load, which cost two rows at head_dim
+// 128 a quarter of the call (plain 186 -> 146 us, AVX-512 XKV 171 -> 131
+// without them). Left: two registers at four plain rows of head_dim 256.
+template <int G, int D>
+constexpr int kTeamOcc = G > 4 && TShape<D>::NR > 3 ? 3 : 4;
 
 template <int G, int D, bool XKV, int ORDER>
-__global__ __launch_bounds__(TShape<D>::W * 64) __attribute__((amdgpu_waves_per_eu(kTeamOcc<G>)))
+__global__ __launch_bounds__(TShape<D>::W * 64) __attribute__((amdgpu_waves_per_eu(kTeamOcc<G, D>)))
 void attn_team_kernel(const HeadDev *__restrict__ heads, const WorkItem *__restrict__ items,
                       const BlockDesc *__restrict__ desc, const uint16_t *__restrict__ q_all,
                       float *__restrict__ out_all, float *__restrict__ lse_all, float *__restrict__ ws) {

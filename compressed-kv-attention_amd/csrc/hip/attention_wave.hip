@@ -1,7 +1,7 @@
 // Entry points of the one-wave split kernel (attention_wave.h) and its
 // merges; the split kernels themselves are instantiated per head_dim and
 // score order in attention_wave_d<D>_o<O>.hip.
-#include "attention_wave.h"
+#include "attention_team.h"
 
 namespace kvexp_launch {
 using namespace kvexp_dev;
@@ -40,6 +40,28 @@ bool wave_supports(int dim) {
         return true;
     default: return false;
     }
+}
+
+// Splits of G query rows that stay resident on a CU: at head_dim 32 and 64 the
+// one-wave kernel's waves (four per SIMD, and three, or two at eight rows,
+// whose LDS leaves room for two workgroups), else the team kernel's teams; the
+// general kernel of the other sizes counts as two four-wave workgroups of four
+// splits each. `ragged`: teams count as four waves per SIMD at any G, since
+// the splits of a ragged batch come in several lengths and the short ones fill
+// in behind the long (four sequences of up to 25,003 tokens x 8 heads, eight
+// rows of head_dim 256: cut for 1,024 teams 90.1 us, for the 768 that fit 93.7;
+// other batches 130.6 and 143.0, 122.4 and 117.8).
+int resident_splits(int dim, int G, bool ragged) {
+#define KVEXP_RESIDENT_CASE(D)                                                                                       \
+    case D: return (G > 4 && !ragged ? team::kTeamOcc<8, D> : team::kTeamOcc<4, D>) * 4 / team::TShape<D>::W;
+    switch (dim) {
+    case 32: return 16;
+    case 64: return G < 8 ? 12 : 8;
+        KVEXP_TEAM_DIMS_32(KVEXP_RESIDENT_CASE)
+        KVEXP_TEAM_DIMS_16(KVEXP_RESIDENT_CASE)
+    default: return 8;
+    }
+#undef KVEXP_RESIDENT_CASE
 }
 
 // Work items per workgroup of the split kernel: consecutive ones share a

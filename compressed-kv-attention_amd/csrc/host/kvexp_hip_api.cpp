@@ -47,6 +47,7 @@ hipError_t plan_refresh(const kvexp_dev::EscJob *jobs, int n_jobs, HeadDev *head
 hipError_t result(const int64_t *value, const uint32_t *status, int64_t *host, hipStream_t s);
 hipError_t gather_first(const kvexp_dev::FirstJob *jobs, int n_jobs, int32_t *out, hipStream_t s);
 bool wave_supports(int dim);
+int resident_splits(int dim, int G, bool ragged);
 hipError_t attention_wave(bool xkv, int order, int G, int dim, const HeadDev *heads, const WorkItem *items,
                           int n_items, int wpg, const kvexp_dev::BlockDesc *desc, const uint16_t *q, float *out,
                           float *lse, float *ws, hipStream_t s);
@@ -957,23 +958,24 @@ int kvexp_hip_suggest_splits(kvexp_hip_ctx *ctx, int n_heads, int seq, int split
 
 namespace {
 
-// One round of the split kernel's resident splits: three single waves per
-// SIMD at head_dim 64 (two for 8 query rows), two two-wave teams at 128, one
-// four-wave team at 256 (per SIMD, four waves either way). The uniform count is the largest one
+// One round of the split kernel's resident splits (resident_splits of a CU,
+// for XKV heads in either score order). The uniform count is the largest one
 // whose longest split is no longer than the mean split of one round
-// (total tokens / resident waves): for equal lengths that is one full round,
+// (total tokens / resident splits): for equal lengths that is one full round,
 // with no second, partly filled one; for ragged lengths the long heads are
 // cut finer, and the shorter splits that come with it are dealt out by the
-// dispatcher as waves retire.
-int suggest_core(const kvexp_hip_ctx *ctx, int64_t total_tokens, int max_seq, int split_tokens, int dim, int n_q,
-                 int order) {
+// dispatcher as waves retire. What a wrong count costs (64 heads x 24,000
+// tokens): five rows of head_dim 128 cut for 2,048 teams where 1,536 fit
+// 177 -> 156 us, eight of 192 for 2,048 where 768 fit 296 -> 283, one of 32
+// for 2,048 waves where 4,096 fit 56 -> 45.
+int suggest_core(const kvexp_hip_ctx *ctx, int64_t total_tokens, int max_seq, bool ragged, int split_tokens, int dim,
+                 int n_q, int order) {
     if (ctx == nullptr || total_tokens <= 0 || max_seq <= 0 || split_tokens <= 0) return 1;
     const int tiles = (max_seq + split_tokens - 1) / split_tokens;
     const int g = std::min(std::max(1, n_q), kMaxQPerLaunch);
-    const int per_simd = dim == 256 ? 1 : (dim == 64 && g < 8 ? 3 : 2); // splits resident per SIMD
     (void)order;
     const int64_t groups = (std::max(1, n_q) + kMaxQPerLaunch - 1) / kMaxQPerLaunch; // device heads per head
-    const int64_t slots = int64_t(4) * per_simd * std::max(1, ctx->cu_count);
+    const int64_t slots = int64_t(kvexp_launch::resident_splits(dim, g, ragged)) * std::max(1, ctx->cu_count);
     const int64_t target = std::max<int64_t>(1, int64_t(max_seq) * slots / (total_tokens * groups));
     return int(std::max<int64_t>(1, std::min<int64_t>(tiles, target)));
 }
@@ -983,20 +985,21 @@ int suggest_core(const kvexp_hip_ctx *ctx, int64_t total_tokens, int max_seq, in
 int kvexp_hip_suggest_splits_for(kvexp_hip_ctx *ctx, int n_heads, int seq, int split_tokens, int dim, int n_q,
                                  int order) {
     if (n_heads <= 0 || seq <= 0) return 1;
-    return suggest_core(ctx, int64_t(n_heads) * seq, seq, split_tokens, dim, n_q, order);
+    return suggest_core(ctx, int64_t(n_heads) * seq, seq, false, split_tokens, dim, n_q, order);
 }
 
 int kvexp_hip_suggest_splits_batch(kvexp_hip_ctx *ctx, int n_heads, const int *seqs, int split_tokens, int dim,
                                    int n_q, int order) {
     if (n_heads <= 0 || seqs == nullptr) return 1;
-    int64_t total = 0;
+    int64_t total = 0, counted = 0;
     int max_seq = 0;
     for (int i = 0; i < n_heads; ++i) {
         if (seqs[i] <= 0) continue;
         total += seqs[i];
+        ++counted;
         max_seq = std::max(max_seq, seqs[i]);
     }
-    return suggest_core(ctx, total, max_seq, split_tokens, dim, n_q, order);
+    return suggest_core(ctx, total, max_seq, total != counted * max_seq, split_tokens, dim, n_q, order);
 }
 
 namespace {
