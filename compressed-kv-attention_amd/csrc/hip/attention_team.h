@@ -71,7 +71,7 @@ struct alignas(16) TeamLds {
     float eT[G][kRowPad]; // e of token t, row g (0 past the chunk's end)
     float aT[G][kRowPad]; // alpha of token t, row g (1 where no running maximum moves)
     uint64_t am[4];       // per wave: tokens that move a running maximum of its rows
-    uint32_t low[4];      // AVX-512 order, plain BF16 rows: whether the wave's rows need the flushing scores
+    uint32_t low[4];      // AVX-512 order, rows as they are (plain or a raw block): whether the wave's need the flushing scores
 };
 
 // Workgroup barrier for LDS traffic only: the global loads in flight stay in
@@ -805,7 +805,7 @@ void attn_team_kernel(const HeadDev *__restrict__ heads, const WorkItem *__restr
         const int tn = t + n, tp = min(tn, wi.tok_end - 1);
 
         // 1. the wave's K rows -> tile, the next ones requested
-        bool flush = false;
+        bool flush = false, checked = !XKV; // checked: S.low holds the waves' answers for the chunk's rows
         if constexpr (XKV) after(RK.c[SH::NR - 1].y);
         stamp(0); // K rows arrived
         if constexpr (XKV) {
@@ -817,8 +817,17 @@ void attn_team_kernel(const HeadDev *__restrict__ heads, const WorkItem *__restr
                     const u16x2 bmin = __builtin_elementwise_min(e, o), bmax = __builtin_elementwise_max(e, o);
                     const uint32_t top = 256u - (1u << kc.mode());
                     flush = __ballot(uint32_t(min(bmin.x, bmin.y)) < kmin || uint32_t(max(bmax.x, bmax.y)) > top) != 0;
-                } else {
-                    flush = true;
+                } else { // the wave's rows < n of a raw block (decode_team_rows)
+                    constexpr int RW = SH::RawRows / W;
+                    low_min_t lo = kLowMinNone;
+#pragma unroll
+                    for (int k = 0; k < SH::NR; ++k) {
+                        const int r = (64 * k + ln) / (D / 8);
+                        if (r < RW && RW * w + r < n) lo = low_min(lo, RK.s[k]);
+                    }
+                    const bool low = any_low(lo, klow);
+                    if (ln == 0) S.low[w] = low ? 1u : 0u;
+                    checked = true;
                 }
             }
             decode_team_rows<D, KP, false>(kc, RK, S.tile, w, n);
@@ -830,18 +839,13 @@ void attn_team_kernel(const HeadDev *__restrict__ heads, const WorkItem *__restr
             load_team_rows<D>(kc, w, tp - kc.t0, min(kChunk, min(kc.t1, wi.tok_end) - tp), RK);
         } else {
             if constexpr (ORDER == 1) {
-                u16x2 lo = {0xFFFFu, 0xFFFFu};
+                low_min_t lo = kLowMinNone;
 #pragma unroll
                 for (int j = 0; j < kTeamRawRegs<D>; ++j) {
                     const int r = (64 * j + ln) / (D / 8);
-                    if (r >= SH::RO || SH::RO * w + r >= n) continue;
-                    const uint32_t c4[4] = {RK[j].x, RK[j].y, RK[j].z, RK[j].w};
-#pragma unroll
-                    for (int k = 0; k < 4; ++k)
-                        lo = __builtin_elementwise_min(lo, (__builtin_bit_cast(u16x2, c4[k]) & uint16_t(0x7FFF)) -
-                                                               uint16_t(1));
+                    if (r < SH::RO && SH::RO * w + r < n) lo = low_min(lo, RK[j]);
                 }
-                const bool low = __ballot(uint32_t(min(lo.x, lo.y)) < klow) != 0;
+                const bool low = any_low(lo, klow);
                 if (ln == 0) S.low[w] = low ? 1u : 0u;
             }
             store_team_raw<D, KP>(RK, S.tile, w);
@@ -858,7 +862,7 @@ void attn_team_kernel(const HeadDev *__restrict__ heads, const WorkItem *__restr
             if constexpr (ORDER == 0) {
                 team_scores<G, D>(row + 2 * CW * w, qa, p);
             } else {
-                if constexpr (!XKV) {
+                if (checked) {
                     uint32_t any = 0;
 #pragma unroll
                     for (int i = 0; i < W; ++i) any |= S.low[i];

@@ -637,12 +637,30 @@ __device__ __forceinline__ void decode_rows(const Cursor &c, Rows<D> &R, const u
 // biased exponents E_k + E_q >= 142 for every nonzero K element and query
 // element of the head (denormal queries read as zero beforehand), no input,
 // chain value or sum is denormal, and the flushes are the identity. A chunk
-// with a smaller K exponent (or a raw block, which is not checked element by
-// element) takes the vector path that applies the flushes.
+// with a smaller K exponent takes the vector path that applies the flushes. A
+// raw block's rows are checked element by element in the registers that hold
+// them (8 heads x 4,100 tokens of raw blocks, eight rows of head_dim 96: 152 us
+// with every such chunk flushing, 51 so; 32: 104 and 36), except at head_dim
+// 64, where every chunk of one takes the flushing path.
 
 // Whether BF16 x is nonzero with exponent field below T, for
 // low = (T << 7) - 1 (T >= 1): (x & 0x7FFF) - 1 wraps to 2^32 - 1 for a zero.
 __device__ __forceinline__ bool low_bf16(uint32_t x, uint32_t low) { return (x & 0x7FFFu) - 1u < low; }
+
+// low_bf16 of the BF16 of a register, two at a time: the smallest (x & 0x7FFF)
+// - 1 of a lane's elements (16 bits each), compared with `low` once.
+typedef uint16_t low_min_t __attribute__((ext_vector_type(2)));
+constexpr low_min_t kLowMinNone = {0xFFFFu, 0xFFFFu};
+__device__ __forceinline__ low_min_t low_min(low_min_t lo, uint32_t pair) {
+    return __builtin_elementwise_min(lo, (__builtin_bit_cast(low_min_t, pair) & uint16_t(0x7FFF)) - uint16_t(1));
+}
+__device__ __forceinline__ low_min_t low_min(low_min_t lo, const uint4 &v) {
+    return low_min(low_min(low_min(low_min(lo, v.x), v.y), v.z), v.w);
+}
+// Whether any lane of the wave holds an element below the bound.
+__device__ __forceinline__ bool any_low(low_min_t lo, uint32_t low) {
+    return __ballot(uint32_t(min(lo.x, lo.y)) < low) != 0;
+}
 
 // Denormal to signed zero (VDPBF16PS's DAZ on inputs and FTZ on results).
 __device__ __forceinline__ float flush_tiny(float x) {
@@ -1290,8 +1308,19 @@ void attn_wave_kernel(const HeadDev *__restrict__ heads, const WorkItem *__restr
                     base_pairs<D>(kc, S.bp);
                     wave_sync();
                 }
-            } else {
-                flush = ORDER == 1;
+            } else if constexpr (ORDER == 1) {
+                if constexpr (kWholeRows<D>) {
+                    flush = true;
+                } else { // the loaded pieces of rows < n (decode_pieces; each lies in one row)
+                    low_min_t lo = kLowMinNone;
+#pragma unroll
+                    for (int k = 0; k < Shape<D>::kPieceRegs; ++k) {
+                        const int os = 1024 * k + 16 * ln, oc = 1024 * Shape<D>::kPieceRegs + 512 * k + 8 * ln;
+                        if (os < 2 * D * n) lo = low_min(lo, RK.s[k]);
+                        if (oc < 2 * D * n) lo = low_min(low_min(lo, RK.c[k].x), RK.c[k].y);
+                    }
+                    flush = any_low(lo, klow);
+                }
             }
             // whole rows: a 4- or 2-bit chunk without escapes (and, in the
             // AVX-512 order, without a possible flush) is decoded octet by
@@ -1307,17 +1336,11 @@ void attn_wave_kernel(const HeadDev *__restrict__ heads, const WorkItem *__restr
             store_raw<D>(RK, S.tile);
             if constexpr (ORDER == 1) {
                 // any element of the chunk's rows (pieces of rows < n) below the bound
-                u16x2 lo = {0xFFFFu, 0xFFFFu};
+                low_min_t lo = kLowMinNone;
 #pragma unroll
-                for (int j = 0; j < D / 8; ++j) {
-                    if ((1024 * j + 16 * ln) / (2 * D) >= n) continue;
-                    const uint32_t c4[4] = {RK[j].x, RK[j].y, RK[j].z, RK[j].w};
-#pragma unroll
-                    for (int k = 0; k < 4; ++k)
-                        lo = __builtin_elementwise_min(lo, (__builtin_bit_cast(u16x2, c4[k]) & uint16_t(0x7FFF)) -
-                                                               uint16_t(1));
-                }
-                flush = __ballot(uint32_t(min(lo.x, lo.y)) < klow) != 0;
+                for (int j = 0; j < D / 8; ++j)
+                    if ((1024 * j + 16 * ln) / (2 * D) < n) lo = low_min(lo, RK[j]);
+                flush = any_low(lo, klow);
             }
         }
         wave_sync();
