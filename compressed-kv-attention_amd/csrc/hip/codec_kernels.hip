@@ -46,6 +46,10 @@ __device__ __forceinline__ bool decode_covers(const int32_t *first, int n_blocks
 // streaming copy (1.5 bytes in, 2 out per element), so the aim is bytes in
 // flight and whole-line accesses; two barriers and a scan per 1,024 elements,
 // with byte loads, took 66 us for one head_dim-128 tensor of 131,072 tokens.
+// Blocks of up to 8,192 elements take shorter segments (4, 2 or 1 octets per
+// lane), which spread them over all four waves and leave no step that only
+// repeats the last octet: 40,000 tokens of head_dim 16 in 16-token blocks took
+// 18.9 us at eight steps each, 10.5 so.
 constexpr int kDecSteps = 8;                              // octets per lane per segment
 constexpr int kDecSegment = 8 * kDecSteps * kThreads;     // elements
 
@@ -72,10 +76,11 @@ __device__ __forceinline__ uint32_t dec_codes(const uint8_t *codes, int o) {
     return uint32_t(*reinterpret_cast<const dec_u16 *>(p)) | (uint32_t(p[2]) << 16);
 }
 
-// One coded block: `octets` of its octets (the rows asked for) to out; every
-// thread of the workgroup calls it. tmp: kWaves ints in LDS.
-template <int MODE>
-__device__ __forceinline__ uint32_t decode_coded(const uint8_t *p, const BlockHdr &h, int dim, int octets, uint16_t *out,
+// One coded block: `octets` of its octets (the rows asked for) to out, STEPS
+// per lane and segment; every thread of the workgroup calls it. tmp: kWaves
+// ints in LDS.
+template <int MODE, int STEPS>
+__device__ __forceinline__ uint32_t decode_steps(const uint8_t *p, const BlockHdr &h, int dim, int octets, uint16_t *out,
                                                  int *tmp) {
     constexpr uint32_t sentinel = (1u << MODE) - 1u;
     const uint8_t *sm = p + dim;
@@ -84,21 +89,21 @@ __device__ __forceinline__ uint32_t decode_coded(const uint8_t *p, const BlockHd
     const int lane = lane_id(), w = int(threadIdx.x) >> 6, cpr = dim / 8;
     uint32_t bad = 0;
     int carry = 0; // sentinels of earlier segments
-    for (int seg = 0; seg < octets; seg += kDecSegment / 8) {
-        const int o0 = seg + w * (kDecSteps * kWave) + lane; // the lane's first octet
-        uint32_t cw[kDecSteps];
-        uint2 s8[kDecSteps], b8[kDecSteps];
+    for (int seg = 0; seg < octets; seg += STEPS * kThreads) {
+        const int o0 = seg + w * (STEPS * kWave) + lane; // the lane's first octet
+        uint32_t cw[STEPS];
+        uint2 s8[STEPS], b8[STEPS];
         int col = o0 % cpr;
         const int step = kWave % cpr;
 #pragma unroll
-        for (int k = 0; k < kDecSteps; ++k) {
+        for (int k = 0; k < STEPS; ++k) {
             const int o = min(o0 + kWave * k, octets - 1);
             cw[k] = dec_codes<MODE>(codes, o);
             const dec_u32x2 x = *reinterpret_cast<const dec_u32x2 *>(sm + 8 * size_t(o));
             s8[k] = make_uint2(x.x, x.y);
         }
 #pragma unroll
-        for (int k = 0; k < kDecSteps; ++k) {
+        for (int k = 0; k < STEPS; ++k) {
             const dec_u32x2 x = *reinterpret_cast<const dec_u32x2 *>(p + 8 * col);
             b8[k] = make_uint2(x.x, x.y);
             col += step;
@@ -109,7 +114,7 @@ __device__ __forceinline__ uint32_t decode_coded(const uint8_t *p, const BlockHd
         if (h.n_escape > 0) {
             int mine = 0;
 #pragma unroll
-            for (int k = 0; k < kDecSteps; ++k)
+            for (int k = 0; k < STEPS; ++k)
                 mine += o0 + kWave * k < octets ? unit_sentinels(cw[k], MODE) : 0;
             const int total = wave_sum_i32(mine);
             __syncthreads(); // the last segment's totals are read
@@ -122,7 +127,7 @@ __device__ __forceinline__ uint32_t decode_coded(const uint8_t *p, const BlockHd
             }
         }
 #pragma unroll
-        for (int k = 0; k < kDecSteps; ++k) {
+        for (int k = 0; k < STEPS; ++k) {
             const int o = o0 + kWave * k;
             const bool in = o < octets;
             const uint32_t c = cw[k];
@@ -154,6 +159,15 @@ __device__ __forceinline__ uint32_t decode_coded(const uint8_t *p, const BlockHd
         }
     }
     return bad;
+}
+
+template <int MODE>
+__device__ __forceinline__ uint32_t decode_coded(const uint8_t *p, const BlockHdr &h, int dim, int octets, uint16_t *out,
+                                                 int *tmp) {
+    if (octets > 4 * kThreads) return decode_steps<MODE, kDecSteps>(p, h, dim, octets, out, tmp);
+    if (octets > 2 * kThreads) return decode_steps<MODE, 4>(p, h, dim, octets, out, tmp);
+    if (octets > kThreads) return decode_steps<MODE, 2>(p, h, dim, octets, out, tmp);
+    return decode_steps<MODE, 1>(p, h, dim, octets, out, tmp);
 }
 
 __global__ __launch_bounds__(kThreads) void decode_octets_kernel(const uint8_t *__restrict__ blob, uint64_t bytes,

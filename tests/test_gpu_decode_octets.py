@@ -38,6 +38,14 @@ def test_decode_octets_edges(ctx, oracle, dim, block):
                 assert bool((out[n * dim:] == 0x5A5A).all())  # nothing past the tokens asked for
 
 
+@pytest.mark.parametrize("dim,block", [(8, 16), (16, 16), (64, 16), (64, 32), (64, 33), (64, 64), (64, 65), (64, 129),
+                                       (72, 28), (72, 29), (72, 57), (72, 114)])
+def test_decode_octets_small_blocks(ctx, oracle, dim, block):
+    """Blocks at the edges of the shorter segments (256, 512 and 1,024 octets)
+    and of a wave and less."""
+    test_decode_octets_edges(ctx, oracle, dim, block)
+
+
 def test_checked_decode_refuses_a_short_index(ctx):
     """More tokens than the index covers: refused, and nothing is written."""
     import torch
