@@ -1560,11 +1560,19 @@ __device__ __forceinline__ void escape_positions(const uint8_t *codes, int mode,
 // workgroup per tensor. With j.first set, every block is also checked against
 // the index (header inside the container, head_dim, n_tokens equal to the
 // index's token count, known mode, payload inside the container); with
-// j.desc set (and j.pos allocated), its descriptor is written.
+// j.desc set (and j.pos allocated), its descriptor is written, and the entry
+// after the last one becomes a zero-token sentinel (a split kernel that reached
+// it would stop there). With j.first_out set, the index's first tokens go there
+// too, so that the host reads those of all tensors with one copy (c2's 96
+// tensors took 96 copies, about 0.9 ms of a plan's 1.25); with j.esc0 null only
+// these.
 __global__ __launch_bounds__(kThreads) void esc_start_kernel(const EscJob *__restrict__ jobs,
                                                             uint32_t *__restrict__ status) {
     __shared__ int scan_tmp[kWaves];
     const EscJob j = jobs[blockIdx.x];
+    if (j.first_out != nullptr)
+        for (int i = int(threadIdx.x); i <= j.n_blocks; i += kThreads) j.first_out[i] = j.first[i];
+    if (j.esc0 == nullptr) return;
     int carry = 0;
     for (int r = 0; r < j.n_blocks; r += kThreads) {
         const int b = r + int(threadIdx.x);
@@ -1598,16 +1606,15 @@ __global__ __launch_bounds__(kThreads) void esc_start_kernel(const EscJob *__res
         }
         carry += tot;
     }
-    if (threadIdx.x == 0) j.esc0[j.n_blocks] = carry;
-}
-
-// The block first tokens of every tensor of a plan, one after another in
-// `out` (one workgroup per tensor): the host then reads them with one copy
-// (c2's 96 tensors took 96 copies, about 0.9 ms of a plan's 1.25).
-__global__ __launch_bounds__(kThreads) void gather_first_kernel(const FirstJob *__restrict__ jobs,
-                                                               int32_t *__restrict__ out) {
-    const FirstJob j = jobs[blockIdx.x];
-    for (int i = int(threadIdx.x); i < j.n; i += kThreads) out[j.at + i] = j.first[i];
+    if (threadIdx.x == 0) {
+        j.esc0[j.n_blocks] = carry;
+        if (j.desc != nullptr) {
+            BlockDesc z{};
+            z.data = j.blob;
+            z.esc = j.pos;
+            j.desc[j.n_blocks] = z;
+        }
+    }
 }
 
 // A 64-bit word (nullable) and the status word to host memory that the GPU can
@@ -1865,12 +1872,6 @@ hipError_t plan_refresh(const EscJob *jobs, int n_jobs, HeadDev *heads, int n_de
 
 hipError_t result(const int64_t *value, const uint32_t *status, int64_t *host, hipStream_t s) {
     hipLaunchKernelGGL(result_kernel, dim3(1), dim3(1), 0, s, value, status, host);
-    return hipGetLastError();
-}
-
-hipError_t gather_first(const FirstJob *jobs, int n_jobs, int32_t *out, hipStream_t s) {
-    if (n_jobs <= 0) return hipSuccess;
-    hipLaunchKernelGGL(gather_first_kernel, dim3(n_jobs), dim3(kThreads), 0, s, jobs, out);
     return hipGetLastError();
 }
 

@@ -62,19 +62,14 @@ struct EscJob {
     uint64_t bytes;
     const int64_t *offs;
     const int32_t *first; // block first tokens (n_blocks + 1)
-    int32_t *esc0;        // out: n_blocks + 1 entries
+    int32_t *esc0;        // out: n_blocks + 1 entries (nullable: blocks not looked at)
+    int32_t *first_out;   // out: copy of `first` (nullable)
     uint32_t *pos;        // out: esc0[n_blocks] escape records
     BlockDesc *desc;      // out: n_blocks entries (nullable)
     int32_t n_blocks;
     int32_t dim;
     int32_t pos_cap;      // records of `pos` (the tensor's escapes plus room for its last block to grow)
-    int32_t seq;          // tokens a plan update attends (esc_tail_kernel checks the index covers them)
-};
-
-// One tensor's block first tokens for gather_first_kernel: n entries to out[at].
-struct FirstJob {
-    const int32_t *first;
-    int32_t n, at;
+    int32_t seq;          // tokens a plan update attends (plan_refresh_kernel checks the index covers them)
 };
 
 // Lengths of a plan's heads as a kernel argument (a plan update then uploads

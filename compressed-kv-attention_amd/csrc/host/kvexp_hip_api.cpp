@@ -45,7 +45,6 @@ hipError_t esc_pos(const kvexp_dev::EscJob *jobs, const int2 *blocks, int n_bloc
 hipError_t plan_refresh(const kvexp_dev::EscJob *jobs, int n_jobs, HeadDev *heads, int n_dev_heads, WorkItem *items,
                         int n_items, int per_head, uint32_t *status, const kvexp_dev::PlanLens &lens, hipStream_t s);
 hipError_t result(const int64_t *value, const uint32_t *status, int64_t *host, hipStream_t s);
-hipError_t gather_first(const kvexp_dev::FirstJob *jobs, int n_jobs, int32_t *out, hipStream_t s);
 bool wave_supports(int dim);
 int resident_splits(int dim, int G, bool ragged);
 hipError_t attention_wave(bool xkv, int order, int G, int dim, const HeadDev *heads, const WorkItem *items,
@@ -272,20 +271,19 @@ struct kvexp_hip_plan {
     // buffers from the context's pool (plans of the host-pointer entry, which
     // synchronises its stream before destroying them); others are freed
     bool pooled = false;
-    // The plan's device arrays lie in one allocation (plan_build sizes it before
-    // the first of them is taken; an allocation takes about 30 us, so eleven of
-    // them were a quarter of a rebuild), an array past its end in one of its own.
+    // The plan's device arrays are parts of one allocation, which plan_build
+    // sizes for all of them.
     static size_t padded(size_t n) { return (n + 255u) & ~size_t(255); }
     void reserve(size_t n) {
         arena = DevBuf(pooled ? &ctx->pool : nullptr, n);
         arena_size = n;
         arena_used = 0;
     }
-    DevBuf alloc(size_t n) {
-        if (arena_used + padded(n) > arena_size) return DevBuf(pooled ? &ctx->pool : nullptr, n);
-        void *at = arena.as<uint8_t>() + arena_used;
+    DevBuf part(size_t n) {
+        void *from = arena.as<uint8_t>() + arena_used;
         arena_used += padded(n);
-        return DevBuf::part_of(at);
+        if (arena_used > arena_size) fail(KVEXP_HIP_LOGIC_ERROR, "kvexp_hip_plan: arrays past their allocation");
+        return DevBuf::part_of(from);
     }
     int n_heads = 0, n_q = 0, dim = 0, order = 0, split_tokens = 0;
     // set when kvexp_hip_plan_update failed after the containers changed: the
@@ -460,95 +458,6 @@ void check_status_word(kvexp_hip_ctx *ctx, uint32_t *d_status, hipStream_t s) {
         fail(KVEXP_HIP_FORMAT_ERROR, status_message(st));
     }
 }
-// Block descriptors and escape records of every XKV tensor of a plan:
-// per block its address, first escape index and header fields (checked
-// against the block index; a mismatch fails the plan with the matching
-// format error), and per escape its element index inside the block. Built on
-// the device from the containers, once per plan; the device heads of one
-// user head share it.
-void build_escape_index(kvexp_hip_plan &p, const kvexp_hip_head *heads, int n_heads, int n_q, int dim,
-                        std::vector<HeadDev> &hv, hipStream_t s) {
-    std::vector<kvexp_dev::EscJob> jobs;
-    std::vector<size_t> e0_at;
-    size_t e0_total = 0;
-    for (int h = 0; h < n_heads; ++h) {
-        for (int kv = 0; kv < 2; ++kv) {
-            kvexp_dev::EscJob j{};
-            j.blob = kv ? heads[h].v_xkv : heads[h].k_xkv;
-            j.bytes = kv ? heads[h].v_bytes : heads[h].k_bytes;
-            j.offs = kv ? heads[h].v_offsets : heads[h].k_offsets;
-            j.first = kv ? heads[h].v_first_token : heads[h].k_first_token;
-            j.n_blocks = kv ? heads[h].v_n_blocks : heads[h].k_n_blocks;
-            j.dim = dim;
-            e0_at.push_back(e0_total);
-            e0_total += size_t(j.n_blocks) + 1;
-            jobs.push_back(j);
-        }
-    }
-    p.esc0 = p.alloc(e0_total * sizeof(int32_t));
-    p.desc = p.alloc(e0_total * sizeof(kvexp_dev::BlockDesc));
-    // HIP memory is not zeroed: the entry after each tensor's last block is
-    // the zero-token sentinel until a plan update writes it again
-    HIPX(hipMemsetAsync(p.desc.p, 0, e0_total * sizeof(kvexp_dev::BlockDesc), s));
-    for (size_t i = 0; i < jobs.size(); ++i) {
-        jobs[i].esc0 = p.esc0.as<int32_t>() + e0_at[i];
-        jobs[i].desc = p.desc.as<kvexp_dev::BlockDesc>() + e0_at[i];
-    }
-    DevBuf djobs = p.alloc(jobs.size() * sizeof(kvexp_dev::EscJob));
-    uint32_t *st = p.status.as<uint32_t>(); // the plan's own status word
-    // pass 1: block checks and escape counts (descriptors need the position array)
-    std::vector<kvexp_dev::EscJob> jobs1 = jobs;
-    for (auto &j : jobs1) j.desc = nullptr;
-    HIPX(hipMemcpyAsync(djobs.p, jobs1.data(), jobs1.size() * sizeof(kvexp_dev::EscJob), hipMemcpyHostToDevice, s));
-    HIPX(kvexp_launch::esc_start(djobs.as<kvexp_dev::EscJob>(), int(jobs.size()), st, s));
-    // the status word and the escape counts with one synchronisation
-    auto *host = static_cast<int32_t *>(pinned_staging(p.ctx, (e0_total + 1) * sizeof(int32_t)));
-    HIPX(hipMemcpyAsync(host, st, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-    HIPX(hipMemcpyAsync(host + 1, p.esc0.p, e0_total * sizeof(int32_t), hipMemcpyDeviceToHost, s));
-    HIPX(hipStreamSynchronize(s));
-    if (host[0] != 0) check_status_word(p.ctx, st, s); // clears the word and reports it
-    std::vector<int32_t> e0(host + 1, host + 1 + e0_total);
-    p.esc_prefix = e0;
-    p.esc_prefix_at = e0_at;
-    // each tensor's positions, then room for its last block to grow to the
-    // largest block the format allows (255 tokens) after appends
-    size_t pos_total = 0;
-    std::vector<size_t> pos_at;
-    std::vector<int2> blocks;
-    for (size_t i = 0; i < jobs.size(); ++i) {
-        pos_at.push_back(pos_total);
-        const size_t own = size_t(e0[e0_at[i] + size_t(jobs[i].n_blocks)]);
-        jobs[i].pos_cap = int32_t(own + size_t(255) * size_t(dim));
-        pos_total += size_t(jobs[i].pos_cap);
-        for (int b = 0; b < jobs[i].n_blocks; ++b) blocks.push_back(make_int2(int(i), b));
-    }
-    // escape records, then kEscPad spare ones: a kernel's window of records
-    // read from any escape stays inside the allocation (zeroed, never used)
-    p.escpos = p.alloc((pos_total + size_t(kvexp_dev::kEscPad)) * sizeof(uint32_t));
-    HIPX(hipMemsetAsync(p.escpos.as<uint32_t>() + pos_total, 0, size_t(kvexp_dev::kEscPad) * sizeof(uint32_t), s));
-    for (size_t i = 0; i < jobs.size(); ++i) jobs[i].pos = p.escpos.as<uint32_t>() + pos_at[i];
-    HIPX(hipMemcpyAsync(djobs.p, jobs.data(), jobs.size() * sizeof(kvexp_dev::EscJob), hipMemcpyHostToDevice, s));
-    // pass 2: descriptors (with the escape-record pointers)
-    HIPX(kvexp_launch::esc_start(djobs.as<kvexp_dev::EscJob>(), int(jobs.size()), st, s));
-    DevBuf dblocks = p.alloc(std::max<size_t>(blocks.size(), 1) * sizeof(int2));
-    HIPX(hipMemcpyAsync(dblocks.p, blocks.data(), blocks.size() * sizeof(int2), hipMemcpyHostToDevice, s));
-    HIPX(kvexp_launch::esc_pos(djobs.as<kvexp_dev::EscJob>(), dblocks.as<int2>(), int(blocks.size()), st, s));
-    check_status_word(p.ctx, st, s); // synchronises s: the host vectors above may go
-    p.jobs = jobs;
-    p.djobs = std::move(djobs);
-    p.jobs_uploaded = true;
-    const int per_head = (n_q + kMaxQPerLaunch - 1) / kMaxQPerLaunch;
-    for (int h = 0; h < n_heads; ++h) {
-        for (int c = 0; c < per_head; ++c) {
-            HeadDev &d = hv[size_t(h * per_head + c)];
-            d.kdesc = jobs[size_t(2 * h)].desc;
-            d.kesc = jobs[size_t(2 * h)].pos;
-            d.vdesc = jobs[size_t(2 * h + 1)].desc;
-            d.vesc = jobs[size_t(2 * h + 1)].pos;
-        }
-    }
-}
-
 } // namespace
 
 extern "C" {
@@ -1048,9 +957,13 @@ void balance_items(kvexp_hip_plan &p, std::vector<WorkItem> &items, bool xkv, co
         const int b = p.group_start[G], e = p.group_start[G + 1];
         const int n = e - b;
         if (n <= wpw || n % wpw != 0) continue; // whole workgroups only
-        std::vector<std::pair<double, int>> order(static_cast<size_t>(n));
-        for (int i = 0; i < n; ++i) order[size_t(i)] = {cost(items[size_t(b + i)]), i};
-        std::stable_sort(order.begin(), order.end(), [](const auto &x, const auto &y) { return x.first > y.first; });
+        // sorted as words, cost in 1/16 tokens above and place below
+        std::vector<uint64_t> order(static_cast<size_t>(n));
+        for (int i = 0; i < n; ++i) {
+            const double c = std::min(16.0 * std::max(0.0, cost(items[size_t(b + i)])), 4294967295.0);
+            order[size_t(i)] = (uint64_t(0xFFFFFFFFu - uint32_t(c)) << 32) | uint32_t(i);
+        }
+        std::sort(order.begin(), order.end());
         const int n_groups = (n + wpw - 1) / wpw;
         std::vector<int> slot_of_group(static_cast<size_t>(n_groups));
         for (int t0 = 0; t0 < n_groups; t0 += C) {
@@ -1063,7 +976,7 @@ void balance_items(kvexp_hip_plan &p, std::vector<WorkItem> &items, bool xkv, co
         for (int r = 0; r < n; ++r) {
             const int gq = r / wpw;
             const int slot = slot_of_group[size_t(gq)];
-            out[size_t(slot * wpw + fill[size_t(slot)]++)] = items[size_t(b + order[size_t(r)].second)];
+            out[size_t(slot * wpw + fill[size_t(slot)]++)] = items[size_t(b) + size_t(uint32_t(order[size_t(r)]))];
         }
         std::copy(out.begin(), out.end(), items.begin() + b);
     }
@@ -1071,60 +984,90 @@ void balance_items(kvexp_hip_plan &p, std::vector<WorkItem> &items, bool xkv, co
 
 // Builds every device-side part of a fresh plan from its heads: work items
 // (token_bounds splits, split starts checked against the block index), device
-// heads, merge work, and for the one-wave kernel the block descriptors and
-// escape records. Stream-ordered on `s`: it first waits for the work
-// already queued there (the encodes or appends that wrote the containers and
-// indexes it reads) and synchronises only `s`. Status words: the plan's own.
+// heads, merge work, and for the one-wave and team kernels the block
+// descriptors and escape records (per block its address, first escape index and
+// header fields, checked against the block index; per escape its element index
+// inside the block; the device heads of one user head share them).
+// Stream-ordered on `s`: it first waits for the work already queued there (the
+// encodes or appends that wrote the containers and indexes it reads) and
+// synchronises only `s`. Status words: the plan's own. A plan costs a launch, a
+// copy and a synchronisation to read the indexes and escape counts, then one
+// copy of every array the host makes, two launches and a synchronisation. With
+// four synchronisations, eleven copies and the items sorted as pairs: one head
+// x 500 tokens of head_dim 96 105 us instead of 55 (48 for the general kernel,
+// which has no records), 48 heads x 8,000 tokens 346 instead of 246, plain 128
+// instead of 82.
 void plan_build(kvexp_hip_plan *p, const kvexp_hip_head *heads, int n_heads, hipStream_t s) {
+    using P = kvexp_hip_plan;
     kvexp_hip_ctx *ctx = p->ctx;
     const int n_q = p->n_q, dim = p->dim, split_tokens = p->split_tokens;
     const bool xkv = heads[0].k_xkv != nullptr;
+    const bool wave = kvexp_launch::wave_supports(dim);
     std::vector<HeadDev> hv;
     std::vector<WorkItem> items;
     std::vector<int32_t> merge;
     int ws_slots = 0;
-    // every XKV head's block first tokens, read with one synchronisation
-    std::vector<size_t> first_at(size_t(n_heads) * 2, 0);
-    std::vector<int32_t> firsts;
-    const int32_t *first_all = nullptr;
+    // every XKV tensor's block first tokens and (one-wave and team kernels) the
+    // escapes before each block, n_blocks + 1 entries each, read with one
+    // synchronisation; the blocks are checked against their index on the way
+    std::vector<size_t> at(size_t(n_heads) * 2, 0); // a tensor's first entry
+    std::vector<kvexp_dev::EscJob> jobs;
+    std::vector<int32_t> firsts, e0;
+    uint32_t blocks_status = 0;
+    size_t total = 0;
     if (xkv) {
-        size_t total = 0;
         for (int h = 0; h < n_heads; ++h) {
             const kvexp_hip_head &H = heads[h];
-            if (H.k_xkv == nullptr || H.k_offsets == nullptr || H.v_offsets == nullptr ||
+            if (H.k_xkv == nullptr || H.v_xkv == nullptr || H.k_offsets == nullptr || H.v_offsets == nullptr ||
                 H.k_first_token == nullptr || H.v_first_token == nullptr || H.k_n_blocks <= 0 || H.v_n_blocks <= 0)
                 break; // reported below, head by head
-            first_at[size_t(2 * h)] = total;
-            total += size_t(H.k_n_blocks) + 1;
-            first_at[size_t(2 * h + 1)] = total;
-            total += size_t(H.v_n_blocks) + 1;
+            for (int kv = 0; kv < 2; ++kv) {
+                kvexp_dev::EscJob j{};
+                j.blob = kv ? H.v_xkv : H.k_xkv;
+                j.bytes = kv ? H.v_bytes : H.k_bytes;
+                j.offs = kv ? H.v_offsets : H.k_offsets;
+                j.first = kv ? H.v_first_token : H.k_first_token;
+                j.n_blocks = kv ? H.v_n_blocks : H.k_n_blocks;
+                j.dim = dim;
+                at[size_t(2 * h + kv)] = total;
+                total += size_t(j.n_blocks) + 1;
+                jobs.push_back(j);
+            }
         }
-        std::vector<kvexp_dev::FirstJob> fj;
-        for (int h = 0; h < n_heads; ++h) {
-            const kvexp_hip_head &H = heads[h];
-            if (H.k_xkv == nullptr || H.k_offsets == nullptr || H.v_offsets == nullptr ||
-                H.k_first_token == nullptr || H.v_first_token == nullptr || H.k_n_blocks <= 0 || H.v_n_blocks <= 0)
-                break;
-            fj.push_back({H.k_first_token, H.k_n_blocks + 1, int32_t(first_at[size_t(2 * h)])});
-            fj.push_back({H.v_first_token, H.v_n_blocks + 1, int32_t(first_at[size_t(2 * h + 1)])});
-        }
-        auto *host = static_cast<int32_t *>(pinned_staging(ctx, total * sizeof(int32_t)));
-        if (total > size_t(INT32_MAX)) fail(KVEXP_HIP_UNSUPPORTED, "kvexp_hip_plan_create: too many blocks in one plan");
-        if (!fj.empty()) {
-            // from the context's pool: their use ends with the synchronisation below
-            DevBuf dj(&ctx->pool, fj.size() * sizeof(kvexp_dev::FirstJob)), out(&ctx->pool, total * sizeof(int32_t));
-            struct SyncOnExit { // (also when a call below fails: before the buffers go back)
+        if (total > size_t(INT32_MAX))
+            fail(KVEXP_HIP_UNSUPPORTED, "kvexp_hip_plan_create: too many blocks in one plan");
+        firsts.resize(total);
+        e0.resize(total);
+        if (!jobs.empty()) {
+            // on the device: the jobs, a status word, the escapes and the first
+            // tokens (from the context's pool: their use ends with the
+            // synchronisation below)
+            const size_t job_bytes = jobs.size() * sizeof(kvexp_dev::EscJob);
+            DevBuf buf(&ctx->pool, job_bytes + (1 + 2 * total) * sizeof(int32_t));
+            auto *words = reinterpret_cast<int32_t *>(buf.as<uint8_t>() + job_bytes);
+            struct SyncOnExit { // (also when a call below fails: before the buffer goes back)
                 hipStream_t s;
                 ~SyncOnExit() { (void)hipStreamSynchronize(s); }
             } sync_on_exit{s};
-            HIPX(hipMemcpyAsync(dj.p, fj.data(), fj.size() * sizeof(kvexp_dev::FirstJob), hipMemcpyHostToDevice, s));
-            HIPX(kvexp_launch::gather_first(dj.as<kvexp_dev::FirstJob>(), int(fj.size()), out.as<int32_t>(), s));
-            HIPX(hipMemcpyAsync(host, out.p, total * sizeof(int32_t), hipMemcpyDeviceToHost, s));
+            std::vector<uint8_t> up(job_bytes + sizeof(uint32_t), 0);
+            for (size_t i = 0; i < jobs.size(); ++i) {
+                kvexp_dev::EscJob j = jobs[i];
+                j.esc0 = wave ? words + 1 + at[i] : nullptr;
+                j.first_out = words + 1 + total + at[i];
+                std::memcpy(up.data() + i * sizeof j, &j, sizeof j);
+            }
+            HIPX(hipMemcpyAsync(buf.p, up.data(), up.size(), hipMemcpyHostToDevice, s));
+            HIPX(kvexp_launch::esc_start(buf.as<kvexp_dev::EscJob>(), int(jobs.size()),
+                                         reinterpret_cast<uint32_t *>(words), s));
+            auto *host = static_cast<int32_t *>(pinned_staging(ctx, (1 + 2 * total) * sizeof(int32_t)));
+            HIPX(hipMemcpyAsync(host, words, (1 + 2 * total) * sizeof(int32_t), hipMemcpyDeviceToHost, s));
             HIPX(hipStreamSynchronize(s));
+            blocks_status = uint32_t(host[0]);
+            e0.assign(host + 1, host + 1 + total);
+            firsts.assign(host + 1 + total, host + 1 + 2 * total);
         }
-        firsts.assign(host, host + total);
-        first_all = firsts.data();
     }
+    const int32_t *first_all = firsts.data();
     for (int h = 0; h < n_heads; ++h) {
         const kvexp_hip_head &H = heads[h];
         const bool raw = H.k_raw != nullptr, x = H.k_xkv != nullptr;
@@ -1139,8 +1082,8 @@ void plan_build(kvexp_hip_plan *p, const kvexp_hip_head *heads, int n_heads, hip
                 H.v_first_token == nullptr || H.k_n_blocks <= 0 || H.v_n_blocks <= 0)
                 fail(KVEXP_HIP_INVALID_ARGUMENT, "kvexp_hip_plan_create: XKV head without a block index");
         }
-        const int32_t *kf0 = x ? first_all + first_at[size_t(2 * h)] : nullptr;
-        const int32_t *vf0 = x ? first_all + first_at[size_t(2 * h + 1)] : nullptr;
+        const int32_t *kf0 = x ? first_all + at[size_t(2 * h)] : nullptr;
+        const int32_t *vf0 = x ? first_all + at[size_t(2 * h + 1)] : nullptr;
         const int32_t *kf1 = x ? kf0 + H.k_n_blocks : nullptr; // last entry: tokens covered
         const int32_t *vf1 = x ? vf0 + H.v_n_blocks : nullptr;
         if (x && (*kf1 < H.seq || *vf1 < H.seq)) fail(KVEXP_HIP_FORMAT_ERROR, "xkv ran out of tokens");
@@ -1187,32 +1130,17 @@ void plan_build(kvexp_hip_plan *p, const kvexp_hip_head *heads, int n_heads, hip
             hv.push_back(d);
         }
     }
+    if (wave && blocks_status != 0u) fail(KVEXP_HIP_FORMAT_ERROR, status_message(blocks_status));
     p->xkv = xkv;
-    p->wave = kvexp_launch::wave_supports(dim);
-    const size_t slot_floats = size_t(kMaxQPerLaunch) * size_t(dim + 2);
-    {
-        using P = kvexp_hip_plan;
-        size_t n = P::padded(sizeof(uint32_t)) + P::padded(hv.size() * sizeof(HeadDev)) +
-                   P::padded(items.size() * sizeof(WorkItem)) +
-                   P::padded(std::max<size_t>(1, merge.size()) * sizeof(int32_t)) +
-                   P::padded(std::max<size_t>(1, size_t(ws_slots)) * slot_floats * sizeof(float)) +
-                   P::padded(size_t(2 * n_heads) * sizeof(kvexp_dev::EscJob));
-        if (p->wave) {
-            n += P::padded(std::max<size_t>(1, merge.size() * size_t(kMaxQPerLaunch)) * sizeof(kvexp_dev::MergeItem));
-            // per block: first escape, descriptor and the position builder's work list
-            const size_t e = firsts.size();
-            if (xkv)
-                n += P::padded(e * sizeof(int32_t)) + P::padded(e * sizeof(kvexp_dev::BlockDesc)) +
-                     P::padded(std::max<size_t>(1, e) * sizeof(int2));
-        }
-        p->reserve(n);
-    }
-    p->status = p->alloc(sizeof(uint32_t));
-    HIPX(hipMemsetAsync(p->status.p, 0, sizeof(uint32_t), s));
+    p->wave = wave;
     p->n_dev_heads = int(hv.size());
     p->n_items = int(items.size());
     p->n_merge = int(merge.size());
-    if (p->wave) {
+    const bool records = wave && xkv;
+    std::vector<kvexp_dev::MergeItem> mi;
+    std::vector<int2> blocks;
+    size_t pos_total = 0;
+    if (wave) {
         // items grouped by G (one launch per distinct G)
         const auto fewer_rows = [&](const WorkItem &a, const WorkItem &b) {
             return hv[size_t(a.head)].n_q < hv[size_t(b.head)].n_q;
@@ -1222,7 +1150,6 @@ void plan_build(kvexp_hip_plan *p, const kvexp_hip_head *heads, int n_heads, hip
         for (int G = 0; G < 10; ++G) p->group_start[G] = 0;
         for (const WorkItem &w : items) ++p->group_start[hv[size_t(w.head)].n_q + 1];
         for (int G = 1; G < 10; ++G) p->group_start[G] += p->group_start[G - 1];
-        std::vector<kvexp_dev::MergeItem> mi;
         for (int32_t dh : merge) {
             const HeadDev &d = hv[size_t(dh)];
             for (int g = 0; g < d.n_q; ++g) mi.push_back(kvexp_dev::MergeItem{d.ws_base, d.n_splits, d.q_row, g});
@@ -1243,39 +1170,94 @@ void plan_build(kvexp_hip_plan *p, const kvexp_hip_head *heads, int n_heads, hip
             }
             if (uni) p->merge_uni = kvexp_dev::MergeItem{f.ws_base, f.n_splits, f.q_row, G};
         }
-        p->mitems = p->alloc(std::max<size_t>(1, mi.size()) * sizeof(kvexp_dev::MergeItem));
-        if (!mi.empty())
-            HIPX(hipMemcpyAsync(p->mitems.p, mi.data(), mi.size() * sizeof(kvexp_dev::MergeItem),
-                                hipMemcpyHostToDevice, s));
-        if (xkv) {
-            build_escape_index(*p, heads, n_heads, n_q, dim, hv, s);
-            balance_items(*p, items, true, first_all, first_at, n_q, dim);
-            // the split's first descriptors as indexes into the plan's array
-            // (device head dh belongs to user head dh / per_head)
-            const int per_head = (n_q + kMaxQPerLaunch - 1) / kMaxQPerLaunch;
-            for (WorkItem &w : items) {
-                const int h = w.head / per_head;
-                w.kdi = int(p->esc_prefix_at[size_t(2 * h)]) + w.kblk;
-                w.vdi = int(p->esc_prefix_at[size_t(2 * h + 1)]) + w.vblk;
+        if (records) {
+            // each tensor's escape records, then room for its last block to grow
+            // to the largest block the format allows (255 tokens) after appends
+            for (size_t i = 0; i < jobs.size(); ++i) {
+                const size_t own = size_t(e0[at[i] + size_t(jobs[i].n_blocks)]);
+                jobs[i].pos_cap = int32_t(own + size_t(255) * size_t(dim));
+                pos_total += size_t(jobs[i].pos_cap);
+                for (int b = 0; b < jobs[i].n_blocks; ++b) blocks.push_back(make_int2(int(i), b));
             }
-        } else {
-            balance_items(*p, items, false, nullptr, std::vector<size_t>(), n_q, dim);
+            p->jobs = jobs;
+            p->esc_prefix = e0;
+            p->esc_prefix_at = at;
+        }
+        balance_items(*p, items, xkv, first_all, at, n_q, dim);
+    }
+    if (!records) p->jobs.assign(xkv ? 0 : size_t(2 * n_heads), kvexp_dev::EscJob{});
+    // The plan's arrays: what the host uploads first (in one copy), then what
+    // the kernels write. Escape records end with kEscPad spare ones: a kernel's
+    // window of records read from any escape stays inside the allocation
+    // (records past a block's count are never used).
+    const size_t slot_floats = size_t(kMaxQPerLaunch) * size_t(dim + 2);
+    const size_t n_status = P::padded(sizeof(uint32_t)), n_heads_b = hv.size() * sizeof(HeadDev),
+                 n_items_b = items.size() * sizeof(WorkItem), n_merge_b = merge.size() * sizeof(int32_t),
+                 n_mitems_b = mi.size() * sizeof(kvexp_dev::MergeItem),
+                 n_jobs_b = p->jobs.size() * sizeof(kvexp_dev::EscJob), n_blocks_b = blocks.size() * sizeof(int2);
+    const size_t n_image = n_status + P::padded(n_heads_b) + P::padded(n_items_b) + P::padded(n_merge_b) +
+                           P::padded(n_mitems_b) + P::padded(n_jobs_b) + P::padded(n_blocks_b);
+    const size_t n_ws = std::max<size_t>(1, size_t(ws_slots)) * slot_floats * sizeof(float);
+    const size_t n_esc0 = records ? total * sizeof(int32_t) : 0, n_desc = records ? total * sizeof(kvexp_dev::BlockDesc) : 0,
+                 n_pos = records ? (pos_total + size_t(kvexp_dev::kEscPad)) * sizeof(uint32_t) : 0;
+    p->reserve(n_image + P::padded(n_ws) + P::padded(n_esc0) + P::padded(n_desc) + P::padded(n_pos));
+    p->status = p->part(n_status);
+    p->heads = p->part(n_heads_b);
+    p->items = p->part(n_items_b);
+    p->merge_ids = p->part(n_merge_b);
+    p->mitems = p->part(n_mitems_b);
+    p->djobs = p->part(n_jobs_b);
+    DevBuf dblocks = p->part(n_blocks_b);
+    p->ws = p->part(n_ws);
+    p->esc0 = p->part(n_esc0);
+    p->desc = p->part(n_desc);
+    p->escpos = p->part(n_pos);
+    if (records) {
+        size_t pos = 0;
+        for (size_t i = 0; i < p->jobs.size(); ++i) {
+            kvexp_dev::EscJob &j = p->jobs[i];
+            j.esc0 = p->esc0.as<int32_t>() + at[i];
+            j.desc = p->desc.as<kvexp_dev::BlockDesc>() + at[i];
+            j.pos = p->escpos.as<uint32_t>() + pos;
+            pos += size_t(j.pos_cap);
+        }
+        // device head dh belongs to user head dh / per_head
+        const int per_head = (n_q + kMaxQPerLaunch - 1) / kMaxQPerLaunch;
+        for (size_t dh = 0; dh < hv.size(); ++dh) {
+            const size_t h = dh / size_t(per_head);
+            hv[dh].kdesc = p->jobs[2 * h].desc;
+            hv[dh].kesc = p->jobs[2 * h].pos;
+            hv[dh].vdesc = p->jobs[2 * h + 1].desc;
+            hv[dh].vesc = p->jobs[2 * h + 1].pos;
+        }
+        // the split's first descriptors as indexes into the plan's array
+        for (WorkItem &w : items) {
+            const size_t h = size_t(w.head / per_head);
+            w.kdi = int(at[2 * h]) + w.kblk;
+            w.vdi = int(at[2 * h + 1]) + w.vblk;
         }
     }
-    p->heads = p->alloc(hv.size() * sizeof(HeadDev));
-    p->items = p->alloc(items.size() * sizeof(WorkItem));
-    p->merge_ids = p->alloc(std::max<size_t>(1, merge.size()) * sizeof(int32_t));
-    p->ws = p->alloc(std::max<size_t>(1, size_t(ws_slots)) * slot_floats * sizeof(float));
-    HIPX(hipMemcpyAsync(p->heads.p, hv.data(), hv.size() * sizeof(HeadDev), hipMemcpyHostToDevice, s));
-    HIPX(hipMemcpyAsync(p->items.p, items.data(), items.size() * sizeof(WorkItem), hipMemcpyHostToDevice, s));
-    if (!merge.empty())
-        HIPX(hipMemcpyAsync(p->merge_ids.p, merge.data(), merge.size() * sizeof(int32_t), hipMemcpyHostToDevice, s));
-    if (!xkv) { // the job table kvexp_hip_plan_update sends lengths through
-        p->jobs.assign(size_t(2 * n_heads), kvexp_dev::EscJob{});
-        p->djobs = p->alloc(p->jobs.size() * sizeof(kvexp_dev::EscJob));
-    }
+    std::vector<uint8_t> image(n_image, 0); // (the status word 0)
+    const auto put = [&](const DevBuf &to, const void *from, size_t n) {
+        if (n) std::memcpy(image.data() + (to.as<uint8_t>() - p->arena.as<uint8_t>()), from, n);
+    };
+    put(p->heads, hv.data(), n_heads_b);
+    put(p->items, items.data(), n_items_b);
+    put(p->merge_ids, merge.data(), n_merge_b);
+    put(p->mitems, mi.data(), n_mitems_b);
+    put(p->djobs, p->jobs.data(), n_jobs_b);
+    put(dblocks, blocks.data(), n_blocks_b);
+    HIPX(hipMemcpyAsync(p->arena.p, image.data(), n_image, hipMemcpyHostToDevice, s));
     p->src.assign(heads, heads + n_heads);
-    HIPX(hipStreamSynchronize(s)); // the host vectors above are the copies' sources
+    if (!records) {
+        HIPX(hipStreamSynchronize(s)); // the image is the copy's source
+        return;
+    }
+    p->jobs_uploaded = true;
+    uint32_t *st = p->status.as<uint32_t>();
+    HIPX(kvexp_launch::esc_start(p->djobs.as<kvexp_dev::EscJob>(), int(p->jobs.size()), st, s));
+    HIPX(kvexp_launch::esc_pos(p->djobs.as<kvexp_dev::EscJob>(), dblocks.as<int2>(), int(blocks.size()), st, s));
+    check_status_word(ctx, st, s); // synchronises s: the image may go
 }
 
 // Moves a freshly built plan's device state into `dst` (an update that
