@@ -46,14 +46,19 @@ bool wave_supports(int dim) {
 // one-wave kernel's waves (four per SIMD, and three, or two at eight rows,
 // whose LDS leaves room for two workgroups), else the team kernel's teams; the
 // general kernel of the other sizes counts as two four-wave workgroups of four
-// splits each. `ragged`: teams count as four waves per SIMD at any G, since
-// the splits of a ragged batch come in several lengths and the short ones fill
-// in behind the long (four sequences of up to 25,003 tokens x 8 heads, eight
-// rows of head_dim 256: cut for 1,024 teams 90.1 us, for the 768 that fit 93.7;
-// other batches 130.6 and 143.0, 122.4 and 117.8).
-int resident_splits(int dim, int G, bool ragged) {
+// splits each. `uneven` (lengths of several sizes, or query rows in launches of
+// several sizes): more teams than fit above four rows, and twice those that fit
+// at 160 to 224, since the short splits fill in behind the long and a launch of
+// some of the rows holds less than a round. Four sequences of up to 25,003
+// tokens x 8 heads, eight rows of 256: cut for 1,024 teams 90.1 us, for the 768
+// that fit 93.7 (other batches 130.6 and 143.0, 122.4 and 117.8); 8 heads x
+// 30,000 tokens, 20 rows of 192: for 2,048 teams 155.9, for 1,024 171.9; 16 x
+// 4,000, twelve plain rows of 256: for 1,024 48.6, for 768 58.0.
+int resident_splits(int dim, int G, bool uneven) {
 #define KVEXP_RESIDENT_CASE(D)                                                                                       \
-    case D: return (G > 4 && !ragged ? team::kTeamOcc<8, D> : team::kTeamOcc<4, D>) * 4 / team::TShape<D>::W;
+    case D:                                                                                                          \
+        return uneven ? (D == 256 ? 4 : 8)                                                                           \
+                      : (G > 4 ? team::kTeamOcc<8, D> : team::kTeamOcc<4, D>) * 4 / team::TShape<D>::W;
     switch (dim) {
     case 32: return 16;
     case 64: return G < 8 ? 12 : 8;

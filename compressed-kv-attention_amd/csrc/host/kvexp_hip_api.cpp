@@ -46,7 +46,7 @@ hipError_t plan_refresh(const kvexp_dev::EscJob *jobs, int n_jobs, HeadDev *head
                         int n_items, int per_head, uint32_t *status, const kvexp_dev::PlanLens &lens, hipStream_t s);
 hipError_t result(const int64_t *value, const uint32_t *status, int64_t *host, hipStream_t s);
 bool wave_supports(int dim);
-int resident_splits(int dim, int G, bool ragged);
+int resident_splits(int dim, int G, bool uneven);
 hipError_t attention_wave(bool xkv, int order, int G, int dim, const HeadDev *heads, const WorkItem *items,
                           int n_items, int wpg, const kvexp_dev::BlockDesc *desc, const uint16_t *q, float *out,
                           float *lse, float *ws, hipStream_t s);
@@ -884,7 +884,9 @@ int suggest_core(const kvexp_hip_ctx *ctx, int64_t total_tokens, int max_seq, bo
     const int g = std::min(std::max(1, n_q), kMaxQPerLaunch);
     (void)order;
     const int64_t groups = (std::max(1, n_q) + kMaxQPerLaunch - 1) / kMaxQPerLaunch; // device heads per head
-    const int64_t slots = int64_t(kvexp_launch::resident_splits(dim, g, ragged)) * std::max(1, ctx->cu_count);
+    // a smaller last group is a launch of its own
+    const bool uneven = ragged || (groups > 1 && n_q % kMaxQPerLaunch != 0);
+    const int64_t slots = int64_t(kvexp_launch::resident_splits(dim, g, uneven)) * std::max(1, ctx->cu_count);
     const int64_t target = std::max<int64_t>(1, int64_t(max_seq) * slots / (total_tokens * groups));
     return int(std::max<int64_t>(1, std::min<int64_t>(tiles, target)));
 }
