@@ -72,3 +72,33 @@ def test_plans_of_one_context_in_turn(ctx):
     for px, pr, _, _ in made:
         px.close()
         pr.close()
+
+
+@pytest.mark.parametrize("dim,order", [(32, 0), (64, 0), (96, 0), (96, 1), (128, 0), (256, 1)])
+@pytest.mark.parametrize("n_q", [9, 10, 12, 14, 15, 16, 17, 21, 24])
+def test_groups_of_query_rows(ctx, oracle, dim, order, n_q):
+    """More than eight query rows: groups of equal size in small plans, of eight
+    in larger ones (more items than CUs), the oracle's bits in both."""
+    import torch
+
+    rng = np.random.default_rng(dim * 100 + n_q)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    seq, splits = 300, 3
+    for n_heads in (2, cus // (splits * 2) + 1):
+        if n_heads > 2 and n_q not in (12, 17):
+            continue
+        say("query row groups", dim, order, n_q, n_heads)
+        kv = [(random_kv(rng, seq, dim), random_kv(rng, seq, dim)) for _ in range(n_heads)]
+        q = random_kv(rng, n_heads * n_q, dim, spread_lo=-4, spread_hi=-2)
+        want = oracle.attention_heads("avx512" if order else "scalar", q,
+                                      [dict(k=k, v=v, seq=seq, threads=splits) for k, v in kv],
+                                      n_q=n_q, dim=dim, split=128)
+        dev = [dict(k=to_dev(k, torch.int16), v=to_dev(v, torch.int16), seq=seq, splits=splits) for k, v in kv]
+        plan = ctx.plan(dev, n_q, dim, 128, order)
+        assert bits_equal(plan.run(to_dev(q, torch.int16), check_errors=True).cpu().numpy(), want)
+        plan.update_heads([seq - 1] * n_heads)  # the fast update: the same groups, one token less
+        want = oracle.attention_heads("avx512" if order else "scalar", q,
+                                      [dict(k=k[:(seq - 1) * dim], v=v[:(seq - 1) * dim], seq=seq - 1, threads=splits)
+                                       for k, v in kv], n_q=n_q, dim=dim, split=128)
+        assert bits_equal(plan.run(to_dev(q, torch.int16), check_errors=True).cpu().numpy(), want)
+        plan.close()
