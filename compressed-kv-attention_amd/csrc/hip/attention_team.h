@@ -105,7 +105,8 @@ struct TRows {
 // 2 bytes below (c.shift): the decode picks the sign/mantissa bytes with other
 // byte selects and moves only the codes, and the two bytes that a piece lacks
 // are in the next lane's first dword (the last lane's: in sx and cx, aligned
-// dwords of which two bytes belong to the block).
+// dwords that start with them; the codes' last two bytes of a block without
+// escapes end it, and there the dword is the one that ends with them: c.back).
 template <int D>
 __device__ __forceinline__ void load_team_rows(Cursor &c, int w, int r0, int rows, TRows<D> &R) {
     using S = TShape<D>;
@@ -117,7 +118,7 @@ __device__ __forceinline__ void load_team_rows(Cursor &c, int w, int r0, int row
     const int cbytes = mode * (D / 8), cw = 2 * mode;
     const int cd = D + c.ntok() * D + cw - 8; // the load that ends with the codes of the block's piece 0
     c.shift = 0;
-    // the dwords behind the wave's rows (shifted rows; else any aligned dword of the block)
+    // the dwords with the last bytes of the wave's rows (shifted rows; else any aligned dword of the block)
     const uint8_t *px = reinterpret_cast<const uint8_t *>(reinterpret_cast<uintptr_t>(c.blk + 8) & ~uintptr_t(3));
     const uint8_t *pc = px;
     if (!raw && c.ntok() - r0 >= kChunk) {
@@ -128,7 +129,8 @@ __device__ __forceinline__ void load_team_rows(Cursor &c, int w, int r0, int row
             sb -= 2;
             cb -= 2;
             px = sb + S::RO * D;
-            pc = cb + (S::RO * cbytes + 8 - cw);
+            c.back = c.nesc() == 0 ? 16 : 0;
+            pc = cb + (S::RO * cbytes + 8 - cw) - c.back / 8;
         }
         const int ll = S::Last < kWave - 1 ? min(lane, S::Last) : lane;
         const uint32_t cl = uint32_t(cw * lane);
@@ -283,7 +285,7 @@ __device__ __forceinline__ uint32_t next_dword(uint32_t x, uint32_t y) {
 
 template <int D, bool PLAIN, int MODE, bool SHIFT>
 __device__ __forceinline__ void decode_team_mode(const TRows<D> &R, const uint32_t (&bp)[8], uint8_t *tile, int w,
-                                                 uint32_t smm) {
+                                                 uint32_t smm, int back = 0) {
     using S = TShape<D>;
     const int lane = lane_here();
     const int lr = lane / S::NP, col = lane - lr * S::NP;
@@ -297,10 +299,10 @@ __device__ __forceinline__ void decode_team_mode(const TRows<D> &R, const uint32
         if constexpr (SHIFT) {
             s4 = next_dword<D, end>(sm.x, end ? R.sx : R.s[kn].x);
             if constexpr (MODE == 4) {
-                const uint32_t c2 = next_dword<D, end>(cd.x, end ? R.cx : R.c[kn].x);
+                const uint32_t c2 = next_dword<D, end>(cd.x, end ? R.cx >> back : R.c[kn].x);
                 cd = make_uint2(__builtin_amdgcn_alignbit(cd.y, cd.x, 16), __builtin_amdgcn_alignbit(c2, cd.y, 16));
             } else { // the lane's codes are the upper four of its 8 bytes, the next lane's 8 start 4 further on
-                const uint32_t c2 = next_dword<D, end>(cd.y, end ? R.cx : R.c[kn].y);
+                const uint32_t c2 = next_dword<D, end>(cd.y, end ? R.cx >> back : R.c[kn].y);
                 cd.y = __builtin_amdgcn_alignbit(c2, cd.y, 16);
             }
         }
@@ -358,10 +360,10 @@ __device__ __forceinline__ void decode_team_rows(const Cursor &c, const TRows<D>
                 bp[4 * h + p] = __builtin_amdgcn_perm(b1, b0, 0x0c000c00u | ((4u + p) << 16) | p) << 7;
         }
         if (mode == 4) {
-            if (c.shift) decode_team_mode<D, PLAIN, 4, true>(R, bp, tile, w, smm);
+            if (c.shift) decode_team_mode<D, PLAIN, 4, true>(R, bp, tile, w, smm, c.back);
             else decode_team_mode<D, PLAIN, 4, false>(R, bp, tile, w, smm);
         } else if (mode == 2) {
-            if (c.shift) decode_team_mode<D, PLAIN, 2, true>(R, bp, tile, w, smm);
+            if (c.shift) decode_team_mode<D, PLAIN, 2, true>(R, bp, tile, w, smm, c.back);
             else decode_team_mode<D, PLAIN, 2, false>(R, bp, tile, w, smm);
         } else {
             decode_team_mode<D, PLAIN, 3, false>(R, bp, tile, w, smm);

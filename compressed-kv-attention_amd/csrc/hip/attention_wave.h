@@ -193,6 +193,7 @@ struct Cursor {
     int ecur;            // first escape of the block not yet written into a tile
     int lrows;           // rows requested by the last load_rows (the raw piece layout depends on it)
     int shift;           // the rows were loaded from 2 bytes below their start (see load_team_rows)
+    int back;            // ... and bits of the codes' last dword before their last two bytes
     uint4 erec;
     uint32_t basew;
     __device__ int mode() const { return int(meta & 0xFFu); }
