@@ -711,18 +711,11 @@ __global__ __launch_bounds__(kThreads) void append_write_kernel(const AppendJobD
 }
 
 // The raw rows of a job's new trailing partial block that are not in its tail
-// buffer yet, copied there: 16 bytes per thread and step where source, tail
-// and row size allow it (32 tails of 86 rows of head_dim 256: 21.8 us with
-// 2-byte copies).
+// buffer yet, copied there.
 __device__ __forceinline__ void copy_rows(const AppendJobDev &j, int dim) {
     const int total = j.copy_rows * dim;
     const uint16_t *from = j.src + size_t(j.copy_from) * size_t(dim);
     uint16_t *to = j.tail + size_t(j.copy_to) * size_t(dim);
-    if (dim % 8 == 0 && ((reinterpret_cast<uintptr_t>(from) | reinterpret_cast<uintptr_t>(to)) & 15u) == 0) {
-        for (int i = int(threadIdx.x); i < total / 8; i += int(blockDim.x))
-            reinterpret_cast<uint4 *>(to)[i] = reinterpret_cast<const uint4 *>(from)[i];
-        return;
-    }
     for (int i = int(threadIdx.x); i < total; i += int(blockDim.x)) to[i] = from[i];
 }
 
@@ -1447,8 +1440,8 @@ __global__ __launch_bounds__(kThreads) void append_one_kernel(const AppendJobDev
 // takes the i-th escape word, which the format stores after the codes; a
 // sentinel count other than n_escape raises kStEscape. All threads of the
 // workgroup call it.
-// octets (total % 8 == 0, as head_dim is a multiple of 8): a segment of 16,384
-// codes at a time, all of its code words in flight together and one barrier
+// The codes go by octets (a plan's head_dims are multiples of 8): a segment of
+// 16,384 codes at a time, all of its code words in flight together and one barrier
 // for the waves' counts, as in decode_coded; a segment that is not full is
 // spread over all waves. The sentinels' element indexes go to LDS by rank and
 // the records are put together at the end, a record per thread with the words
@@ -1521,51 +1514,21 @@ __device__ __forceinline__ void escape_positions(const uint8_t *codes, int mode,
                                                  uint32_t *__restrict__ pos, int *scan_tmp,
                                                  uint32_t *__restrict__ status) {
     __shared__ uint16_t at[kRecWin];
-    int carry = 0;
-    if (total % 8 == 0) {
-        carry = mode == 4   ? escape_octets<4>(codes, total / 8, n_escape, pos, scan_tmp, at)
-                : mode == 2 ? escape_octets<2>(codes, total / 8, n_escape, pos, scan_tmp, at)
-                            : escape_octets<3>(codes, total / 8, n_escape, pos, scan_tmp, at);
-    } else { // 2- and 4-bit codes, four elements per thread and step
-        const uint8_t *words = codes + (total * mode + 7) / 8;
-        const uint32_t sentinel = (1u << mode) - 1u;
-        const int units = total / 4;
-        for (int r = 0; r < units; r += kThreads) {
-            const int u = r + int(threadIdx.x);
-            const bool act = u < units;
-            uint32_t cw = 0;
-            int cnt = 0;
-            if (act) {
-                cw = load_codes(codes, mode, u);
-                cnt = unit_sentinels(cw, mode);
-            }
-            int tot = 0;
-            int rank = carry + block_excl_scan<kWaves>(cnt, scan_tmp, &tot);
-            carry += tot;
-            if (act && cnt) {
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    if (unit_code(cw, mode, k) == sentinel) {
-                        if (rank < n_escape) pos[rank] = uint32_t(4 * u + k) | (load_u16_any(words + 2 * rank) << 16);
-                        ++rank;
-                    }
-                }
-            }
-        }
-    }
+    const int carry = mode == 4   ? escape_octets<4>(codes, total / 8, n_escape, pos, scan_tmp, at)
+                      : mode == 2 ? escape_octets<2>(codes, total / 8, n_escape, pos, scan_tmp, at)
+                                  : escape_octets<3>(codes, total / 8, n_escape, pos, scan_tmp, at);
     if (threadIdx.x == 0 && carry != n_escape) atomicOr(status, kStEscape);
 }
 
 // esc0[b] = escape words in blocks before b (raw blocks count 0), one
-// workgroup per tensor. With j.first set, every block is also checked against
-// the index (header inside the container, head_dim, n_tokens equal to the
-// index's token count, known mode, payload inside the container); with
-// j.desc set (and j.pos allocated), its descriptor is written, and the entry
-// after the last one becomes a zero-token sentinel (a split kernel that reached
-// it would stop there). With j.first_out set, the index's first tokens go there
-// too, so that the host reads those of all tensors with one copy (c2's 96
-// tensors took 96 copies, about 0.9 ms of a plan's 1.25); with j.esc0 null only
-// these.
+// workgroup per tensor. Every block is checked against the index (header inside
+// the container, head_dim, n_tokens equal to the index's token count, known
+// mode, payload inside the container); with j.desc set (and j.pos allocated),
+// its descriptor is written, and the entry after the last one becomes a
+// zero-token sentinel (a split kernel that reached it would stop there). With
+// j.first_out set, the index's first tokens go there too, so that the host
+// reads those of all tensors with one copy (c2's 96 tensors took 96 copies,
+// about 0.9 ms of a plan's 1.25); with j.esc0 null only these.
 __global__ __launch_bounds__(kThreads) void esc_start_kernel(const EscJob *__restrict__ jobs,
                                                             uint32_t *__restrict__ status) {
     __shared__ int scan_tmp[kWaves];
@@ -1582,13 +1545,7 @@ __global__ __launch_bounds__(kThreads) void esc_start_kernel(const EscJob *__res
         int64_t off = 0;
         if (b < j.n_blocks) {
             off = j.offs[b];
-            if (j.first != nullptr) {
-                st = check_block(j.blob, j.bytes, off, j.dim, j.first[b + 1] - j.first[b], &h);
-            } else if (off >= 0 && uint64_t(off) + 8u <= j.bytes) {
-                h = read_hdr(j.blob + off);
-            } else {
-                st = kStHeader;
-            }
+            st = check_block(j.blob, j.bytes, off, j.dim, j.first[b + 1] - j.first[b], &h);
             if (st != 0u) atomicOr(status, st);
             else ne = h.mode == 0 ? 0 : h.n_escape;
         }

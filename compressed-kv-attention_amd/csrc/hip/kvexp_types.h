@@ -24,7 +24,7 @@ struct HeadDev {
     const int64_t *koff, *voff;  // block byte offsets (n_blocks + 1)
     const int32_t *kfirst, *vfirst; // block first tokens (n_blocks + 1)
     const uint16_t *kraw, *vraw; // [seq, dim] BF16 (raw heads)
-    // Plan-owned, XKV heads of the wave kernel: validated block descriptors
+    // Plan-owned, XKV heads of the one-wave and team kernels: validated block descriptors
     // and the escape records (block b's escapes are records
     // [desc[b].esc, desc[b].esc + n_escape), in scan order; format at kEscPad).
     const struct BlockDesc *kdesc, *vdesc;
@@ -40,11 +40,10 @@ struct HeadDev {
 // An escape record: the escape's element index inside its block (row * dim
 // + channel) in bits 0..15 and its BF16 word in bits 16..31. The plan copies
 // each block's escape words out of the container next to their positions, so
-// the wave kernel reads a window of escapes with 16-byte loads per lane (up
-// to 2,048 records). Every records array ends with kEscPad spare records, so
-// such a window read from any escape of any block stays inside the
-// allocation.
-constexpr int kEscPad = 2052;
+// the split kernels read a window of escapes with at most 16 bytes per lane
+// (256 records). Every records array ends with kEscPad spare records, so such a
+// window read from any escape of any block stays inside the allocation.
+constexpr int kEscPad = 260;
 
 // One block of a container as the wave kernel reads it, built and checked
 // against the block index once per plan (esc_start_kernel). 32 bytes, so a
