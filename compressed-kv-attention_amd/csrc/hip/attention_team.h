@@ -71,7 +71,7 @@ struct alignas(16) TeamLds {
     float eT[G][kRowPad]; // e of token t, row g (0 past the chunk's end)
     float aT[G][kRowPad]; // alpha of token t, row g (1 where no running maximum moves)
     uint64_t am[4];       // per wave: tokens that move a running maximum of its rows
-    uint32_t low[4];      // AVX-512 order, rows as they are (plain or a raw block): whether the wave's need the flushing scores
+    uint32_t low[4];      // AVX-512 order, plain BF16 rows: whether the wave's rows need the flushing scores
 };
 
 // Workgroup barrier for LDS traffic only: the global loads in flight stay in
@@ -96,7 +96,8 @@ struct TRows {
 // holds a whole chunk of coded rows the addresses are the streams' starts plus
 // the lane's offset (the lanes of the last register past the wave's rows
 // repeat its last piece); elsewhere loads past the chunk's rows repeat their
-// last piece. None leaves the block, and both paths issue the same loads.
+// last piece. Both paths issue the same loads, which stay in the block but for
+// the half dword named below.
 //
 // Blocks are 2-byte aligned, and loads of 16 or 8 bytes at an address that is
 // not a multiple of 4 keep the CU's address unit about four times as long
@@ -105,8 +106,13 @@ struct TRows {
 // 2 bytes below (c.shift): the decode picks the sign/mantissa bytes with other
 // byte selects and moves only the codes, and the two bytes that a piece lacks
 // are in the next lane's first dword (the last lane's: in sx and cx, aligned
-// dwords that start with them; the codes' last two bytes of a block without
-// escapes end it, and there the dword is the one that ends with them: c.back).
+// dwords that start with them). Where a block without escapes ends with the
+// wave's codes, the upper half of cx lies past the block, and past the container
+// if it is the last one: an aligned dword whose lower half is inside is in the
+// same page, so it can be read, and the upper half is not used. (Kept inside by
+// 2-byte loads, or by the dword that ends with the codes and a shift, eight rows
+// of head_dim 256 took 91.5 for 90.4 us, and three rows of one head x 4,096
+// tokens 25.7 for 25.0.)
 template <int D>
 __device__ __forceinline__ void load_team_rows(Cursor &c, int w, int r0, int rows, TRows<D> &R) {
     using S = TShape<D>;
@@ -129,8 +135,7 @@ __device__ __forceinline__ void load_team_rows(Cursor &c, int w, int r0, int row
             sb -= 2;
             cb -= 2;
             px = sb + S::RO * D;
-            c.back = c.nesc() == 0 ? 16 : 0;
-            pc = cb + (S::RO * cbytes + 8 - cw) - c.back / 8;
+            pc = cb + (S::RO * cbytes + 8 - cw);
         }
         const int ll = S::Last < kWave - 1 ? min(lane, S::Last) : lane;
         const uint32_t cl = uint32_t(cw * lane);
@@ -285,7 +290,7 @@ __device__ __forceinline__ uint32_t next_dword(uint32_t x, uint32_t y) {
 
 template <int D, bool PLAIN, int MODE, bool SHIFT>
 __device__ __forceinline__ void decode_team_mode(const TRows<D> &R, const uint32_t (&bp)[8], uint8_t *tile, int w,
-                                                 uint32_t smm, int back = 0) {
+                                                 uint32_t smm) {
     using S = TShape<D>;
     const int lane = lane_here();
     const int lr = lane / S::NP, col = lane - lr * S::NP;
@@ -299,10 +304,10 @@ __device__ __forceinline__ void decode_team_mode(const TRows<D> &R, const uint32
         if constexpr (SHIFT) {
             s4 = next_dword<D, end>(sm.x, end ? R.sx : R.s[kn].x);
             if constexpr (MODE == 4) {
-                const uint32_t c2 = next_dword<D, end>(cd.x, end ? R.cx >> back : R.c[kn].x);
+                const uint32_t c2 = next_dword<D, end>(cd.x, end ? R.cx : R.c[kn].x);
                 cd = make_uint2(__builtin_amdgcn_alignbit(cd.y, cd.x, 16), __builtin_amdgcn_alignbit(c2, cd.y, 16));
             } else { // the lane's codes are the upper four of its 8 bytes, the next lane's 8 start 4 further on
-                const uint32_t c2 = next_dword<D, end>(cd.y, end ? R.cx >> back : R.c[kn].y);
+                const uint32_t c2 = next_dword<D, end>(cd.y, end ? R.cx : R.c[kn].y);
                 cd.y = __builtin_amdgcn_alignbit(c2, cd.y, 16);
             }
         }
@@ -360,10 +365,10 @@ __device__ __forceinline__ void decode_team_rows(const Cursor &c, const TRows<D>
                 bp[4 * h + p] = __builtin_amdgcn_perm(b1, b0, 0x0c000c00u | ((4u + p) << 16) | p) << 7;
         }
         if (mode == 4) {
-            if (c.shift) decode_team_mode<D, PLAIN, 4, true>(R, bp, tile, w, smm, c.back);
+            if (c.shift) decode_team_mode<D, PLAIN, 4, true>(R, bp, tile, w, smm);
             else decode_team_mode<D, PLAIN, 4, false>(R, bp, tile, w, smm);
         } else if (mode == 2) {
-            if (c.shift) decode_team_mode<D, PLAIN, 2, true>(R, bp, tile, w, smm, c.back);
+            if (c.shift) decode_team_mode<D, PLAIN, 2, true>(R, bp, tile, w, smm);
             else decode_team_mode<D, PLAIN, 2, false>(R, bp, tile, w, smm);
         } else {
             decode_team_mode<D, PLAIN, 3, false>(R, bp, tile, w, smm);
@@ -516,9 +521,12 @@ __device__ __forceinline__ void team_scores_dp(const uint8_t *row, int w, const 
                         ch[rg][J] = mfma_rank1<(i0 + e) % 16>(qa[rg][(i0 + e) / 16], k, ch[rg][J]);
                 });
             });
-            // octet by octet (all octets read ahead spilled above four rows)
-            __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);
-            __builtin_amdgcn_sched_group_barrier(0x008, 8 * NG, 0);
+            // octet by octet (all octets read ahead spilled above four rows; one
+            // head x 4,096 tokens, three rows of head_dim 128: 26.6 us with, 26.2 without)
+            if constexpr (NG > 1 || S::W == 4) {
+                __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, 8 * NG, 0);
+            }
         });
 #pragma unroll
         for (int rg = 0; rg < NG; ++rg) {
@@ -527,6 +535,21 @@ __device__ __forceinline__ void team_scores_dp(const uint8_t *row, int w, const 
             else p[rg] = p[rg] + a;
         }
     });
+}
+
+// Whether the wave's channels of any `in` lane's tile row hold an element below
+// the bound (see low_bf16). A wave's own chains flush or do not: the others'
+// answers may differ.
+template <int D>
+__device__ __forceinline__ bool team_row_low(const uint8_t *row, int w, bool in, uint32_t low) {
+    constexpr int NQ = 4 / TShape<D>::W;
+    low_min_t lo = kLowMinNone;
+#pragma unroll 1
+    for (int c = 0; c < D / 32; ++c)
+#pragma unroll
+        for (int x = 0; x < NQ; ++x)
+            lo = low_min(lo, *reinterpret_cast<const uint4 *>(row + 16 * (4 * c + NQ * w + x)));
+    return any_low(in ? lo : kLowMinNone, low);
 }
 
 // The same with every flush applied (scores_dp_flush), on the vector ALU.
@@ -807,7 +830,7 @@ void attn_team_kernel(const HeadDev *__restrict__ heads, const WorkItem *__restr
         const int tn = t + n, tp = min(tn, wi.tok_end - 1);
 
         // 1. the wave's K rows -> tile, the next ones requested
-        bool flush = false, checked = !XKV; // checked: S.low holds the waves' answers for the chunk's rows
+        bool flush = false, kraw = false; // kraw: rows of a raw block, checked in the tile
         if constexpr (XKV) after(RK.c[SH::NR - 1].y);
         stamp(0); // K rows arrived
         if constexpr (XKV) {
@@ -819,17 +842,10 @@ void attn_team_kernel(const HeadDev *__restrict__ heads, const WorkItem *__restr
                     const u16x2 bmin = __builtin_elementwise_min(e, o), bmax = __builtin_elementwise_max(e, o);
                     const uint32_t top = 256u - (1u << kc.mode());
                     flush = __ballot(uint32_t(min(bmin.x, bmin.y)) < kmin || uint32_t(max(bmax.x, bmax.y)) > top) != 0;
-                } else { // the wave's rows < n of a raw block (decode_team_rows)
-                    constexpr int RW = SH::RawRows / W;
-                    low_min_t lo = kLowMinNone;
-#pragma unroll
-                    for (int k = 0; k < SH::NR; ++k) {
-                        const int r = (64 * k + ln) / (D / 8);
-                        if (r < RW && RW * w + r < n) lo = low_min(lo, RK.s[k]);
-                    }
-                    const bool low = any_low(lo, klow);
-                    if (ln == 0) S.low[w] = low ? 1u : 0u;
-                    checked = true;
+                } else if constexpr (kRawChecked<D>) {
+                    kraw = true;
+                } else {
+                    flush = true;
                 }
             }
             decode_team_rows<D, KP, false>(kc, RK, S.tile, w, n);
@@ -864,11 +880,14 @@ void attn_team_kernel(const HeadDev *__restrict__ heads, const WorkItem *__restr
             if constexpr (ORDER == 0) {
                 team_scores<G, D>(row + 2 * CW * w, qa, p);
             } else {
-                if (checked) {
+                if constexpr (!XKV) {
                     uint32_t any = 0;
 #pragma unroll
                     for (int i = 0; i < W; ++i) any |= S.low[i];
                     flush = __builtin_amdgcn_readfirstlane(any) != 0;
+                }
+                if constexpr (XKV && kRawChecked<D>) {
+                    if (kraw) flush = team_row_low<D>(row, w, ln < n, klow);
                 }
                 if (!flush) team_scores_dp<G, D>(row, w, qa, p);
                 else team_scores_dp_flush<G, D>(row, w, qh, p);

@@ -193,7 +193,6 @@ struct Cursor {
     int ecur;            // first escape of the block not yet written into a tile
     int lrows;           // rows requested by the last load_rows (the raw piece layout depends on it)
     int shift;           // the rows were loaded from 2 bytes below their start (see load_team_rows)
-    int back;            // ... and bits of the codes' last dword before their last two bytes
     uint4 erec;
     uint32_t basew;
     __device__ int mode() const { return int(meta & 0xFFu); }
@@ -639,10 +638,14 @@ __device__ __forceinline__ void decode_rows(const Cursor &c, Rows<D> &R, const u
 // element of the head (denormal queries read as zero beforehand), no input,
 // chain value or sum is denormal, and the flushes are the identity. A chunk
 // with a smaller K exponent takes the vector path that applies the flushes. A
-// raw block's rows are checked element by element in the registers that hold
-// them (8 heads x 4,100 tokens of raw blocks, eight rows of head_dim 96: 152 us
-// with every such chunk flushing, 51 so; 32: 104 and 36), except at head_dim
-// 64, where every chunk of one takes the flushing path.
+// raw block's rows are checked element by element (8 heads x 4,100 tokens of raw
+// blocks, eight rows of head_dim 96: 152 us with every such chunk flushing, 51
+// so; 32: 104 and 36), except at head_dim 64, where a lane holds them by whole
+// rows, and at 256, where the check costs coded rows 2 to 3 % (64 heads x 24,000
+// tokens, three rows: 254 to 261 us): there every chunk of one takes the
+// flushing path.
+template <int D>
+constexpr bool kRawChecked = D != 64 && D != 256;
 
 // Whether BF16 x is nonzero with exponent field below T, for
 // low = (T << 7) - 1 (T >= 1): (x & 0x7FFF) - 1 wraps to 2^32 - 1 for a zero.
@@ -1310,7 +1313,7 @@ void attn_wave_kernel(const HeadDev *__restrict__ heads, const WorkItem *__restr
                     wave_sync();
                 }
             } else if constexpr (ORDER == 1) {
-                if constexpr (kWholeRows<D>) {
+                if constexpr (!kRawChecked<D>) {
                     flush = true;
                 } else { // the loaded pieces of rows < n (decode_pieces; each lies in one row)
                     low_min_t lo = kLowMinNone;
