@@ -959,10 +959,10 @@ void balance_items(kvexp_hip_plan &p, std::vector<WorkItem> &items, bool xkv, co
         const int b = p.group_start[G], e = p.group_start[G + 1];
         const int n = e - b;
         if (n <= wpw || n % wpw != 0) continue; // whole workgroups only
-        // sorted as words, cost in 1/16 tokens above and place below
+        // sorted as words, cost in 1/256 tokens above and place below
         std::vector<uint64_t> order(static_cast<size_t>(n));
         for (int i = 0; i < n; ++i) {
-            const double c = std::min(16.0 * std::max(0.0, cost(items[size_t(b + i)])), 4294967295.0);
+            const double c = std::min(256.0 * std::max(0.0, cost(items[size_t(b + i)])), 4294967295.0);
             order[size_t(i)] = (uint64_t(0xFFFFFFFFu - uint32_t(c)) << 32) | uint32_t(i);
         }
         std::sort(order.begin(), order.end());
