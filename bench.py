@@ -625,7 +625,7 @@ def bench_config(a, torch, np, kvexp_amd, synth) -> int:
         "xkv_bit_equal_raw": same,
         "roofline": {"bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBPS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBPS, 4), "traffic": None,
-                     "kernel": f"attn_wave_kernel<{G}, {D}, true, 0>", "kernel_us": round(kern_avg_ms * 1e3, 2),
+                     "kernel": f"attn_{'wave' if D <= 64 else 'team'}_kernel<{G}, {D}, true, 0>", "kernel_us": round(kern_avg_ms * 1e3, 2),
                      "algorithmic_bytes": algo},
     }), flush=True)
     return 0 if same else 1

@@ -27,11 +27,12 @@
 // The operations of every score, coefficient and accumulator are those of
 // the one-wave kernel in the same order, so the outputs are its bits.
 //
-// Bound: instruction issue (at head_dim 128 the vector and matrix pipes are
-// busy about 80 % of the launch at the clock it runs at), then HBM. Measured,
+// Bound: instruction issue, then HBM (SQ counters: the vector and matrix pipes
+// are busy 77 % of a launch at head_dim 128, 68 % at 96 and 51 % at eight rows
+// of 256, where three waves per SIMD wait at five barriers per chunk). Measured,
 // per attention call, before (one wave per split at 128 and 256, a four-wave
 // kernel on the vector ALU at the other sizes) and with teams: 64 heads x 4
-// queries, head_dim 128, 65,536 tokens: 373 -> 324-335 us (4.8-5.0 TB/s);
+// queries, head_dim 128, 65,536 tokens: 373 -> 332-338 us (4.8-4.9 TB/s);
 // four sequences of up to 25,003 tokens x 8 heads x 8 queries, head_dim 256:
 // 204 -> 90 us; 64 heads x 4 queries, head_dim 96, 16,411 tokens: 735 -> 83 us.
 // At head_dim 64 one wave stays: half the lanes of a two-wave team's fold

@@ -748,7 +748,8 @@ __global__ __launch_bounds__(kThreads) void append_tail_kernel(const AppendJobDe
 // and escape ranks are computed (so that the earlier blocks have had that
 // long to publish). Then the block is written from the registers.
 // Bound: vector instructions (about 1,000 per wave and block at head_dim 64;
-// the pipe is busy about 80 % of the launch) and the block's chain of
+// SQ counters: the vector pipe is busy 74 % of that launch, 54 % at head_dim 256,
+// where two workgroups fit a CU) and the block's chain of
 // barriers, which eight workgroups per CU overlap. Per prefill call: 96
 // containers x 32,768 tokens of head_dim 64, 264 -> 224 us (2.7 -> 3.2 TB/s);
 // 32 x 8,150 tokens of head_dim 256 (blocks of 32,768 elements, which took the
@@ -855,8 +856,8 @@ __device__ __forceinline__ EscRanks<NL> fused_escape_ranks(const uint32_t (&v)[E
 // 1,024 for blocks of 8,193 to 32,768 elements) are slower: what a thread does
 // once per block outweighs the waves gained (prefill of 48 x 16,384 tokens of
 // head_dim 128: 129 -> 180 us, 32 x 8,150 of 256: 96 -> 122 us).
-// Waves per SIMD the one-pass encoder is compiled for (its registers fit
-// 512 / waves without spilling): 8 with up to four chunk rows per thread.
+// Waves per SIMD the one-pass encoder is compiled for: 8 with up to four chunk
+// rows per thread (64 registers; at four rows two more are spilled).
 template <int NL>
 constexpr int kFusedWaves = NL <= 4 ? 8 : 4;
 // Fewest waves per SIMD the compiler may plan for. Up to two chunk rows per
