@@ -1720,16 +1720,20 @@ hipError_t launch_fused_j(const AppendJobDev *jobs, int n_jobs, const AppendJobD
     if (configured != hipSuccess) return configured;
     const size_t lds = fused_lds_bytes(dim, bt);
     // P workgroups per job: as many as are resident together over all jobs
-    // (each loops over its job's blocks), at most the longest job's blocks
-    int dev = 0, cus = 0, per_cu = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    if (e == hipSuccess)
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &per_cu, reinterpret_cast<const void *>(encode_fused_kernel<NL, TH, JOBS>), TH, lds);
-    if (e != hipSuccess) return e;
-    const int64_t resident = std::max<int64_t>(1, int64_t(cus) * std::max(per_cu, 1));
-    const int per_job = int(std::max<int64_t>(1, std::min<int64_t>(max_job_blocks, resident / std::max(n_jobs, 1))));
+    // (each loops over its job's blocks), at most the longest job's blocks (a
+    // decode step's jobs have one each: nothing to ask the runtime)
+    int64_t per_job = 1;
+    if (max_job_blocks > 1) {
+        int dev = 0, cus = 0, per_cu = 0;
+        hipError_t e = hipGetDevice(&dev);
+        if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+        if (e == hipSuccess)
+            e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                &per_cu, reinterpret_cast<const void *>(encode_fused_kernel<NL, TH, JOBS>), TH, lds);
+        if (e != hipSuccess) return e;
+        const int64_t resident = std::max<int64_t>(1, int64_t(cus) * std::max(per_cu, 1));
+        per_job = std::max<int64_t>(1, std::min<int64_t>(max_job_blocks, resident / std::max(n_jobs, 1)));
+    }
     hipLaunchKernelGGL((encode_fused_kernel<NL, TH, JOBS>), dim3(unsigned(per_job), unsigned(n_jobs)),
                        dim3(TH), lds, s, jobs, one, dim, bt, modes, lb.words, lb.tickets, lb.epoch, status);
     return hipGetLastError();
