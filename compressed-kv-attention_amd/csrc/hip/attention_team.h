@@ -603,14 +603,15 @@ struct TFoldIn {
 
 // Token T of the ordered fold (see fold_token), one channel per lane. L: the
 // wave also carries l.
-template <int G, int D, int T, bool MOVE, bool L>
+template <int G, int D, int T, bool MOVE, bool L, bool AHEAD>
 __device__ __forceinline__ void team_fold_token(const TeamLds<G, D> &S, lds_f32 *eb, lds_f32 *ab, const uint8_t *trb,
                                                 const uint32_t (&am)[2], const float (&ea)[kGroups<G>][4], TFoldIn &in,
                                                 f4 &a4, f4 (&acc)[kGroups<G>], float &lvec) {
     constexpr int NG = kGroups<G>, TS = TShape<D>::TS, Q = T / 4;
     if constexpr (T % 4 == 0) {
         if constexpr (4 * (Q + 2) < kChunk) in.vq[(Q + 2) % 3] = load_tr(trb + 4 * (Q + 2) * TS);
-        if constexpr (L && 4 * (Q + 1) < kChunk) in.e4[(Q + 1) & 1] = *reinterpret_cast<lds_f4 *>(eb + 4 * (Q + 1));
+        if constexpr (L && AHEAD && 4 * (Q + 1) < kChunk)
+            in.e4[(Q + 1) & 1] = *reinterpret_cast<lds_f4 *>(eb + 4 * (Q + 1));
         if constexpr (L && MOVE) a4 = *reinterpret_cast<lds_f4 *>(ab + 4 * Q);
     }
     const float v = quad_f32<T % 4>(in.vq[Q % 3]);
@@ -627,16 +628,17 @@ __device__ __forceinline__ void team_fold_token(const TeamLds<G, D> &S, lds_f32 
         }
     }
     if constexpr (L) {
-        const float el = in.e4[Q & 1][T % 4];
+        const float el = in.e4[AHEAD ? Q & 1 : 0][T % 4];
         if constexpr (MOVE) lvec = fmaf(lvec, a4[T % 4], el);
         else lvec = lvec + el;
         asm volatile("" : "+v"(lvec)); // the l chain in token order (see fold_token)
+        if constexpr (!AHEAD && T % 4 == 3 && T + 1 < kChunk) in.e4[0] = *reinterpret_cast<lds_f4 *>(eb + T + 1);
     }
 #pragma unroll
     for (int rg = 0; rg < NG; ++rg) acc[rg] = mfma_rank1<T % 16>(ea[rg][T / 16], v, acc[rg]);
 }
 
-template <int G, int D, int T, bool L>
+template <int G, int D, int T, bool L, bool AHEAD>
 __device__ __forceinline__ void team_fold(const TeamLds<G, D> &S, lds_f32 *eb, lds_f32 *ab, const uint8_t *trb,
                                           const uint32_t (&am)[2], const float (&ea)[kGroups<G>][4], TFoldIn &in,
                                           f4 (&acc)[kGroups<G>], float &lvec) {
@@ -646,7 +648,7 @@ __device__ __forceinline__ void team_fold(const TeamLds<G, D> &S, lds_f32 *eb, l
         f4 a4;
         if ((am[T / 32] & gm) == 0) {
             static_for<0, GS>([&](auto K) {
-                team_fold_token<G, D, T + decltype(K)::value, false, L>(S, eb, ab, trb, am, ea, in, a4, acc, lvec);
+                team_fold_token<G, D, T + decltype(K)::value, false, L, AHEAD>(S, eb, ab, trb, am, ea, in, a4, acc, lvec);
             });
             static_for<0, GS / 4>([&](auto) {
                 __builtin_amdgcn_sched_group_barrier(0x002, L ? 8 : 4, 0);
@@ -654,12 +656,12 @@ __device__ __forceinline__ void team_fold(const TeamLds<G, D> &S, lds_f32 *eb, l
             });
         } else {
             static_for<0, GS>([&](auto K) {
-                team_fold_token<G, D, T + decltype(K)::value, true, L>(S, eb, ab, trb, am, ea, in, a4, acc, lvec);
+                team_fold_token<G, D, T + decltype(K)::value, true, L, AHEAD>(S, eb, ab, trb, am, ea, in, a4, acc, lvec);
                 // (two rows: quad by quad, or registers of the rows in flight are moved and spilled)
                 if constexpr (G == 2 && decltype(K)::value % 4 == 3) asm volatile("" : "+v"(acc[0]));
             });
         }
-        team_fold<G, D, T + GS, L>(S, eb, ab, trb, am, ea, in, acc, lvec);
+        team_fold<G, D, T + GS, L, AHEAD>(S, eb, ab, trb, am, ea, in, acc, lvec);
     }
 }
 
@@ -711,9 +713,15 @@ template <int D> struct TRegsOf<false, D> { typedef uint4 T[kTeamRawRegs<D>]; };
 // instead of four (80 and 160). A spill or a move of a register that a row in
 // flight is loaded into waits for the load, which cost two rows at head_dim
 // 128 a quarter of the call (plain 186 -> 146 us, AVX-512 XKV 171 -> 131
-// without them). Left: two registers at four plain rows of head_dim 256.
+// without them).
 template <int G, int D>
 constexpr int kTeamOcc = G > 4 && TShape<D>::NR > 3 ? 3 : 4;
+
+// Whether wave 0 reads e of a quad of tokens a whole quad ahead. Not at four
+// plain rows of head_dim 256: those four registers would spill two that rows
+// are in flight to (64 heads x 65,536 tokens: 774 us, 735 without).
+template <int G, int D, bool XKV>
+constexpr bool kFoldAhead = XKV || D < 256 || G != 4;
 
 template <int G, int D, bool XKV, int ORDER>
 __global__ __launch_bounds__(TShape<D>::W * 64) __attribute__((amdgpu_waves_per_eu(kTeamOcc<G, D>)))
@@ -1000,9 +1008,9 @@ void attn_team_kernel(const HeadDev *__restrict__ heads, const WorkItem *__restr
             for (int k = 0; k < 2; ++k) in.vq[k] = load_tr(trb + 4 * k * TS);
             if (w == 0) {
                 in.e4[0] = *reinterpret_cast<lds_f4 *>(eb);
-                team_fold<G, D, 0, true>(S, eb, ab, trb, am, ea, in, acc, lvec);
+                team_fold<G, D, 0, true, kFoldAhead<G, D, XKV>>(S, eb, ab, trb, am, ea, in, acc, lvec);
             } else {
-                team_fold<G, D, 0, false>(S, eb, ab, trb, am, ea, in, acc, lvec);
+                team_fold<G, D, 0, false, true>(S, eb, ab, trb, am, ea, in, acc, lvec);
             }
         }
         after(__float_as_uint(acc[0].x));
